@@ -348,7 +348,7 @@ size_t bwd_workspace(const Dims& d, int algo, int qkv_dtype) {
   if (bwd_all_mfma(d, qkv_dtype, algo))
     return 2 * bwd_state_bytes(d) + align_up(mfma_bwd_workspace(d), 256) +
            mfma_chunk_bwd_partials(d);
-  return align_up(generic_bwd_workspace(d), 256) + (algo == DN_ALGO_MFMA ? mfma_bwd_workspace(d) : 0);
+  return align_up(generic_bwd_workspace(d), 256);
 }
 
 }  // namespace
@@ -662,10 +662,7 @@ int dn_chunk_bwd(const dn_chunk_bwd_args* a, hipStream_t stream) {
   } else {
     e = generic_bwd(d, a->qkv_dtype, a->grad_dtype, a->d_y, a->d_state_final, a->q, a->k, a->v,
                     a->erase, a->write, g, a->state_in, a->d_q, a->d_k, a->d_v, a->d_erase,
-                    a->d_write, a->has_gate ? a->d_g : nullptr, a->d_state, ws, stream,
-                    algo == DN_ALGO_MFMA
-                        ? static_cast<char*>(ws) + align_up(generic_bwd_workspace(d), 256)
-                        : nullptr);
+                    a->d_write, a->has_gate ? a->d_g : nullptr, a->d_state, ws, stream);
   }
   if (e != hipSuccess) return hip_fail(e, "dn_chunk_bwd launch");
   if (a->check_finite) {

@@ -1,0 +1,715 @@
+// The fp32 chunk backward (chunk_f32.hpp): the reverse scan and the
+// chunk-local gradients. combined_backward.rs:72-513 with the identities of
+// the bf16 kernels: dT = dV'·Xᵀ and d_kg = −(Tᵀ·dV')·S₀ᵀ.
+#include "chunk_f32.hpp"
+
+namespace dn {
+namespace {
+
+// ---------------------------------------------------------------------------
+// reverse scan
+// ---------------------------------------------------------------------------
+// The forward scan's split (a team of four waves per 16 value columns, one
+// token block each, dS's row blocks dealt to them, everything exchanged
+// through LDS in accumulator order), walking the chunks backwards:
+//   dV' = attnᵀ·dY + kc·dS,  Z = Tᵀ·dV',  dS ← egl⊙dS + qgᵀ·dY − kgᵀ·Z.
+// Leaves dS (leaving each chunk), dV' and Z in the workspace.
+template <int KB, int C, bool FOLD, class TG>
+__global__ __launch_bounds__(256 * C) void f32_rev_scan_kernel(FParams p) {
+  constexpr Lay o = lay(KB, FOLD);
+  constexpr int NT = 256 * C;
+  constexpr int kCopy = o.vec / 4;
+  constexpr int NPF = (kCopy + NT - 1) / NT;
+  constexpr int kVec = 4 * kC + 16 * KB;
+  constexpr int NPV = (kVec + NT - 1) / NT;
+  constexpr int NR = (KB + 3) / 4;
+  __shared__ __attribute__((aligned(16))) float tl[kCopy * 4];
+  __shared__ __attribute__((aligned(16))) float vec[kVec];
+  __shared__ __attribute__((aligned(16))) float Sx[C][KB * kBlk];
+  __shared__ __attribute__((aligned(16))) float Yx[C][4 * kBlk], Vx[C][4 * kBlk], Zx[C][4 * kBlk];
+
+  const Dims& d = p.d;
+  const int BH = d.B * d.H, VB = (d.V + 15) / 16, ntile = (VB + C - 1) / C;
+  const int group = blockIdx.x / (8 * ntile), within = blockIdx.x % (8 * ntile);
+  const int tile = within / 8, bh = group * 8 + within % 8;
+  if (bh >= BH) return;
+  const int b = bh / d.H, h = bh % d.H;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int team = wave >> 2, tw = wave & 3;
+  const int tb = (team & 1) ? 3 - tw : tw;
+  const int m16 = lane & 15, g4 = lane >> 4;
+  const int fo = (g4 * 16 + (m16 ^ g4)) * 4;
+  int to[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) to[r] = blk(4 * g4 + r, m16);
+  const int ct = tile * C + team, col = 16 * ct + m16;
+  const bool live = col < d.V;
+  const int cl = min(col, d.V - 1);
+  const TG* dyp = static_cast<const TG*>(p.dy);
+
+  f32x4 S[NR];
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    const int rb = tw + 4 * i;
+    S[i] = zero4();
+    if (p.ds_final) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 16 * rb + 4 * g4 + r;
+        const float x = p.ds_final[(size_t(bh) * d.K + min(row, d.K - 1)) * d.V + cl];
+        S[i][r] = live && row < d.K ? x : 0.f;
+      }
+    }
+    if (rb < KB) st4(&Sx[team][rb * kBlk + 4 * lane], S[i]);
+  }
+  auto chunk = [&](int n) { return (size_t(b) * d.N + n) * d.H + h; };
+  f32x4 pf[NPF], py;
+  float pv[NPV];
+  auto fetch = [&](int n) {
+    const float* src = p.ws + chunk(n) * o.per;
+#pragma unroll
+    for (int i = 0; i < NPF; ++i) pf[i] = ld4(src + 4 * min(tid + NT * i, kCopy - 1));
+#pragma unroll
+    for (int i = 0; i < NPV; ++i) pv[i] = src[o.vec + min(tid + NT * i, kVec - 1)];
+    const int rl = min(kC, d.S - n * kC);
+    const size_t row0 = (size_t(b) * d.S + size_t(n) * kC) * d.H + h;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int t = 16 * tb + 4 * g4 + r;
+      const float x = ld(dyp, (row0 + size_t(min(t, rl - 1)) * d.H) * d.V + cl);
+      py[r] = live && t < rl ? x : 0.f;
+    }
+  };
+  auto stage = [&] {
+#pragma unroll
+    for (int i = 0; i < NPF; ++i)
+      if (NT * (i + 1) <= kCopy || tid + NT * i < kCopy) st4(&tl[4 * (tid + NT * i)], pf[i]);
+#pragma unroll
+    for (int i = 0; i < NPV; ++i)
+      if (tid + NT * i < kVec) vec[tid + NT * i] = pv[i];
+    st4(&Yx[team][tb * kBlk + 4 * lane], py);
+  };
+  fetch(d.N - 1);
+  stage();
+  __syncthreads();
+  for (int n = d.N - 1; n >= 0; --n) {
+    const size_t cid = chunk(n);
+    fetch(max(n - 1, 0));
+    if (ct < VB)
+#pragma unroll
+      for (int i = 0; i < NR; ++i)
+        if (tw + 4 * i < KB)
+          st4(p.ds_after + ((cid * KB + tw + 4 * i) * VB + ct) * kBlk + 4 * lane, S[i]);
+    f32x4 dv = zero4(), av = zero4();
+#pragma unroll
+    for (int cb = 0; cb < KB; ++cb)
+      dv = mm(ld4(&tl[o.u + (tb * KB + cb) * kBlk + fo]), ld4(&Sx[team][cb * kBlk + 4 * lane]),
+              dv);
+    // A transposed block's operand: its four words in column order.
+    auto tr = [&](const float* x) { return f32x4{x[to[0]], x[to[1]], x[to[2]], x[to[3]]}; };
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (j >= tb)
+        av = mm(tr(&tl[o.at + tri_blk(j, tb) * kBlk]), ld4(&Yx[team][j * kBlk + 4 * lane]), av);
+    {
+      const f32x4 gk = ld4(&vec[128 + 16 * tb + 4 * g4]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) dv[r] = av[r] + (FOLD ? dv[r] : gk[r] * dv[r]);
+    }
+    st4(&Vx[team][tb * kBlk + 4 * lane], dv);
+    if (ct < VB) st4(p.dvn + ((cid * 4 + tb) * VB + ct) * kBlk + 4 * lane, dv);
+    lds_barrier();
+    f32x4 z = zero4();
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (j >= tb)
+        z = mm(tr(&tl[o.t + tri_blk(j, tb) * kBlk]), ld4(&Vx[team][j * kBlk + 4 * lane]), z);
+    st4(&Zx[team][tb * kBlk + 4 * lane], z);
+    if (ct < VB) st4(p.z + ((cid * 4 + tb) * VB + ct) * kBlk + 4 * lane, z);
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+      if (tw + 4 * i < KB) {
+        const f32x4 e = ld4(&vec[256 + 16 * (tw + 4 * i) + 4 * g4]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[i][r] *= e[r];
+      }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      f32x4 y = ld4(&Yx[team][j * kBlk + 4 * lane]), zj = ld4(&Zx[team][j * kBlk + 4 * lane]);
+      const f32x4 xe = ld4(&vec[16 * j + 4 * g4]), ys = ld4(&vec[64 + 16 * j + 4 * g4]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        y[r] *= FOLD ? 1.f : ys[r];
+        zj[r] *= FOLD ? -1.f : -xe[r];
+      }
+#pragma unroll
+      for (int i = 0; i < NR; ++i)
+        if (tw + 4 * i < KB) {
+          const int at = (j * KB + tw + 4 * i) * kBlk;
+          S[i] = mm(tr(&tl[o.q + at]), y, S[i]);
+          S[i] = mm(tr(&tl[o.a + at]), zj, S[i]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+      if (tw + 4 * i < KB) st4(&Sx[team][(tw + 4 * i) * kBlk + 4 * lane], S[i]);
+    lds_barrier();
+    stage();
+    lds_barrier();
+  }
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 16 * (tw + 4 * i) + 4 * g4 + r;
+      if (live && row < d.K) p.dstate[(size_t(bh) * d.K + row) * d.V + col] = S[i][r];
+    }
+}
+
+// ---------------------------------------------------------------------------
+// chunk-local gradients
+// ---------------------------------------------------------------------------
+// One workgroup per chunk-head. Phase B walks the value axis 16 columns at a
+// time, double-buffered through LDS (one barrier a step): wave w owns key
+// channels 16w … 16w+15 and sums V'·dSᵀ, dY·S₀ᵀ and Z·S₀ᵀ for all 64 tokens,
+// 48 accumulator registers; the ten lower blocks of dY·V'ᵀ and dV'·Xᵀ are
+// dealt over the waves. Then dAkk = −tril(Tᵀ·dT·Tᵀ, −1) through LDS, and the
+// score backward per channel block, its k, q and gates in registers in the
+// accumulators' own layout.
+template <int KB, bool PCG, bool EK, class TQ, class TG>
+__global__ __launch_bounds__(64 * (KB < 4 ? 4 : KB)) void f32_chunk_bwd_kernel(FParams p) {
+  constexpr bool kFold = PCG || EK;
+  constexpr Lay o = lay(KB, kFold);
+  constexpr int NW = KB < 4 ? 4 : KB;
+  constexpr int kTiles = 20 + 2 * KB;  // X, V', dV', Z, dY (4 blocks each), S₀, dS
+  constexpr int kPlain = 12 + 2 * KB;  // all but dY and Z
+  constexpr int NPT = (kPlain + NW - 1) / NW;
+  constexpr int NP = (10 + NW - 1) / NW;
+  constexpr int kStage = 2 * kTiles * kBlk;
+  constexpr int kLds = kStage > 5 * kTri ? kStage : 5 * kTri;
+  __shared__ __attribute__((aligned(16))) float lds[kLds];
+  __shared__ float sG[kC], red[2][NW][kC];
+
+  const Dims& d = p.d;
+  const int cid = blockIdx.x;
+  const int h = cid % d.H, n = (cid / d.H) % d.N, b = cid / (d.H * d.N);
+  const int VB = (d.V + 15) / 16;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m16 = lane & 15, g4 = lane >> 4;
+  const int fo = (g4 * 16 + (m16 ^ g4)) * 4;
+  int to[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) to[r] = blk(4 * g4 + r, m16);
+  auto tr = [&](const float* x) { return f32x4{x[to[0]], x[to[1]], x[to[2]], x[to[3]]}; };
+  const int rl = min(kC, d.S - n * kC);
+  const size_t row0 = (size_t(b) * d.S + size_t(n) * kC) * d.H + h;
+  const float* ws = p.ws + size_t(cid) * o.per;
+  const TQ* qp = static_cast<const TQ*>(p.q);
+  const TQ* kp = static_cast<const TQ*>(p.k);
+  const TQ* vp = static_cast<const TQ*>(p.v);
+  const TG* dyp = static_cast<const TG*>(p.dy);
+  const bool gated = d.dw > 0;
+
+  // --- phase B ---------------------------------------------------------------
+  // Waves 0 … 3 load token block `wave` of dY and of Z, with v and the write
+  // gate beside Z; the other blocks are dealt over all waves, one scalar
+  // address each.
+  f32x4 pf[NPT], py, pz;
+  float vz[4], wz[4], dwr[4] = {0.f, 0.f, 0.f, 0.f};
+  const float* src[NPT];
+#pragma unroll
+  for (int i = 0; i < NPT; ++i) {
+    const int t = min((wave + 4) % NW + NW * i, kPlain - 1);
+    if (t < 12) {
+      src[i] = (t < 4 ? p.xs : t < 8 ? p.vn : p.dvn) + (size_t(cid) * 4 + (t & 3)) * VB * kBlk;
+    } else {
+      const int sb = t - 12;
+      src[i] = (sb < KB ? p.states : p.ds_after) +
+               (size_t(cid) * KB + (sb < KB ? sb : sb - KB)) * VB * kBlk;
+    }
+  }
+  const float* zsrc = p.z + (size_t(cid) * 4 + (wave & 3)) * VB * kBlk;
+  size_t at4[4];  // this lane's rows of dY, v and d_v (waves 0 … 3)
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    at4[r] = (row0 + size_t(min(16 * (wave & 3) + 4 * g4 + r, rl - 1)) * d.H) * d.V;
+  auto load = [&](int vt) {
+#pragma unroll
+    for (int i = 0; i < NPT; ++i) pf[i] = ld4(src[i] + size_t(vt) * kBlk + 4 * lane);
+    if (wave < 4) {
+      const int col = 16 * vt + m16, cl = min(col, d.V - 1);
+      pz = ld4(zsrc + size_t(vt) * kBlk + 4 * lane);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        py[r] = ld(dyp, at4[r] + cl);
+        vz[r] = ld(vp, at4[r] + cl);
+        if (d.ww != 1) wz[r] = p.write[at4[r] + cl];
+      }
+    }
+  };
+  if (wave < 4 && d.ww == 1)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      wz[r] = p.write[row0 + size_t(min(16 * wave + 4 * g4 + r, rl - 1)) * d.H];
+  // To LDS with rows and columns swapped (a lane's four values are rows), and
+  // from Z the gradients of v and the write gate.
+  auto stage = [&](float* buf, int vt) {
+#pragma unroll
+    for (int i = 0; i < NPT; ++i) {
+      const int t = (wave + 4) % NW + NW * i;
+      if (t >= kPlain) continue;
+      // X, V', dV' at blocks 0 … 11; Z and dY at 12 … 19; S₀ and dS after.
+      float* dst = buf + (t < 12 ? t : t + 8) * kBlk;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) dst[to[r]] = pf[i][r];
+    }
+    if (wave < 4) {
+      const int col = 16 * vt + m16;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const bool ok = 16 * wave + 4 * g4 + r < rl && col < d.V;
+        buf[(12 + wave) * kBlk + to[r]] = pz[r];
+        buf[(16 + wave) * kBlk + to[r]] = ok ? py[r] : 0.f;
+        const float dw = pz[r] * vz[r];
+        if (ok) {
+          st(static_cast<TG*>(p.dv), at4[r] + col, pz[r] * wz[r]);
+          if (d.ww != 1) p.dwrite[at4[r] + col] = dw;
+        }
+        dwr[r] += ok ? dw : 0.f;
+      }
+    }
+  };
+  f32x4 dkc[4], dqr[4], dkg[4], dat[NP], dtt[NP];
+  float degl = 0.f;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) dkc[t] = dqr[t] = dkg[t] = zero4();
+#pragma unroll
+  for (int u = 0; u < NP; ++u) dat[u] = dtt[u] = zero4();
+  load(0);
+  for (int vt = 0; vt < VB; ++vt) {
+    float* buf = lds + (vt & 1) * kTiles * kBlk;
+    stage(buf, vt);
+    lds_barrier();
+    if (vt + 1 < VB) load(vt + 1);
+    if (wave < KB) {
+      const f32x4 s0 = ld4(&buf[(20 + wave) * kBlk + fo]);
+      const f32x4 ds = ld4(&buf[(20 + KB + wave) * kBlk + fo]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) degl += s0[r] * ds[r];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        dkc[t] = mm(ld4(&buf[(4 + t) * kBlk + fo]), ds, dkc[t]);
+        dqr[t] = mm(ld4(&buf[(16 + t) * kBlk + fo]), s0, dqr[t]);
+        dkg[t] = mm(ld4(&buf[(12 + t) * kBlk + fo]), s0, dkg[t]);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+      const int pr = wave + NW * u;
+      if (pr >= 10) continue;
+      const int ti = pr < 1 ? 0 : pr < 3 ? 1 : pr < 6 ? 2 : 3, tj = pr - tri_blk(ti, 0);
+      dat[u] = mm(ld4(&buf[(16 + ti) * kBlk + fo]), ld4(&buf[(4 + tj) * kBlk + fo]), dat[u]);
+      dtt[u] = mm(ld4(&buf[(8 + ti) * kBlk + fo]), ld4(&buf[tj * kBlk + fo]), dtt[u]);
+    }
+  }
+  if (d.ww == 1 && wave < 4) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float x = dwr[r];
+#pragma unroll
+      for (int s = 1; s < 16; s *= 2) x += __shfl_xor(x, s, 64);
+      const int tok = 16 * wave + 4 * g4 + r;
+      if (m16 == 0 && tok < rl) p.dwrite[row0 + size_t(tok) * d.H] = x;
+    }
+  }
+  if (!PCG && tid < kC) sG[tid] = ws[o.vec + 192 + tid];
+  __syncthreads();
+
+  // --- phase C: dAkk and the decayed score cotangents -------------------------
+  float *lT = lds, *lD = lds + kTri, *lP = lds + 2 * kTri, *rkk = lds + 3 * kTri,
+        *rqk = lds + 4 * kTri;
+  for (int i = tid; i < kTri / 4; i += 64 * NW) st4(&lT[4 * i], ld4(ws + o.t + 4 * i));
+#pragma unroll
+  for (int u = 0; u < NP; ++u) {
+    const int pr = wave + NW * u;
+    if (pr >= 10) continue;
+    const int ti = pr < 1 ? 0 : pr < 3 ? 1 : pr < 6 ? 2 : 3, tj = pr - tri_blk(ti, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = 16 * ti + 4 * g4 + r, j = 16 * tj + m16;
+      const float m = PCG ? 1.f : expf(sG[i] - sG[j]);
+      lD[pr * kBlk + to[r]] = dtt[u][r];
+      rqk[pr * kBlk + to[r]] = j <= i ? dat[u][r] * m : 0.f;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < NP; ++u) {
+    const int pr = wave + NW * u;
+    if (pr >= 10) continue;
+    const int ti = pr < 1 ? 0 : pr < 3 ? 1 : pr < 6 ? 2 : 3, tj = pr - tri_blk(ti, 0);
+    f32x4 acc = zero4();  // (dT·Tᵀ)(ti, tj)
+    for (int bi = 0; bi <= tj; ++bi)
+      acc = mm(ld4(&lD[tri_blk(ti, bi) * kBlk + fo]), ld4(&lT[tri_blk(tj, bi) * kBlk + fo]), acc);
+    st4(&lP[pr * kBlk + 4 * lane], acc);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < NP; ++u) {
+    const int pr = wave + NW * u;
+    if (pr >= 10) continue;
+    const int ti = pr < 1 ? 0 : pr < 3 ? 1 : pr < 6 ? 2 : 3, tj = pr - tri_blk(ti, 0);
+    f32x4 acc = zero4();  // (Tᵀ·dT·Tᵀ)(ti, tj)
+    for (int ai = ti; ai < 4; ++ai)
+      acc = mm(tr(&lT[tri_blk(ai, ti) * kBlk]), ld4(&lP[tri_blk(ai, tj) * kBlk + 4 * lane]), acc);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = 16 * ti + 4 * g4 + r, j = 16 * tj + m16;
+      const float m = PCG ? 1.f : expf(sG[i] - sG[j]);
+      rkk[pr * kBlk + to[r]] = j < i ? -acc[r] * m : 0.f;
+    }
+  }
+  __syncthreads();
+
+  // --- phase D: per key channel ------------------------------------------------
+  if (wave < KB) {
+    const int c = 16 * wave + m16, cc = min(c, d.K - 1);
+    const bool cok = c < d.K;
+    f32x4 k[4], q[4], e[4], G[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int tok = 16 * t + 4 * g4 + r;
+        const size_t row = row0 + size_t(min(tok, rl - 1)) * d.H;
+        const bool ok = cok && tok < rl;
+        const float kx = ld(kp, row * d.K + cc), qx = ld(qp, row * d.K + cc);
+        const float ex = p.erase[EK ? row * d.K + cc : row];
+        const float gx = PCG ? p.g[row * d.K + cc] : 0.f;
+        k[t][r] = ok ? kx : 0.f;
+        q[t][r] = ok ? qx * d.scale : 0.f;
+        e[t][r] = ok ? ex : 0.f;
+        G[t][r] = PCG ? (ok ? gx : 0.f) : sG[tok];
+      }
+    float Gl;
+    if constexpr (PCG) {
+      // Cumulative sums down the channel: within a lane's four rows, over the
+      // four lane groups of a block, then over the blocks.
+      float base = 0.f;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+#pragma unroll
+        for (int r = 1; r < 4; ++r) G[t][r] += G[t][r - 1];
+        float x = G[t][3];
+        float up = __shfl_up(x, 16, 64);
+        if (g4 >= 1) x += up;
+        up = __shfl_up(x, 32, 64);
+        if (g4 >= 2) x += up;
+        const float ex = base + (x - G[t][3]);
+        base += __shfl(x, 48 + m16, 64);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) G[t][r] += ex;
+      }
+      Gl = base;
+    } else {
+      Gl = sG[63];
+    }
+    f32x4 dG[4];
+    float carry = 0.f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float eg = expf(G[t][r]), ec = expf(Gl - G[t][r]);
+        const float dkg_ = -dkg[t][r];
+        const float cr = dkc[t][r] * k[t][r] * ec;
+        carry += cr;
+        dG[t][r] = (dqr[t][r] * q[t][r] + dkg_ * k[t][r] * e[t][r]) * eg - cr;
+        dkc[t][r] *= ec;        // → d_k
+        dqr[t][r] *= eg;        // → d_q
+        dkg[t][r] = dkg_ * eg;  // → d(e⊙k)
+      }
+    carry += degl * expf(Gl);
+    carry += __shfl_xor(carry, 16, 64);
+    carry += __shfl_xor(carry, 32, 64);
+    if (g4 == 3) dG[3][3] += carry;
+
+    if constexpr (!PCG) {
+      // head_scores_backward (combined_backward.rs:376-416); the gate's share,
+      // Σ_j of the masked score cotangents against the raw scores, is per row
+      // Σ_c of the products below against ke, q and k.
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        f32x4 a1 = zero4(), a2 = zero4(), a3 = zero4();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (j <= t) {
+            a1 = mm(ld4(&rkk[tri_blk(t, j) * kBlk + fo]), k[j], a1);
+            a2 = mm(ld4(&rqk[tri_blk(t, j) * kBlk + fo]), k[j], a2);
+          }
+          if (j >= t) {
+            f32x4 ke;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) ke[r] = k[j][r] * e[j][r];
+            a3 = mm(tr(&rkk[tri_blk(j, t) * kBlk]), ke, a3);
+            a3 = mm(tr(&rqk[tri_blk(j, t) * kBlk]), q[j], a3);
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          dkg[t][r] += a1[r];
+          dqr[t][r] += a2[r];
+          dkc[t][r] += a3[r];
+          dG[t][r] += k[t][r] * e[t][r] * a1[r] + q[t][r] * a2[r] - k[t][r] * a3[r];
+        }
+      }
+    } else {
+      // channel_scores_backward (combined_backward.rs:421-513): row block pb
+      // through its reference token 8; a clamped exponent passes no gradient.
+#pragma unroll
+      for (int pb = 0; pb < 4; ++pb) {
+        const float Gr = __shfl(G[pb][0], 32 + m16, 64);
+        f32x4 rf, rk, rq, accE = zero4(), accQ = zero4();
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          rf[r] = expf(fminf(G[pb][r] - Gr, kMaxExp));
+          rk[r] = k[pb][r] * e[pb][r] * rf[r];
+          rq[r] = q[pb][r] * rf[r];
+        }
+        float dref = 0.f;
+#pragma unroll
+        for (int jb = 0; jb <= pb; ++jb) {
+          __builtin_amdgcn_sched_barrier(0);  // one block pair's factors at a time
+          f32x4 ce, cb;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            ce[r] = expf(fminf(Gr - G[jb][r], kMaxExp));
+            cb[r] = k[jb][r] * ce[r];
+          }
+          const float *xk = &rkk[tri_blk(pb, jb) * kBlk], *xq = &rqk[tri_blk(pb, jb) * kBlk];
+          accE = mm(ld4(xk + fo), cb, accE);
+          accQ = mm(ld4(xq + fo), cb, accQ);
+          f32x4 dc = mm(tr(xk), rk, zero4());
+          dc = mm(tr(xq), rq, dc);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            dkc[jb][r] += dc[r] * ce[r];
+            const float x = Gr - G[jb][r] >= kMaxExp ? 0.f : dc[r] * cb[r];
+            dG[jb][r] -= x;
+            dref += x;
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          dkg[pb][r] += accE[r] * rf[r];
+          dqr[pb][r] += accQ[r] * rf[r];
+          const float x =
+              G[pb][r] - Gr >= kMaxExp ? 0.f : accE[r] * rk[r] + accQ[r] * rq[r];
+          dG[pb][r] += x;
+          dref -= x;
+        }
+        dref += __shfl_xor(dref, 16, 64);
+        dref += __shfl_xor(dref, 32, 64);
+        if (g4 == 2) dG[pb][0] += dref;
+        // Left to itself the compiler moves these sums into the stores at the
+        // end, every term of them live until then.
+#pragma unroll
+        for (int t = 0; t <= pb; ++t) asm volatile("" : "+v"(dkc[t]), "+v"(dG[t]));
+        asm volatile("" : "+v"(dkg[pb]), "+v"(dqr[pb]));
+      }
+    }
+    // Front end (combined_backward.rs:153-188).
+    if constexpr (PCG) {
+      // d_g: the reverse of the cumulative sum.
+      float base = 0.f;
+#pragma unroll
+      for (int t = 3; t >= 0; --t) {
+#pragma unroll
+        for (int r = 2; r >= 0; --r) dG[t][r] += dG[t][r + 1];
+        float x = dG[t][0];
+        float dn = __shfl_down(x, 16, 64);
+        if (g4 <= 2) x += dn;
+        dn = __shfl_down(x, 32, 64);
+        if (g4 <= 1) x += dn;
+        const float ex = base + (x - dG[t][0]);
+        base += __shfl(x, m16, 64);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) dG[t][r] += ex;
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int tok = 16 * t + 4 * g4 + r;
+        const size_t at = (row0 + size_t(tok) * d.H) * d.K + c;
+        const float de = dkg[t][r] * k[t][r];
+        if (cok && tok < rl) {
+          st(static_cast<TG*>(p.dq), at, dqr[t][r] * d.scale);
+          st(static_cast<TG*>(p.dk), at, dkc[t][r] + dkg[t][r] * e[t][r]);
+          if constexpr (EK) p.derase[at] = de;
+          if constexpr (PCG)
+            if (p.dg) p.dg[at] = dG[t][r];
+        }
+        // Width-1 gates: sums over the key channels, per token (channels past
+        // head_k_dim hold zeros).
+        if constexpr (!EK || !PCG) {
+          float x = EK ? 0.f : de, y = PCG ? 0.f : dG[t][r];
+#pragma unroll
+          for (int s = 1; s < 16; s *= 2) {
+            if constexpr (!EK) x += __shfl_xor(x, s, 64);
+            if constexpr (!PCG) y += __shfl_xor(y, s, 64);
+          }
+          if (m16 == 0) {
+            red[0][wave][tok] = x;
+            red[1][wave][tok] = y;
+          }
+        }
+      }
+  }
+  if constexpr (!EK || !PCG) {
+    __syncthreads();
+    if (wave == 0) {
+      float x = 0.f, y = 0.f;
+#pragma unroll
+      for (int w = 0; w < KB; ++w) {
+        x += red[0][w][lane];
+        y += red[1][w][lane];
+      }
+      // d_g of a token sums the cumulative gate's cotangents from it on.
+#pragma unroll
+      for (int s = 1; s < 64; s *= 2) {
+        const float dn = __shfl_down(y, s, 64);
+        if (lane + s < 64) y += dn;
+      }
+      if (lane < rl) {
+        const size_t row = row0 + size_t(lane) * d.H;
+        if constexpr (!EK) p.derase[row] = x;
+        if constexpr (!PCG)
+          if (gated && p.dg) p.dg[row] = y;
+      }
+    }
+  }
+}
+
+hipError_t launch_rev(const FParams& p, int grad_dtype, hipStream_t stream) {
+  const Dims& d = p.d;
+  const int teams = scan_teams(d);
+  const dim3 grid(scan_blocks(d, teams)), block(256 * teams);
+  const bool g16 = grad_dtype == DN_BF16, fold = folds(d);
+  ProfScope ps("dn_f32_rev_scan", stream);
+#define DN_R(KB, C, F)                                                                       \
+  do {                                                                                       \
+    if (g16)                                                                                 \
+      hipLaunchKernelGGL((f32_rev_scan_kernel<KB, C, F, bf16>), grid, block, 0, stream, p);  \
+    else                                                                                     \
+      hipLaunchKernelGGL((f32_rev_scan_kernel<KB, C, F, float>), grid, block, 0, stream, p); \
+  } while (0)
+#define DN_RK(KB)                                                           \
+  do {                                                                      \
+    if (teams == 1) { if (fold) DN_R(KB, 1, true); else DN_R(KB, 1, false); } \
+    else { if (fold) DN_R(KB, 2, true); else DN_R(KB, 2, false); }          \
+  } while (0)
+  switch (key_blocks(d.K)) {
+    case 2: DN_RK(2); break;
+    case 4: DN_RK(4); break;
+    case 6: DN_RK(6); break;
+    default: DN_RK(8); break;
+  }
+#undef DN_RK
+#undef DN_R
+  return hipGetLastError();
+}
+
+hipError_t launch_chunk_bwd(const FParams& p, int qkv_dtype, int grad_dtype, hipStream_t stream) {
+  const Dims& d = p.d;
+  const bool pcg = d.dw > 1, ek = d.ew > 1;
+  const bool b16 = qkv_dtype == DN_BF16, g16 = grad_dtype == DN_BF16;
+  const int kb = key_blocks(d.K);
+  const dim3 grid(unsigned(chunk_heads(d))), block(64 * (kb < 4 ? 4 : kb));
+  ProfScope ps("dn_f32_chunk_bwd", stream);
+#define DN_C(KB, PC, EK, TQ, TG) \
+  hipLaunchKernelGGL((f32_chunk_bwd_kernel<KB, PC, EK, TQ, TG>), grid, block, 0, stream, p)
+#define DN_CT(KB, PC, EK)                                                                \
+  do {                                                                                   \
+    if (b16) { if (g16) DN_C(KB, PC, EK, bf16, bf16); else DN_C(KB, PC, EK, bf16, float); }  \
+    else { if (g16) DN_C(KB, PC, EK, float, bf16); else DN_C(KB, PC, EK, float, float); }    \
+  } while (0)
+#define DN_CG(KB)                                                             \
+  do {                                                                        \
+    if (pcg) { if (ek) DN_CT(KB, true, true); else DN_CT(KB, true, false); }  \
+    else { if (ek) DN_CT(KB, false, true); else DN_CT(KB, false, false); }    \
+  } while (0)
+  switch (kb) {
+    case 2: DN_CG(2); break;
+    case 4: DN_CG(4); break;
+    case 6: DN_CG(6); break;
+    default: DN_CG(8); break;
+  }
+#undef DN_CG
+#undef DN_CT
+#undef DN_C
+  return hipGetLastError();
+}
+
+// The backward's buffers after the tiles.
+struct BwdSizes {
+  size_t state, rows;  // bytes of one [G][KB][VB] and one [G][4][VB] block array
+};
+BwdSizes bwd_sizes(const Dims& d) {
+  const size_t blocks = chunk_heads(d) * size_t((d.V + 15) / 16) * kBlk;
+  return {bytes_of(blocks * key_blocks(d.K)), bytes_of(blocks * 4)};
+}
+
+}  // namespace
+
+size_t f32_bwd_workspace(const Dims& d) {
+  const BwdSizes s = bwd_sizes(d);
+  return f32_fwd_workspace(d) + 2 * s.state + 4 * s.rows +
+         bytes_of(size_t(d.B) * d.H * d.K * d.V);  // the recompute's final state (unused)
+}
+
+hipError_t f32_bwd(const Dims& d, int qkv_dtype, int grad_dtype, const void* dy,
+                   const float* dstate_final, const void* q, const void* k, const void* v,
+                   const float* erase, const float* write, const float* g, const float* state_in,
+                   void* dq, void* dk, void* dv, float* derase, float* dwrite, float* dg,
+                   float* dstate, void* ws, hipStream_t stream) {
+  FParams p = f32_params(d, qkv_dtype, q, k, v, erase, write, g, state_in, ws);
+  const BwdSizes s = bwd_sizes(d);
+  char* base = static_cast<char*>(ws) + f32_fwd_workspace(d);
+  auto take = [&](size_t bytes) {
+    float* at = reinterpret_cast<float*>(base);
+    base += bytes;
+    return at;
+  };
+  p.states = take(s.state);
+  p.ds_after = take(s.state);
+  p.xs = take(s.rows);
+  p.vn = take(s.rows);
+  p.dvn = take(s.rows);
+  p.z = take(s.rows);
+  p.s_out = take(0);
+  p.dy = dy;
+  p.ds_final = dstate_final;
+  p.dstate = dstate;
+  p.dq = dq;
+  p.dk = dk;
+  p.dv = dv;
+  p.derase = derase;
+  p.dwrite = dwrite;
+  p.dg = dg;
+  hipError_t e = f32_intra(p, qkv_dtype, stream);
+  if (e != hipSuccess) return e;
+  // The two scans need nothing from each other: the reverse one runs on the
+  // calling stream's second stream.
+  hipStream_t side = nullptr;
+  if ((e = side_fork(stream, &side)) != hipSuccess) return e;
+  if ((e = launch_rev(p, grad_dtype, side)) != hipSuccess) return e;
+  if ((e = f32_scan(p, qkv_dtype, DN_F32, true, stream)) != hipSuccess) return e;
+  if ((e = side_join(stream)) != hipSuccess) return e;
+  return launch_chunk_bwd(p, qkv_dtype, grad_dtype, stream);
+}
+
+}  // namespace dn

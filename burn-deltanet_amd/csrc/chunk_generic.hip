@@ -1,5 +1,8 @@
 // The chunkwise WY forward and its backward in fp32 arithmetic, for any
-// shape, gate width and chunk length.
+// shape, gate width and chunk length: what the fp32 matrix-core kernels
+// (chunk_f32.hpp) do not take, that is head_k_dim above 128, a per-channel
+// forget gate at a chunk length other than 64, and calls so small that
+// 64-token chunks would need more workspace than their own.
 //
 // Same three stages as the reference (src/delta/chunk_recalculated/forward.rs):
 //   intra   one workgroup per chunk-head (b, n, h), fully parallel:
@@ -859,16 +862,48 @@ size_t G_of(const Dims& d) { return size_t(d.B) * d.N * d.H; }
 
 }  // namespace
 
-size_t generic_fwd_workspace(const Dims& d) {
+static size_t own_fwd_workspace(const Dims& d) {
   return align_up(G_of(d) * make_layout(d).per * sizeof(float), 256);
 }
 
-size_t generic_bwd_workspace(const Dims& d) {
+static size_t own_bwd_workspace(const Dims& d) {
   const size_t G = G_of(d);
-  size_t bytes = generic_fwd_workspace(d);
+  size_t bytes = own_fwd_workspace(d);
   bytes += align_up(G * make_bwd_layout(d).per * sizeof(float), 256);
   bytes += 2 * align_up(G * size_t(d.K) * d.V * sizeof(float), 256);
   return bytes;
+}
+
+// Whether the matrix-core kernels run a call, and the dims they run it with:
+// 64-token chunks, which without a per-channel forget gate order the
+// roundings and nothing else (with one, the block decay's clamp depends on
+// where chunks start, so another length keeps its kernels). They take every
+// such call whose workspace they do not enlarge, so that a caller's fixed
+// scratch holds what it held; short chunks of small heads are the exception
+// (S = 64 in chunks of 16 with K = V = 4: 38 KB a head against 23).
+static Dims f32_dims(const Dims& d) {
+  Dims f = d;
+  if (d.dw <= 1 || d.K == 1) {
+    f.L = 64;
+    f.N = (d.S + 63) / 64;
+  }
+  return f;
+}
+static bool f32_takes_fwd(const Dims& d) {
+  const Dims f = f32_dims(d);
+  return f32_supported(f) && f32_fwd_workspace(f) <= own_fwd_workspace(d);
+}
+static bool f32_takes_bwd(const Dims& d) {
+  const Dims f = f32_dims(d);
+  return f32_supported(f) && f32_bwd_workspace(f) <= own_bwd_workspace(d);
+}
+
+size_t generic_fwd_workspace(const Dims& d) {
+  return f32_takes_fwd(d) ? f32_fwd_workspace(f32_dims(d)) : own_fwd_workspace(d);
+}
+
+size_t generic_bwd_workspace(const Dims& d) {
+  return f32_takes_bwd(d) ? f32_bwd_workspace(f32_dims(d)) : own_bwd_workspace(d);
 }
 
 static hipError_t launch_intra(const Dims& d, int qkv_dtype, const void* q, const void* k,
@@ -889,6 +924,9 @@ hipError_t generic_fwd(const Dims& d, int qkv_dtype, int y_dtype, const void* q,
                        const void* v, const float* erase, const float* write, const float* g,
                        const float* state_in, void* y, float* state_out, void* wsv,
                        hipStream_t stream) {
+  if (f32_takes_fwd(d))
+    return f32_fwd(f32_dims(d), qkv_dtype, y_dtype, q, k, v, erase, write, g, state_in, y,
+                   state_out, wsv, stream);
   float* ws = static_cast<float*>(wsv);
   hipError_t e = launch_intra(d, qkv_dtype, q, k, v, erase, write, g, ws, stream);
   if (e != hipSuccess) return e;
@@ -913,12 +951,14 @@ hipError_t generic_bwd(const Dims& d, int qkv_dtype, int grad_dtype, const void*
                        const float* dstate_final, const void* q, const void* k, const void* v,
                        const float* erase, const float* write, const float* g,
                        const float* state_in, void* dq, void* dk, void* dv, float* derase,
-                       float* dwrite, float* dg, float* dstate, void* wsv, hipStream_t stream,
-                       void* mfma_ws) {
+                       float* dwrite, float* dg, float* dstate, void* wsv, hipStream_t stream) {
+  if (f32_takes_bwd(d))
+    return f32_bwd(f32_dims(d), qkv_dtype, grad_dtype, dy, dstate_final, q, k, v, erase, write, g,
+                   state_in, dq, dk, dv, derase, dwrite, dg, dstate, wsv, stream);
   const size_t G = G_of(d);
   char* base = static_cast<char*>(wsv);
   float* ws = reinterpret_cast<float*>(base);
-  base += generic_fwd_workspace(d);
+  base += own_fwd_workspace(d);
   float* bws = reinterpret_cast<float*>(base);
   base += align_up(G * make_bwd_layout(d).per * sizeof(float), 256);
   float* states = reinterpret_cast<float*>(base);
@@ -927,15 +967,9 @@ hipError_t generic_bwd(const Dims& d, int qkv_dtype, int grad_dtype, const void*
 
   hipError_t e = launch_intra(d, qkv_dtype, q, k, v, erase, write, g, ws, stream);
   if (e != hipSuccess) return e;
-  if (mfma_ws) {
-    // Both scans on MFMA; the chunk-local gradients below are unchanged.
-    e = mfma_bwd_scans(d, grad_dtype, dy, dstate_final, q, k, v, erase, write, g, state_in,
-                       states, ds_after, dstate, mfma_ws, stream, false);
-    if (e != hipSuccess) return e;
-  } else if ((e = generic_bwd_scans(d, grad_dtype, dy, dstate_final, state_in, ws, states,
-                                    ds_after, dstate, stream)) != hipSuccess) {
+  if ((e = generic_bwd_scans(d, grad_dtype, dy, dstate_final, state_in, ws, states, ds_after,
+                             dstate, stream)) != hipSuccess)
     return e;
-  }
   ChunkBwdParams cp{d,     make_layout(d), make_bwd_layout(d), ws,     bws,   states,
                     ds_after, dy,           dq,                 dk,     dv,    derase,
                     dwrite,   dg};

@@ -110,8 +110,22 @@ hipError_t generic_bwd(const Dims& d, int qkv_dtype, int grad_dtype, const void*
                        const float* dstate_final, const void* q, const void* k, const void* v,
                        const float* erase, const float* write, const float* g,
                        const float* state_in, void* dq, void* dk, void* dv, float* derase,
-                       float* dwrite, float* dg, float* dstate, void* ws, hipStream_t stream,
-                       void* mfma_ws = nullptr);
+                       float* dwrite, float* dg, float* dstate, void* ws, hipStream_t stream);
+
+// The chunk forward and backward in fp32 on fp32 matrix cores (chunk_f32.hpp),
+// in chunks of 64 tokens: head_k_dim up to 128, any head_v_dim and gates.
+bool f32_supported(const Dims& d);
+size_t f32_fwd_workspace(const Dims& d);
+hipError_t f32_fwd(const Dims& d, int qkv_dtype, int y_dtype, const void* q, const void* k,
+                   const void* v, const float* erase, const float* write, const float* g,
+                   const float* state_in, void* y, float* state_out, void* ws,
+                   hipStream_t stream);
+size_t f32_bwd_workspace(const Dims& d);
+hipError_t f32_bwd(const Dims& d, int qkv_dtype, int grad_dtype, const void* dy,
+                   const float* dstate_final, const void* q, const void* k, const void* v,
+                   const float* erase, const float* write, const float* g, const float* state_in,
+                   void* dq, void* dk, void* dv, float* derase, float* dwrite, float* dg,
+                   float* dstate, void* ws, hipStream_t stream);
 
 bool mfma_fwd_supported(const Dims& d, int qkv_dtype, int y_dtype);
 bool mfma_bwd_supported(const Dims& d, int qkv_dtype);

@@ -68,7 +68,8 @@ typedef enum {
  * generic kernels and an explicit MFMA request is refused. */
 typedef enum {
   DN_ALGO_AUTO = 0,
-  DN_ALGO_GENERIC = 1, /* fp32 arithmetic, any shape */
+  DN_ALGO_GENERIC = 1, /* fp32 arithmetic, any shape (fp32 matrix cores up to
+                          head_k_dim 128) */
   DN_ALGO_MFMA = 2,    /* bf16 MFMA tiles; DN_ERR_UNSUPPORTED if the shape does not fit.
                           The forward runs two kernels (intra-chunk tiles through the
                           workspace, then the scan). */

@@ -1,0 +1,100 @@
+"""The fp32 matrix-core chunk kernels (csrc/chunk_f32.hpp), which run what
+DN_ALGO_GENERIC names at head_k_dim up to 128, against the float64 oracle at
+the edges of their tiles: key blocks of 32, value columns of 16 in one- and
+two-team workgroups, a chunk's 64 tokens.
+
+Bar: an output is a sum of products over at most K keys and two triangles of
+64 tokens, each rounded to 2^-24 of the running sum; twice that worst case,
+normwise."""
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import random_raw, rel_err
+from gpu_util import DEV, announce, as_oracle_inputs, np_of, pkg, to_gpu
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+GENERIC = pkg.abi.DN_ALGO_GENERIC
+
+
+def bar(K):
+    return 2 * (K + 2 * 64) * 2.0 ** -24
+
+
+def inputs(rng, B, S, H, K, V, erase, write, decay):
+    """Gates by width: 1, the head's (None: no forget gate)."""
+    q, k, v, e, w, g, s = random_raw(rng, B, S, H, K, V, channel=True)
+    cut = lambda x, width: x[..., :1].copy() if width == 1 else x
+    return [q, k, v, cut(e, erase), cut(w, write), None if decay is None else cut(g, decay), s]
+
+
+# B, S, H, K, V, chunk_len, widths of erase, write and decay
+CASES = [
+    (1, 1, 1, 1, 1, 64, (1, 1, 1)),
+    (1, 64, 1, 32, 16, 64, (1, 1, None)),
+    (2, 65, 3, 33, 17, 64, (33, 1, 1)),
+    (1, 63, 2, 64, 5, 64, (1, 5, 64)),
+    (2, 130, 1, 100, 48, 64, (100, 48, 100)),
+    (1, 128, 2, 128, 40, 64, (1, 1, 1)),
+    (1, 96, 2, 128, 130, 64, (128, 130, 128)),
+    (3, 70, 1, 96, 33, 100, (1, 33, 1)),
+    (1, 200, 2, 66, 32, 32, (66, 1, None)),
+    # 288 column tiles: more than the device's CUs, so two-team workgroups
+    (9, 66, 16, 64, 24, 64, (1, 1, 1)),
+    (9, 66, 16, 128, 24, 64, (128, 24, 128)),
+]
+
+
+def profiled(f):
+    pkg.abi.profile_enable(True)
+    out = f()
+    torch.cuda.synchronize()
+    names = pkg.abi.profile_read()
+    pkg.abi.profile_enable(False)
+    assert names and all(n.startswith("dn_f32") for n in names), names
+    return out
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("case", CASES)
+def test_f32_forward_and_backward_match_oracle(rng, case, dtype):
+    B, S, H, K, V, L, (ew, ww, dw) = case
+    announce(f"f32 kernels {case} {dtype}")
+    args = inputs(rng, B, S, H, K, V, ew, ww, dw)
+    g_args = to_gpu(args, dtype)
+    ref = as_oracle_inputs(g_args)
+    scale = 1.0 / np.sqrt(K)
+    y, s = profiled(lambda: pkg.delta_chunk_recalculated(
+        *g_args, dw is not None, L, scale, algo=GENERIC, y_dtype=torch.float32))
+    want_y, want_s = O.chunk_fwd(*ref, chunk_len=L)
+    assert rel_err(np_of(y), want_y) < bar(K)
+    assert rel_err(np_of(s), want_s) < bar(K)
+    dy = torch.tensor(rng.standard_normal((B, S, H, V)), dtype=torch.float32, device=DEV)
+    ds = torch.tensor(rng.standard_normal((B, H, K, V)), dtype=torch.float32, device=DEV)
+    got = profiled(lambda: pkg.combined_backward(dy, ds, *g_args, L, scale, algo=GENERIC))
+    want = O.chunk_bwd(np_of(dy), np_of(ds), *ref, chunk_len=L)
+    names = ("d_q_bshk", "d_k_bshk", "d_v_bshv", "d_erase_bshK", "d_write_bshV", "d_g_bshK",
+             "d_state_bhkv")
+    # d_g sums q ⊙ d_q and k ⊙ d_k with both signs (at one token of one channel
+    # the sum is 1e-3 of its terms): its rounding is that of the terms.
+    term = max(float(np.abs(want[i] * ref[i]).max()) for i in (0, 1))
+    for name, x in zip(names, want):
+        if x is not None:
+            least = term if name == "d_g_bshK" else 0.0
+            err = np.abs(np_of(getattr(got, name)) - x).max() / max(np.abs(x).max(), least)
+            assert err < bar(K), name
+
+
+def test_f32_kernels_do_not_enlarge_a_workspace(rng):
+    """Short chunks of small heads keep kernels of their own: 64-token tiles
+    would need more scratch than a caller held for them."""
+    args = to_gpu(inputs(rng, 1, 64, 1, 4, 4, 1, 1, 1))
+    pkg.abi.profile_enable(True)
+    pkg.delta_chunk_recalculated(*args, True, 16, 0.5, algo=GENERIC)
+    torch.cuda.synchronize()
+    names = pkg.abi.profile_read()
+    pkg.abi.profile_enable(False)
+    assert all(n.startswith("dn_generic") for n in names), names
