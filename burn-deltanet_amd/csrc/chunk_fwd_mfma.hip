@@ -1472,19 +1472,37 @@ hipError_t launch_intra(const MfmaParams& p, const Dims& d, hipStream_t stream,
   return hipGetLastError();
 }
 
-// Scan workgroup width: 128 or 64 value columns (8 or 4 waves) when that
-// still yields a workgroup per CU, else 32 so more CUs share the sequences
-// (config 4, 64 sequences of dv = 128: 256 two-wave workgroups run its scan
-// 3% faster than 128 four-wave ones).
-int scan_waves(const Dims& d) {
+// Scan workgroup width in waves of 16 value columns. A workgroup holds a CU's
+// LDS, so a scan runs in rounds of one workgroup per CU, each as long as the
+// sequence; a wider workgroup's chunk takes longer, but fewer rounds may do.
+// The width is the one whose rounds cost least, with the time of a chunk as
+// measured at head_k_dim 128, in one round: per-head gates 3.2, 3.6 and 4.0 us
+// at 2, 4 and 8 waves, per-channel 3.4, 3.6 and 5.3 (at head_k_dim 64 the
+// ratios are flatter). In the backward at head_k_dim 128 the states scan and
+// the reverse scan share the device and do not fit on one CU together
+// (`pair`); at 64 they do. us a chunk (forward) and us a call (backward) at 16
+// chunks, narrowest width that fills the device -> this choice: forward dv 256,
+// 48 heads 6.05 -> 3.72 (4 waves), 96 heads 7.11 -> 4.30 (8); dv 128, 96 heads
+// 6.09 -> 3.72; per channel, dv 256, 48 heads 6.62 -> 3.79. Backward dv 256, 24
+// heads 271 -> 232, 48 heads 452 -> 382; dv 128, 96 heads 469 -> 404.
+int scan_waves(const Dims& d, bool backward = false) {
   // head_k_dim 256: eight waves, whose staging registers (11 per lane) fit
   // beside the 64 of the state's rows.
   if (d.K == 256) return 8;
-  const int groups = (d.B * d.H + 7) / 8;
-  const int cus = device_cu_count();
-  if (d.V % 128 == 0 && size_t(groups) * 8 * (d.V / 128) >= size_t(cus)) return 8;
-  if (d.V % 64 == 0 && size_t(groups) * 8 * (d.V / 64) >= size_t(cus)) return 4;
-  return 2;
+  const size_t cus = size_t(device_cu_count()), copies = backward && d.K == 128 ? 2 : 1;
+  int best = 2;
+  float least = 0.f;
+  for (int w = 2; w <= 8; w *= 2) {
+    if (d.V % (16 * w) != 0) break;
+    const size_t wgs = size_t(d.B) * d.H * (d.V / (16 * w)) * copies;
+    const float t = w == 2 ? 1.f : w == 4 ? (pc_path(d) ? 1.05f : 1.1f) : (pc_path(d) ? 1.6f : 1.25f);
+    const float cost = t * float((wgs + cus - 1) / cus);
+    if (w == 2 || cost < least) {
+      best = w;
+      least = cost;
+    }
+  }
+  return best;
 }
 
 // Segments per sequence for the scans. A scan workgroup holds a CU's LDS,
@@ -1563,7 +1581,7 @@ hipError_t launch_scan(const MfmaParams& p, const Dims& d, bool yb, hipStream_t 
       return hipGetLastError();
     }
   }
-  const int waves = scan_waves(d);
+  const int waves = scan_waves(d, ST);
   const unsigned blocks = unsigned(((d.B * d.H + 7) / 8) * 8 * (d.V / (16 * waves)));
   ProfScope ps(ST ? (pc ? "dn_mfma_scan_pc_states" : "dn_mfma_scan_states")
                   : (pc ? "dn_mfma_scan_pc" : "dn_mfma_scan"),
@@ -1848,7 +1866,7 @@ hipError_t mfma_bwd_scans(const Dims& d, int grad_dtype, const void* dy,
   // tiles; eight waves spilled there). At B=8 T=4096 H=16 dv=256: eight
   // waves row-major 5.05 ms, four 3.85, four in row groups 1.61, eight in
   // row groups 1.36.
-  const int waves = d.K == 256 && !g4 ? 4 : scan_waves(d);
+  const int waves = d.K == 256 && !g4 ? 4 : scan_waves(d, true);
   const unsigned blocks = unsigned(((d.B * d.H + 7) / 8) * 8 * (d.V / (16 * waves)));
   {
   ProfScope ps("dn_mfma_rev_scan", side);
