@@ -53,18 +53,6 @@ namespace {
 constexpr int kThreads = 256;  // 4 waves
 constexpr int kBV = 64;       // head_v_dim granularity of the MFMA path
 
-// The backward's transposed tiles. The reverse scan contracts over a chunk's
-// tokens where the forward contracts over its rows, so it reads Tᵀ (hi, lo),
-// attnᵀ, Kc = (Kcᵀ)ᵀ, and Qgᵀ = (scale·e^G⊙Q)ᵀ, Kgᵀ = (e⊙e^G⊙K)ᵀ
-// (combined_backward.rs:272-282: the state cotangent picks up qrᵀ·dy and
-// Wᵀ·dV' = kgᵀ·(Tᵀ·dV')). The intra kernels write them in their BT mode.
-struct BwdTiles {
-  uint16_t *Tt, *Ttl, *AtT;  // [G][64][64]
-  uint16_t* Kc;              // [G][64][K]
-  uint16_t *QgT, *KgT;       // [G][K][64]
-  float* egl;                // [G][K] e^{G_last} per key channel
-};
-
 // ---------------------------------------------------------------------------
 // intra
 // ---------------------------------------------------------------------------
@@ -880,39 +868,38 @@ __global__ __launch_bounds__(kThreads) void mfma_intra_pc_kernel(MfmaParams p, B
 // seg = 1 mode produces for every segment at once. Here one workgroup of
 // four waves per (b, h, 16 state columns) walks its segments in order:
 // start(0) = S_in, start(s+1) = M_s·start(s) + H_s, written to seg_start for
-// the seg = 2 scan. Wave w forms state rows 32w … 32w+31; the four waves
+// the seg = 2 scan. Wave w forms a quarter of the state rows; the four waves
 // exchange the state through LDS once per step, and each holds its rows of
 // the next M and H in registers, loaded while the current step finishes.
 // The fp32 products run as bf16 MFMAs of hi + lo parts (Mh·Sh + Mh·Sl +
 // Ml·Sh, relative error about 2⁻¹⁶).
 template <int K>
 __global__ __launch_bounds__(256) void seg_carry_kernel(MfmaParams p) {
-  static_assert(K == 128, "four waves of 32 state rows");
-  constexpr int KK = K / 32;
+  constexpr int KK = K / 32, J = K / 64;  // k-steps; 16-row blocks per wave
   __shared__ float Ss[K][17];  // the state's 16 columns
   const int ncol = p.V / 16, P = p.seg_p;
   const int bh = blockIdx.x / ncol, ct = blockIdx.x % ncol;
   const int b = bh / p.H, h = bh % p.H;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r16 = lane & 15, q4 = lane >> 4;
-  const int col = 16 * ct + r16, row0 = 32 * wave;
-  f32x4 S[2];  // rows row0 + 16j + 4q4 + r
+  const int col = 16 * ct + r16, row0 = 16 * J * wave;
+  f32x4 S[J];  // rows row0 + 16j + 4q4 + r
   {
     const float* sin = p.s_in + size_t(bh) * K * p.V + col;
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < J; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) S[j][r] = sin[size_t(row0 + 16 * j + 4 * q4 + r) * p.V];
   }
   // This wave's rows of M_s (channels 32kk + 4q4 + 0…3 and 32kk + 16 + 4q4 +
   // 0…3, the B fragment's order) and of H_s.
-  float4 mA[2][KK][2];
-  f32x4 hA[2];
+  float4 mA[J][KK][2];
+  f32x4 hA[J];
   auto fetch = [&](int s) {
     const size_t seg = size_t(b * P + s) * p.H + h;
     const float* M = p.seg_m + seg * K * K;
     const float* Hs = p.seg_h + seg * K * p.V + col;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < J; ++j) {
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk) {
         const float* mr = M + size_t(row0 + 16 * j + r16) * K + 32 * kk + 4 * q4;
@@ -928,7 +915,7 @@ __global__ __launch_bounds__(256) void seg_carry_kernel(MfmaParams p) {
   for (int s = 0; s < P; ++s) {
     float* st = p.seg_start + (size_t(b * P + s) * p.H + h) * K * p.V + col;
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < J; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         st[size_t(row0 + 16 * j + 4 * q4 + r) * p.V] = S[j][r];
@@ -936,7 +923,9 @@ __global__ __launch_bounds__(256) void seg_carry_kernel(MfmaParams p) {
       }
     if (s + 1 == P) break;
     __syncthreads();  // the whole state is in Ss
-    f32x4 acc[2] = {hA[0], hA[1]};
+    f32x4 acc[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) acc[j] = hA[j];
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
       f32x4 s0, s1;
@@ -948,7 +937,7 @@ __global__ __launch_bounds__(256) void seg_carry_kernel(MfmaParams p) {
       const uint4 sh = frag_hi(s0, s1);
       const uint4 sl = frag_lo(s0, s1, sh);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < J; ++j) {
         const float4 a0 = mA[j][kk][0], a1 = mA[j][kk][1];
         const f32x4 m0 = {a0.x, a0.y, a0.z, a0.w}, m1 = {a1.x, a1.y, a1.z, a1.w};
         const uint4 mh = frag_hi(m0, m1);
@@ -960,8 +949,8 @@ __global__ __launch_bounds__(256) void seg_carry_kernel(MfmaParams p) {
     }
     if (s + 2 < P) fetch(s + 1);
     __syncthreads();  // every wave has read Ss
-    S[0] = acc[0];
-    S[1] = acc[1];
+#pragma unroll
+    for (int j = 0; j < J; ++j) S[j] = acc[j];
   }
 }
 
@@ -980,15 +969,6 @@ __global__ __launch_bounds__(256) void seg_carry_kernel(MfmaParams p) {
 // once in double-buffered LDS with the same k-permutation (head_k_dim 256:
 // 120 KB a chunk, single-buffered between two barriers). dS is read as bf16
 // hi + lo parts, dV' likewise for Tᵀ·dV'.
-struct RevParams {
-  int B, S, H, V, N;
-  const void* dy;            // [B, S, H, V], bf16 or fp32
-  const float* dstate_final;  // [B, H, K, V] or null (zeros)
-  float* ds_after;            // [G][K][V]
-  float* dstate;              // [B, H, K, V] cotangent of the initial state
-  BwdTiles bt;
-};
-
 // G4: ds_after in row groups of four ([G][K/4][V][4], states_g4).
 template <int K, class TG, int WAVES, bool G4 = false>
 __global__ __launch_bounds__(64 * WAVES) void mfma_rev_scan_kernel(RevParams p) {
@@ -1150,77 +1130,29 @@ __global__ __launch_bounds__(64 * WAVES) void mfma_rev_scan_kernel(RevParams p) 
                            pk_bf16(dyR[kk][4], dyR[kk][5]), pk_bf16(dyR[kk][6], dyR[kk][7]));
 
     // Phase 1: dV' = attnᵀ·dY + Kc·dS in [token][column] orientation.
-    // Two-wave workgroups (one wave per SIMD) split each k-step's dS
-    // fragments under the previous step's MFMAs (the first under attnᵀ·dY),
-    // one MFMA to three VALU instructions: config 5's reverse scan 1010 →
-    // 893 µs. With two waves per SIMD the other wave covers the split, and
-    // so interleaved the eight-wave scan measured slower (875 → 904 µs).
-    constexpr bool kPipe = WAVES == 2;
     f32x4 dV[4];
 #pragma unroll
     for (int tb = 0; tb < 4; ++tb) dV[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if constexpr (kPipe) {
-      uint4 sh = frag_hi(dS[0], dS[1]);
-      uint4 sl = frag_lo(dS[0], dS[1], sh);
 #pragma unroll
-      for (int tb = 0; tb < 4; ++tb)
+    for (int tb = 0; tb < 4; ++tb)
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk)
-          dV[tb] = mfma16(ld8(&tl[oAt + tile_at<kL>(16 * tb + r16, 32 * kk + k8)]),
-                          as8(dyf[kk]), dV[tb]);
+      for (int kk = 0; kk < 2; ++kk)
+        dV[tb] = mfma16(ld8(&tl[oAt + tile_at<kL>(16 * tb + r16, 32 * kk + k8)]),
+                        as8(dyf[kk]), dV[tb]);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-        __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);  // three VALU
-      }
+    for (int kk = 0; kk < KK; ++kk) {
+      const uint4 sh = frag_hi(dS[2 * kk], dS[2 * kk + 1]);
+      const uint4 sl = frag_lo(dS[2 * kk], dS[2 * kk + 1], sh);
 #pragma unroll
-      for (int kk = 0; kk < KK; ++kk) {
-        uint4 shn = sh, sln = sl;
-        if (kk + 1 < KK) {
-          shn = frag_hi(dS[2 * kk + 2], dS[2 * kk + 3]);
-          sln = frag_lo(dS[2 * kk + 2], dS[2 * kk + 3], shn);
-        }
-#pragma unroll
-        for (int tb = 0; tb < 4; ++tb) {
-          const bf16x8 kf = ld8(&tl[oKc + tile_at<K>(16 * tb + r16, 32 * kk + k8)]);
-          dV[tb] = mfma16(kf, as8(sh), dV[tb]);
-          dV[tb] = mfma16(kf, as8(sl), dV[tb]);
-        }
-        if (kk + 1 < KK) {
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-            __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);  // three VALU
-          }
-        }
-        sh = shn;
-        sl = sln;
-      }
-    } else {
-#pragma unroll
-      for (int tb = 0; tb < 4; ++tb)
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk)
-          dV[tb] = mfma16(ld8(&tl[oAt + tile_at<kL>(16 * tb + r16, 32 * kk + k8)]),
-                          as8(dyf[kk]), dV[tb]);
-#pragma unroll
-      for (int kk = 0; kk < KK; ++kk) {
-        const uint4 sh = frag_hi(dS[2 * kk], dS[2 * kk + 1]);
-        const uint4 sl = frag_lo(dS[2 * kk], dS[2 * kk + 1], sh);
-#pragma unroll
-        for (int tb = 0; tb < 4; ++tb) {
-          const bf16x8 kf = ld8(&tl[oKc + tile_at<K>(16 * tb + r16, 32 * kk + k8)]);
-          dV[tb] = mfma16(kf, as8(sh), dV[tb]);
-          dV[tb] = mfma16(kf, as8(sl), dV[tb]);
-        }
+      for (int tb = 0; tb < 4; ++tb) {
+        const bf16x8 kf = ld8(&tl[oKc + tile_at<K>(16 * tb + r16, 32 * kk + k8)]);
+        dV[tb] = mfma16(kf, as8(sh), dV[tb]);
+        dV[tb] = mfma16(kf, as8(sl), dV[tb]);
       }
     }
     load_dy(nn);
 
     // Phase 2: Z = Tᵀ·dV' with hi + lo parts of both factors.
-    // (Tᵀ and attnᵀ are upper triangular, but skipping their zero blocks
-    // here measured slower: 1010 → 1265 µs for the two-wave reverse scan of
-    // BASELINE config 5, with the same register use.)
     uint4 vh[2], vl[2];
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
@@ -1472,32 +1404,73 @@ hipError_t launch_intra(const MfmaParams& p, const Dims& d, hipStream_t stream,
   return hipGetLastError();
 }
 
-// Scan workgroup width in waves of 16 value columns. A workgroup holds a CU's
-// LDS, so a scan runs in rounds of one workgroup per CU, each as long as the
-// sequence; a wider workgroup's chunk takes longer, but fewer rounds may do.
-// The width is the one whose rounds cost least, with the time of a chunk as
-// measured at head_k_dim 128, in one round: per-head gates 3.2, 3.6 and 4.0 us
-// at 2, 4 and 8 waves, per-channel 3.4, 3.6 and 5.3 (at head_k_dim 64 the
-// ratios are flatter). In the backward at head_k_dim 128 the states scan and
-// the reverse scan share the device and do not fit on one CU together
-// (`pair`); at 64 they do. us a chunk (forward) and us a call (backward) at 16
-// chunks, narrowest width that fills the device -> this choice: forward dv 256,
-// 48 heads 6.05 -> 3.72 (4 waves), 96 heads 7.11 -> 4.30 (8); dv 128, 96 heads
-// 6.09 -> 3.72; per channel, dv 256, 48 heads 6.62 -> 3.79. Backward dv 256, 24
-// heads 271 -> 232, 48 heads 452 -> 382; dv 128, 96 heads 469 -> 404.
-int scan_waves(const Dims& d, bool backward = false) {
+// How a scan covers the value columns: teams of four waves per 16 columns
+// (mfma_team.hpp), one or two to a workgroup, or workgroups of 4 or 8 waves
+// that each walk 16 columns alone (mfma_scan_kernel).
+struct ScanShape {
+  int teams, waves;  // teams 0: waves alone
+};
+
+// A chunk of one workgroup, in us: a workgroup holds a CU's LDS, so a scan runs
+// in rounds of one workgroup per CU, each as long as the sequence. Measured in
+// one round, at 16 chunks. Narrow workgroups have the shorter chain (a team's
+// chunk is 22 MFMAs a wave against 88, and stages in waves of its own); wide
+// ones stage a chunk's tiles for more columns.
+inline float chunk_us(const Dims& d, ScanShape s) {
+  const bool pc = pc_path(d);
+  if (d.K == 128)
+    return s.teams == 1   ? (pc ? 1.85f : 1.7f)
+           : s.teams == 2 ? (pc ? 2.25f : 2.05f)
+           : s.waves == 4 ? 3.6f
+                          : (pc ? 5.4f : 4.1f);
+  return s.teams == 1   ? (pc ? 1.4f : 1.35f)
+         : s.teams == 2 ? (pc ? 1.65f : 1.6f)
+         : s.waves == 4 ? (pc ? 2.6f : 2.55f)
+                        : (pc ? 3.8f : 2.65f);
+}
+inline size_t scan_rounds(const Dims& d, int columns, int copies) {
+  const size_t wgs = size_t(d.B) * d.H * ((d.V + columns - 1) / columns) * copies;
+  const size_t cus = size_t(device_cu_count());
+  return (wgs + cus - 1) / cus;
+}
+
+// The shape whose rounds cost least. In the backward at head_k_dim 128 the
+// states scan and the reverse scan share the device and do not fit on one CU
+// together (copies); at 64 they do. us a chunk (forward) and us a call
+// (backward) at 16 chunks, the narrowest of 2, 4 and 8 lone waves that fills
+// the device -> this choice: forward dv 256, 16 heads 3.3 -> 1.7, 32 heads
+// 3.2 -> 2.1, 48 heads 6.05 -> 3.7, 96 heads 7.1 -> 4.3; per channel, dv 256,
+// 16 heads 3.5 -> 1.85. Backward dv 256, 16 heads 171 -> 144, 48 heads
+// 452 -> 382; per channel, dv 128, 32 heads 221 -> 199.
+ScanShape scan_shape(const Dims& d, bool backward) {
   // head_k_dim 256: eight waves, whose staging registers (11 per lane) fit
   // beside the 64 of the state's rows.
-  if (d.K == 256) return 8;
-  const size_t cus = size_t(device_cu_count()), copies = backward && d.K == 128 ? 2 : 1;
-  int best = 2;
+  if (d.K == 256) return {0, 8};
+  const int copies = backward && d.K == 128 ? 2 : 1;
+  const ScanShape shapes[] = {{1, 0}, {2, 0}, {0, 4}, {0, 8}};
+  ScanShape best = shapes[0];
   float least = 0.f;
-  for (int w = 2; w <= 8; w *= 2) {
-    if (d.V % (16 * w) != 0) break;
-    const size_t wgs = size_t(d.B) * d.H * (d.V / (16 * w)) * copies;
-    const float t = w == 2 ? 1.f : w == 4 ? (pc_path(d) ? 1.05f : 1.1f) : (pc_path(d) ? 1.6f : 1.25f);
-    const float cost = t * float((wgs + cus - 1) / cus);
-    if (w == 2 || cost < least) {
+  for (const ScanShape& s : shapes) {
+    const int columns = s.teams ? 16 * s.teams : 16 * s.waves;
+    if (!s.teams && d.V % columns != 0) continue;
+    const float cost = chunk_us(d, s) * float(scan_rounds(d, columns, copies));
+    if (least == 0.f || cost < least) {
+      best = s;
+      least = cost;
+    }
+  }
+  return best;
+}
+
+// The scan with the output norm in its y write has lone waves only: 2, 4 or 8,
+// by the same count (3.2 us a chunk at two waves).
+int norm_scan_waves(const Dims& d) {
+  if (d.K == 256) return 8;
+  int best = 2;
+  float least = 3.2f * float(scan_rounds(d, 32, 1));
+  for (int w = 4; w <= 8 && d.V % (16 * w) == 0; w *= 2) {
+    const float cost = chunk_us(d, {0, w}) * float(scan_rounds(d, 16 * w, 1));
+    if (cost < least) {
       best = w;
       least = cost;
     }
@@ -1505,15 +1478,68 @@ int scan_waves(const Dims& d, bool backward = false) {
   return best;
 }
 
-// Segments per sequence for the scans. A scan workgroup holds a CU's LDS,
-// and 8-wave workgroups do about twice the work per CU of the 2-wave ones
-// the unsegmented scan falls back to, while segmenting triples the scans'
-// work (the transitions cover K extra columns, then the outputs). So the
-// sequence is cut only when even 2-wave workgroups would leave half the
-// device idle, into enough segments to fill it with 8-wave workgroups, of
-// at least 16 whole chunks each (head_k_dim 128, head_v_dim a multiple of
-// 128, a sequence of whole chunks).
+// Segments per sequence for a scan by teams, where its three passes (the
+// transitions cover K extra columns; then the carry; then the outputs) cost
+// less than one scan by a twelfth: a pass is its chunks and about 4 us, the
+// carry 3 us a segment (1.3 at head_k_dim 64), two more launches 5. Sequences
+// of 32 whole chunks or more, in segments of 8 or more; the last may be shorter. The
+// segments' buffers must not take a call past the fixed scratch of
+// dn_chunk_fwd_noalloc that its tiles fit. Calls, us, whole and segmented:
+// S=8192 dk=dv=128, 1 head, per channel 190 and 90; 4 heads, per-head gates,
+// dv 256: S=16384 323 and 197, S=8192 166 and 122; dk 64, 2 heads: S=16384 258
+// and 75. 32 heads at S=16384 per channel, 596 us of scans in segments of
+// eight-wave workgroups before, take 514 whole.
+float teams_us(const Dims& d, int V, int P) {
+  Dims s = d;
+  s.B = d.B * P;
+  s.V = V;
+  float least = 0.f;
+  for (int t = 1; t <= 2; ++t) {
+    const float us = chunk_us(d, {t, 0}) * float(scan_rounds(s, 16 * t, 1));
+    if (least == 0.f || us < least) least = us;
+  }
+  return least;
+}
+int teams_of(const Dims& d, int V, int P) {
+  Dims s = d;
+  s.B = d.B * P;
+  s.V = V;
+  return chunk_us(d, {1, 0}) * float(scan_rounds(s, 16, 1)) <=
+                 chunk_us(d, {2, 0}) * float(scan_rounds(s, 32, 1))
+             ? 1
+             : 2;
+}
+size_t seg_bytes(const Dims& d, int P) {
+  const size_t bh = size_t(d.B) * P * d.H, K = size_t(d.K);
+  return P == 1 ? 0 : region(bh * K * K * 4) + 2 * region(bh * K * d.V * 4);
+}
 int seg_parts(const Dims& d) {
+  if (d.K > 128 || d.N < 32 || size_t(d.S) != size_t(d.N) * d.L) return 1;
+  const ScanShape w = scan_shape(d, false);
+  float least = chunk_us(d, w) * float(d.N) *
+                    float(scan_rounds(d, w.teams ? 16 * w.teams : 16 * w.waves, 1)) + 4.f;
+  int best = 1;
+  for (int P = 2; d.N >= 8 * P && P <= 64; P *= 2) {
+    const size_t tiles = tiles_workspace(d);
+    if (tiles <= DN_NOALLOC_SCRATCH_BYTES && tiles + seg_bytes(d, P) > DN_NOALLOC_SCRATCH_BYTES)
+      break;
+    const float n = float((d.N + P - 1) / P);
+    const float cut = n * (teams_us(d, d.V + d.K, P) + teams_us(d, d.V, P)) +
+                      (d.K == 128 ? 3.05f : 1.3f) * float(P) + 13.f;
+    if (cut < 0.92f * least) {
+      best = P;
+      least = cut;
+    }
+  }
+  return best;
+}
+
+// Segments for the scan with the output norm in its y write, which has
+// 8-wave workgroups in both passes: enough to fill the device with them, of
+// at least 16 whole chunks each (head_k_dim 128, head_v_dim a multiple of
+// 128, a sequence of whole chunks), where even 2-wave workgroups would leave
+// half the device idle, since segmenting triples the scans' work.
+int norm_seg_parts(const Dims& d) {
   if (d.K != 128 || d.V % 128 != 0 || size_t(d.S) != size_t(d.N) * d.L) return 1;
   const size_t cus = size_t(device_cu_count());
   if (size_t(d.B) * d.H * (d.V / 32) * 2 > cus) return 1;
@@ -1524,21 +1550,24 @@ int seg_parts(const Dims& d) {
 }
 
 // The segmented scan's buffers, after the tiles in the workspace.
-size_t seg_workspace(const Dims& d) {
-  const int P = seg_parts(d);
-  if (P == 1) return 0;
+void carve_seg(MfmaParams& p, const Dims& d, int P, void* seg_ws) {
   const size_t bh = size_t(d.B) * P * d.H, K = size_t(d.K);
-  return region(bh * K * K * 4) + 2 * region(bh * K * d.V * 4);
-}
-
-void carve_seg(MfmaParams& p, const Dims& d, void* seg_ws) {
-  const size_t bh = size_t(d.B) * seg_parts(d) * d.H, K = size_t(d.K);
   char* base = static_cast<char*>(seg_ws);
   p.seg_m = reinterpret_cast<float*>(base);
   base += region(bh * K * K * 4);
   p.seg_h = reinterpret_cast<float*>(base);
   base += region(bh * K * d.V * 4);
   p.seg_start = reinterpret_cast<float*>(base);
+}
+
+hipError_t launch_carry(const MfmaParams& p, const Dims& d, hipStream_t stream) {
+  ProfScope ps("dn_mfma_seg_carry", stream);
+  const dim3 grid(unsigned(d.B * d.H * (d.V / 16))), block(256);
+  if (d.K == 128)
+    hipLaunchKernelGGL(seg_carry_kernel<128>, grid, block, 0, stream, p);
+  else
+    hipLaunchKernelGGL(seg_carry_kernel<64>, grid, block, 0, stream, p);
+  return hipGetLastError();
 }
 
 // The dims of the segmented scans: batch b·P + s runs segment s of batch b.
@@ -1557,35 +1586,26 @@ hipError_t launch_scan(const MfmaParams& p, const Dims& d, bool yb, hipStream_t 
   const bool pc = pc_path(d);
   if constexpr (!ST) {
     if (p.seg) {
-      // The segmented scans: 8-wave workgroups, head_k_dim 128.
+      // The transitions of the output norm's segmented scan: 8-wave
+      // workgroups, head_k_dim 128.
       const unsigned blocks = unsigned(((d.B * d.H + 7) / 8) * 8 * (p.vx / 128));
-      ProfScope ps(p.seg == 1 ? (pc ? "dn_mfma_scan_pc_segs" : "dn_mfma_scan_segs")
-                              : (pc ? "dn_mfma_scan_pc" : "dn_mfma_scan"),
-                   stream);
-#define DN_SEG(TY, SG)                                                                           \
-  do {                                                                                           \
-    if (pc)                                                                                      \
-      hipLaunchKernelGGL((mfma_scan_kernel<128, TY, 8, true, false, SG>), dim3(blocks),          \
-                         dim3(512), 0, stream, p);                                               \
-    else                                                                                         \
-      hipLaunchKernelGGL((mfma_scan_kernel<128, TY, 8, false, false, SG>), dim3(blocks),         \
-                         dim3(512), 0, stream, p);                                               \
-  } while (0)
-      if (p.seg == 1)
-        DN_SEG(float, 1);  // no y
-      else if (yb)
-        DN_SEG(bf16, 2);
+      ProfScope ps(pc ? "dn_mfma_scan_pc_segs" : "dn_mfma_scan_segs", stream);
+      if (pc)
+        hipLaunchKernelGGL((mfma_scan_kernel<128, float, 8, true, false, 1>), dim3(blocks),
+                           dim3(512), 0, stream, p);
       else
-        DN_SEG(float, 2);
-#undef DN_SEG
+        hipLaunchKernelGGL((mfma_scan_kernel<128, float, 8, false, false, 1>), dim3(blocks),
+                           dim3(512), 0, stream, p);
       return hipGetLastError();
     }
   }
-  const int waves = scan_waves(d, ST);
-  const unsigned blocks = unsigned(((d.B * d.H + 7) / 8) * 8 * (d.V / (16 * waves)));
+  const ScanShape shape = scan_shape(d, ST);
   ProfScope ps(ST ? (pc ? "dn_mfma_scan_pc_states" : "dn_mfma_scan_states")
                   : (pc ? "dn_mfma_scan_pc" : "dn_mfma_scan"),
                stream);
+  if (shape.teams && !g4) return launch_team_scan(p, d.K, pc, ST, yb, shape.teams, stream);
+  const int waves = shape.waves;
+  const unsigned blocks = unsigned(((d.B * d.H + 7) / 8) * 8 * (d.V / (16 * waves)));
 #define DN_SCAN(KD, TY, W)                                                                        \
   do {                                                                                            \
     if (pc)                                                                                       \
@@ -1596,7 +1616,7 @@ hipError_t launch_scan(const MfmaParams& p, const Dims& d, bool yb, hipStream_t 
                          stream, p);                                                              \
   } while (0)
 #define DN_SCAN_W(KD, TY) \
-  do { if (waves == 8) DN_SCAN(KD, TY, 8); else if (waves == 4) DN_SCAN(KD, TY, 4); else DN_SCAN(KD, TY, 2); } while (0)
+  do { if (waves == 8) DN_SCAN(KD, TY, 8); else DN_SCAN(KD, TY, 4); } while (0)
   if constexpr (ST) {
     if (g4) {
       // Eight-wave workgroups (head_k_dim 64, 128, 256).
@@ -1648,7 +1668,7 @@ __global__ __launch_bounds__(256) void zero_words_kernel(unsigned long long* w, 
 size_t norm_words(const Dims& d, int P, int waves) {
   return size_t(d.B) * P * d.H * (d.V / (16 * waves)) * 4 * kL;
 }
-size_t norm_exchange_bytes(const Dims& d) { return region(norm_words(d, seg_parts(d), 2) * 8); }
+size_t norm_exchange_bytes(const Dims& d) { return region(norm_words(d, norm_seg_parts(d), 2) * 8); }
 
 // The output-norm scan's launch geometry for dims `d` (the segmented output
 // pass's dims when seg): workgroup waves and column workgroups per head.
@@ -1659,7 +1679,7 @@ struct NormLaunch {
 };
 NormLaunch norm_launch(const Dims& d, bool seg, bool yb, bool gated) {
   NormLaunch l;
-  l.waves = seg ? 8 : scan_waves(d);
+  l.waves = seg ? 8 : norm_scan_waves(d);
   l.ntile = d.V / (16 * l.waves);
   l.blocks = unsigned(((d.B * d.H + 7) / 8) * 8 * l.ntile);
   l.fn = norm_scan_fn(d.K, pc_path(d), seg, yb, l.waves, gated);
@@ -1721,7 +1741,7 @@ bool mfma_bwd_supported(const Dims& d, int qkv_dtype) {
 }
 
 size_t mfma_fwd_workspace(const Dims& d, bool fused) {
-  return fused ? fused_fwd_workspace(d) : tiles_workspace(d) + seg_workspace(d);
+  return fused ? fused_fwd_workspace(d) : tiles_workspace(d) + seg_bytes(d, seg_parts(d));
 }
 
 hipError_t mfma_fwd(const Dims& d, int y_dtype, const void* q, const void* k, const void* v,
@@ -1734,38 +1754,29 @@ hipError_t mfma_fwd(const Dims& d, int y_dtype, const void* q, const void* k, co
   hipError_t e = launch_intra(p, d, stream, nullptr, fe);
   if (e != hipSuccess) return e;
   const int P = seg_parts(d);
-  if (P == 1) return launch_scan<false>(p, d, y_dtype == DN_BF16, stream);
+  const bool yb = y_dtype == DN_BF16, pc = pc_path(d);
+  if (P == 1) return launch_scan<false>(p, d, yb, stream);
   // Segmented: the segments' transitions, the carry, then the outputs.
-  carve_seg(p, d, static_cast<char*>(ws) + tiles_workspace(d));
-  const Dims ds = seg_dims(d, P);
+  carve_seg(p, d, P, static_cast<char*>(ws) + tiles_workspace(d));
+  p.seg_p = P;
+  p.seg_n = (d.N + P - 1) / P;
   MfmaParams pa = p;
-  pa.B = ds.B;
-  pa.S = ds.S;
-  pa.N = ds.N;
   pa.seg = 1;
-  pa.seg_p = P;
-  pa.vx = d.V + d.K;
-  pa.y = nullptr;
-  if ((e = launch_scan<false>(pa, ds, y_dtype == DN_BF16, stream)) != hipSuccess) return e;
   {
-    ProfScope ps("dn_mfma_seg_carry", stream);
-    MfmaParams pb = p;
-    pb.seg_p = P;
-    hipLaunchKernelGGL(seg_carry_kernel<128>, dim3(unsigned(d.B * d.H * (d.V / 16))), dim3(256),
-                       0, stream, pb);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    ProfScope ps(pc ? "dn_mfma_scan_pc_segs" : "dn_mfma_scan_segs", stream);
+    e = launch_team_scan(pa, d.K, pc, false, yb, teams_of(d, d.V + d.K, P), stream);
+    if (e != hipSuccess) return e;
   }
-  MfmaParams pc = pa;
-  pc.seg = 2;
-  pc.vx = d.V;
-  pc.s_in = p.seg_start;
-  pc.y = y;
-  pc.seg_final = state_out;
-  return launch_scan<false>(pc, ds, y_dtype == DN_BF16, stream);
+  if ((e = launch_carry(p, d, stream)) != hipSuccess) return e;
+  pa.seg = 2;
+  pa.s_in = p.seg_start;
+  pa.seg_final = state_out;
+  ProfScope ps(pc ? "dn_mfma_scan_pc" : "dn_mfma_scan", stream);
+  return launch_team_scan(pa, d.K, pc, false, yb, teams_of(d, d.V, P), stream);
 }
 
 size_t mfma_fwd_norm_workspace(const Dims& d) {
-  return tiles_workspace(d) + seg_workspace(d) + norm_exchange_bytes(d);
+  return tiles_workspace(d) + seg_bytes(d, norm_seg_parts(d)) + norm_exchange_bytes(d);
 }
 
 hipError_t mfma_fwd_norm(const Dims& d, int y_dtype, const void* q, const void* k, const void* v,
@@ -1777,11 +1788,11 @@ hipError_t mfma_fwd_norm(const Dims& d, int y_dtype, const void* q, const void* 
   p.ng_stride = nm.gate_stride;
   p.nw = nm.weight;
   p.neps = nm.eps;
+  const int P = norm_seg_parts(d);
   p.nx = reinterpret_cast<unsigned long long*>(static_cast<char*>(ws) + tiles_workspace(d) +
-                                               seg_workspace(d));
+                                               seg_bytes(d, P));
   p.nfault = nm.fault;
   p.nspin = nm.spin;
-  const int P = seg_parts(d);
   // Whether the scan can run as launched, decided before any launch so that
   // the caller's fallback starts from a clean slate.
   {
@@ -1792,7 +1803,7 @@ hipError_t mfma_fwd_norm(const Dims& d, int y_dtype, const void* q, const void* 
   hipError_t e = launch_intra(p, d, stream);
   if (e != hipSuccess) return e;
   if (P == 1) return launch_scan_norm(p, d, y_dtype == DN_BF16, stream);
-  carve_seg(p, d, static_cast<char*>(ws) + tiles_workspace(d));
+  carve_seg(p, d, P, static_cast<char*>(ws) + tiles_workspace(d));
   const Dims ds = seg_dims(d, P);
   MfmaParams pa = p;
   pa.B = ds.B;
@@ -1803,14 +1814,9 @@ hipError_t mfma_fwd_norm(const Dims& d, int y_dtype, const void* q, const void* 
   pa.vx = d.V + d.K;
   pa.y = nullptr;
   if ((e = launch_scan<false>(pa, ds, y_dtype == DN_BF16, stream)) != hipSuccess) return e;
-  {
-    ProfScope ps("dn_mfma_seg_carry", stream);
-    MfmaParams pb = p;
-    pb.seg_p = P;
-    hipLaunchKernelGGL(seg_carry_kernel<128>, dim3(unsigned(d.B * d.H * (d.V / 16))), dim3(256),
-                       0, stream, pb);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-  }
+  MfmaParams pb = p;
+  pb.seg_p = P;
+  if ((e = launch_carry(pb, d, stream)) != hipSuccess) return e;
   MfmaParams pc = pa;
   pc.seg = 2;
   pc.vx = d.V;
@@ -1866,17 +1872,23 @@ hipError_t mfma_bwd_scans(const Dims& d, int grad_dtype, const void* dy,
   // tiles; eight waves spilled there). At B=8 T=4096 H=16 dv=256: eight
   // waves row-major 5.05 ms, four 3.85, four in row groups 1.61, eight in
   // row groups 1.36.
-  const int waves = d.K == 256 && !g4 ? 4 : scan_waves(d, true);
-  const unsigned blocks = unsigned(((d.B * d.H + 7) / 8) * 8 * (d.V / (16 * waves)));
+  const ScanShape shape = scan_shape(d, true);
+  const int waves = d.K == 256 && !g4 ? 4 : shape.waves;
   {
   ProfScope ps("dn_mfma_rev_scan", side);
+  if (shape.teams) {
+    if (g4) return hipErrorInvalidValue;
+    if ((e = launch_team_rev(rp, d.K, grad_dtype == DN_BF16, shape.teams, side)) != hipSuccess)
+      return e;
+  } else {
+  const unsigned blocks = unsigned(((d.B * d.H + 7) / 8) * 8 * (d.V / (16 * waves)));
 #define DN_REV(KD, TG, W) \
   hipLaunchKernelGGL((mfma_rev_scan_kernel<KD, TG, W>), dim3(blocks), dim3(64 * W), 0, side, rp)
 #define DN_REV4(KD, TG, W)                                                                     \
   hipLaunchKernelGGL((mfma_rev_scan_kernel<KD, TG, W, true>), dim3(blocks), dim3(64 * W), 0,  \
                      side, rp)
 #define DN_REV_W(KD, TG) \
-  do { if (waves == 8) DN_REV(KD, TG, 8); else if (waves == 4) DN_REV(KD, TG, 4); else DN_REV(KD, TG, 2); } while (0)
+  do { if (waves == 8) DN_REV(KD, TG, 8); else DN_REV(KD, TG, 4); } while (0)
   if (g4 && waves != 8 && d.K != 256) return hipErrorInvalidValue;
   if (d.K == 256) {
     if (g4) {
@@ -1898,6 +1910,7 @@ hipError_t mfma_bwd_scans(const Dims& d, int grad_dtype, const void* dy,
 #undef DN_REV_W
 #undef DN_REV4
 #undef DN_REV
+  }
   }
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if ((e = launch_scan<true>(p, d, false, stream, g4)) != hipSuccess) return e;

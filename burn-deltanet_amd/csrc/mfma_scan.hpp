@@ -11,7 +11,6 @@
 #include "mfma_util.hpp"
 
 namespace dn {
-namespace {
 
 constexpr int kL = 64;  // chunk length
 
@@ -44,6 +43,7 @@ struct MfmaParams {
   // start at the identity and see no v) and offset H (the end state from
   // S = 0); 2: outputs and states from the carried segment starts.
   int seg, seg_p;
+  int seg_n;        // chunks per segment (the team scans, whose last segments may be short)
   int vx;           // state columns the launch covers: V, or V + K when seg = 1
   float* seg_m;     // [B·seg_p·H][K][K] M of each segment (seg = 1)
   float* seg_h;     // [B·seg_p·H][K][V] H of each segment (seg = 1)
@@ -67,6 +67,37 @@ struct MfmaParams {
   int* nfault;
   int nspin;
 };
+
+// The backward's transposed tiles. The reverse scan contracts over a chunk's
+// tokens where the forward contracts over its rows, so it reads Tᵀ (hi, lo),
+// attnᵀ, Kc = (Kcᵀ)ᵀ, and Qgᵀ = (scale·e^G⊙Q)ᵀ, Kgᵀ = (e⊙e^G⊙K)ᵀ
+// (combined_backward.rs:272-282: the state cotangent picks up qrᵀ·dy and
+// Wᵀ·dV' = kgᵀ·(Tᵀ·dV')). The intra kernels write them in their BT mode.
+struct BwdTiles {
+  uint16_t *Tt, *Ttl, *AtT;  // [G][64][64]
+  uint16_t* Kc;              // [G][64][K]
+  uint16_t *QgT, *KgT;       // [G][K][64]
+  float* egl;                // [G][K] e^{G_last} per key channel
+};
+
+// The reverse scan (combined_backward.rs:240-319, the dS recurrence).
+struct RevParams {
+  int B, S, H, V, N;
+  const void* dy;            // [B, S, H, V], bf16 or fp32
+  const float* dstate_final;  // [B, H, K, V] or null (zeros)
+  float* ds_after;            // [G][K][V]
+  float* dstate;              // [B, H, K, V] cotangent of the initial state
+  BwdTiles bt;
+};
+
+// The scans with a team of four waves per 16 value columns (chunk_team.hip),
+// `teams` (1 or 2) to a workgroup: head_k_dim 64 and 128.
+hipError_t launch_team_scan(const MfmaParams& p, int K, bool pc, bool states, bool y_bf16,
+                            int teams, hipStream_t stream);
+hipError_t launch_team_rev(const RevParams& p, int K, bool grad_bf16, int teams,
+                           hipStream_t stream);
+
+namespace {
 
 // ---------------------------------------------------------------------------
 // scan

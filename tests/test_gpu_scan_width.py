@@ -1,6 +1,8 @@
-"""The scans' workgroup width (scan_waves) at head counts either side of where
-a wider workgroup saves a round: the bf16 MFMA forward and backward against
-the fp32 kernels, at the bf16 path's bar."""
+"""How the scans cover the device (scan_shape): one or two four-wave teams, or
+4 or 8 lone waves, to a workgroup, at head counts either side of where the
+choice turns, and the team scans' segments where they are uneven or empty. The
+bf16 MFMA forward and backward against the fp32 kernels, at the bf16 path's
+bar."""
 
 import numpy as np
 import pytest
@@ -14,23 +16,55 @@ pytestmark = pytest.mark.gpu
 MFMA, GENERIC = pkg.abi.DN_ALGO_MFMA, pkg.abi.DN_ALGO_GENERIC
 
 
-# H heads of V columns on 256 CUs: forward widths 2 | 4 | 8 with H·V/32, H·V/64
-# and H·V/128 workgroups; the backward's pair of scans reaches each at half.
-@pytest.mark.parametrize("H,K,V,channel", [(32, 128, 256, False), (33, 128, 256, False),
-                                           (65, 128, 256, False), (17, 128, 256, False),
-                                           (65, 64, 64, False), (33, 128, 256, True),
-                                           (66, 64, 128, True)])
-def test_scan_width(rng, H, K, V, channel):
-    announce(f"scan width H {H} K {K} V {V} channel {channel}")
-    args = to_gpu(random_raw(rng, 1, 70, H, K, V, channel=channel), torch.bfloat16)
-    dy = torch.tensor(rng.standard_normal((1, 70, H, V)), device=args[0].device).bfloat16()
+# On 256 CUs, H·V/16 teams: forward one team a workgroup to 256 of them, two to
+# 512, then 4 and 8 lone waves; the backward's pair of scans turns at half.
+@pytest.mark.parametrize("H,K,V,gates", [
+    (3, 128, 64, "none"), (7, 128, 256, "head"), (17, 128, 256, "head"), (32, 128, 256, "head"),
+    (33, 128, 256, "head"), (65, 128, 256, "head"), (5, 64, 192, "none"), (65, 64, 64, "head"),
+    (9, 128, 128, "channel"), (33, 128, 256, "channel"), (66, 64, 128, "channel")])
+@pytest.mark.parametrize("S", [1, 70])
+def test_scan_width(rng, H, K, V, gates, S):
+    announce(f"scan width H {H} K {K} V {V} {gates} S {S}")
+    raw = random_raw(rng, 1, S, H, K, V, gated=gates != "none", channel=gates == "channel")
+    args = to_gpu(raw, torch.bfloat16)
+    dy = torch.tensor(rng.standard_normal((1, S, H, V)), device=args[0].device).bfloat16()
+    ds = torch.tensor(rng.standard_normal((1, H, K, V)), device=args[0].device).float()
     scale = 1.0 / np.sqrt(K)
-    fwd, bwd = {}, {}
+    out = {}
     for algo in (MFMA, GENERIC):
-        fwd[algo] = pkg.delta_chunk_recalculated(*args, True, 64, scale, algo=algo)
-        g = pkg.combined_backward(dy, None, *args, 64, scale, algo=algo)
-        bwd[algo] = (g.d_q_bshk, g.d_k_bshk, g.d_v_bshv, g.d_erase_bshK, g.d_write_bshV,
-                     g.d_g_bshK, g.d_state_bhkv)
+        y, s = pkg.delta_chunk_recalculated(*args, gates != "none", 64, scale, algo=algo)
+        g = pkg.combined_backward(dy, ds, *args, 64, scale, algo=algo)
+        out[algo] = [y, s, g.d_q_bshk, g.d_k_bshk, g.d_v_bshv, g.d_erase_bshK, g.d_write_bshV,
+                     g.d_g_bshK, g.d_state_bhkv]
     torch.cuda.synchronize()
-    for got, want in zip(fwd[MFMA] + bwd[MFMA], fwd[GENERIC] + bwd[GENERIC]):
-        assert rel_err(np_of(got), np_of(want)) < 2e-2
+    # A single token's d_g is a difference of q ⊙ d_q and k ⊙ d_k (bf16 terms).
+    least = max(rel_base(out[GENERIC][2], args[0]), rel_base(out[GENERIC][3], args[1]))
+    for i, (got, want) in enumerate(zip(out[MFMA], out[GENERIC])):
+        if want is not None:
+            scale_ = max(np.abs(np_of(want)).max(), least if i == 7 else 0.0)
+            assert np.abs(np_of(got) - np_of(want)).max() / scale_ < 2e-2, i
+
+
+def rel_base(grad, x):
+    return float(np.abs(np_of(grad) * np_of(x)).max())
+
+
+@pytest.mark.parametrize("N,K,V,gates", [(50, 128, 64, "head"), (45, 64, 128, "head"),
+                                         (41, 128, 64, "channel"), (37, 64, 64, "none"),
+                                         (161, 128, 64, "head")])  # the last segment is empty
+def test_uneven_segments(rng, N, K, V, gates):
+    announce(f"uneven segments N {N} K {K} V {V} {gates}")
+    args = to_gpu(random_raw(rng, 1, 64 * N, 1, K, V, gated=gates != "none",
+                             channel=gates == "channel"), torch.bfloat16)
+    run = lambda algo: pkg.delta_chunk_recalculated(*args, gates != "none", 64, 1.0 / np.sqrt(K),
+                                                    algo=algo, y_dtype=torch.float32)
+    want = run(GENERIC)
+    torch.cuda.synchronize()
+    pkg.abi.profile_enable(True)
+    got = run(MFMA)
+    torch.cuda.synchronize()
+    names = pkg.abi.profile_read()
+    pkg.abi.profile_enable(False)
+    assert "dn_mfma_seg_carry" in names, names
+    for a, b in zip(got, want):
+        assert rel_err(np_of(a), np_of(b)) < 2e-2
