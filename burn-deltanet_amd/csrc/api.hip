@@ -649,7 +649,11 @@ int dn_chunk_bwd(const dn_chunk_bwd_args* a, hipStream_t stream) {
     const bool g4 = states_g4(d);
     e = mfma_bwd_scans(d, a->grad_dtype, a->d_y, a->d_state_final, a->q, a->k, a->v, a->erase,
                        a->write, g, a->state_in, states, ds_after, a->d_state, mws, stream, g4);
-    if (e == hipSuccess)
+    if (e == hipSuccess && local_bwd_takes(d))
+      e = local_bwd(d, a->grad_dtype, a->d_y, a->q, a->k, a->v, a->erase, a->write, g, states,
+                    ds_after, a->d_q, a->d_k, a->d_v, a->d_erase, a->d_write,
+                    a->has_gate ? a->d_g : nullptr, mfma_bwd_tiles(d, mws), stream);
+    else if (e == hipSuccess)
       e = mfma_chunk_bwd(
           d, a->grad_dtype, a->d_y, a->q, a->k, a->v, a->erase, a->write, g, states, ds_after,
           a->d_q, a->d_k, a->d_v, a->d_erase, a->d_write, a->has_gate ? a->d_g : nullptr,

@@ -1,7 +1,7 @@
 // The fp32 chunk backward (chunk_f32.hpp): the reverse scan and the
 // chunk-local gradients. combined_backward.rs:72-513 with the identities of
 // the bf16 kernels: dT = dV'·Xᵀ and d_kg = −(Tᵀ·dV')·S₀ᵀ.
-#include "chunk_f32.hpp"
+#include "chunk_bwd_tail.hpp"
 
 namespace dn {
 namespace {
@@ -174,9 +174,7 @@ __global__ __launch_bounds__(256 * C) void f32_rev_scan_kernel(FParams p) {
 // time, double-buffered through LDS (one barrier a step): wave w owns key
 // channels 16w … 16w+15 and sums V'·dSᵀ, dY·S₀ᵀ and Z·S₀ᵀ for all 64 tokens,
 // 48 accumulator registers; the ten lower blocks of dY·V'ᵀ and dV'·Xᵀ are
-// dealt over the waves. Then dAkk = −tril(Tᵀ·dT·Tᵀ, −1) through LDS, and the
-// score backward per channel block, its k, q and gates in registers in the
-// accumulators' own layout.
+// dealt over the waves. Then the score backward (chunk_bwd_tail).
 template <int KB, bool PCG, bool EK, class TQ, class TG>
 __global__ __launch_bounds__(64 * (KB < 4 ? 4 : KB)) void f32_chunk_bwd_kernel(FParams p) {
   constexpr bool kFold = PCG || EK;
@@ -199,18 +197,11 @@ __global__ __launch_bounds__(64 * (KB < 4 ? 4 : KB)) void f32_chunk_bwd_kernel(F
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m16 = lane & 15, g4 = lane >> 4;
   const int fo = (g4 * 16 + (m16 ^ g4)) * 4;
-  int to[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) to[r] = blk(4 * g4 + r, m16);
-  auto tr = [&](const float* x) { return f32x4{x[to[0]], x[to[1]], x[to[2]], x[to[3]]}; };
   const int rl = min(kC, d.S - n * kC);
   const size_t row0 = (size_t(b) * d.S + size_t(n) * kC) * d.H + h;
   const float* ws = p.ws + size_t(cid) * o.per;
-  const TQ* qp = static_cast<const TQ*>(p.q);
-  const TQ* kp = static_cast<const TQ*>(p.k);
   const TQ* vp = static_cast<const TQ*>(p.v);
   const TG* dyp = static_cast<const TG*>(p.dy);
-  const bool gated = d.dw > 0;
 
   // --- phase B ---------------------------------------------------------------
   // Waves 0 … 3 load token block `wave` of dY and of Z, with v and the write
@@ -327,271 +318,11 @@ __global__ __launch_bounds__(64 * (KB < 4 ? 4 : KB)) void f32_chunk_bwd_kernel(F
   if (!PCG && tid < kC) sG[tid] = ws[o.vec + 192 + tid];
   __syncthreads();
 
-  // --- phase C: dAkk and the decayed score cotangents -------------------------
-  float *lT = lds, *lD = lds + kTri, *lP = lds + 2 * kTri, *rkk = lds + 3 * kTri,
-        *rqk = lds + 4 * kTri;
+  float *lT = lds;
   for (int i = tid; i < kTri / 4; i += 64 * NW) st4(&lT[4 * i], ld4(ws + o.t + 4 * i));
-#pragma unroll
-  for (int u = 0; u < NP; ++u) {
-    const int pr = wave + NW * u;
-    if (pr >= 10) continue;
-    const int ti = pr < 1 ? 0 : pr < 3 ? 1 : pr < 6 ? 2 : 3, tj = pr - tri_blk(ti, 0);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = 16 * ti + 4 * g4 + r, j = 16 * tj + m16;
-      const float m = PCG ? 1.f : expf(sG[i] - sG[j]);
-      lD[pr * kBlk + to[r]] = dtt[u][r];
-      rqk[pr * kBlk + to[r]] = j <= i ? dat[u][r] * m : 0.f;
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int u = 0; u < NP; ++u) {
-    const int pr = wave + NW * u;
-    if (pr >= 10) continue;
-    const int ti = pr < 1 ? 0 : pr < 3 ? 1 : pr < 6 ? 2 : 3, tj = pr - tri_blk(ti, 0);
-    f32x4 acc = zero4();  // (dT·Tᵀ)(ti, tj)
-    for (int bi = 0; bi <= tj; ++bi)
-      acc = mm(ld4(&lD[tri_blk(ti, bi) * kBlk + fo]), ld4(&lT[tri_blk(tj, bi) * kBlk + fo]), acc);
-    st4(&lP[pr * kBlk + 4 * lane], acc);
-  }
-  __syncthreads();
-#pragma unroll
-  for (int u = 0; u < NP; ++u) {
-    const int pr = wave + NW * u;
-    if (pr >= 10) continue;
-    const int ti = pr < 1 ? 0 : pr < 3 ? 1 : pr < 6 ? 2 : 3, tj = pr - tri_blk(ti, 0);
-    f32x4 acc = zero4();  // (Tᵀ·dT·Tᵀ)(ti, tj)
-    for (int ai = ti; ai < 4; ++ai)
-      acc = mm(tr(&lT[tri_blk(ai, ti) * kBlk]), ld4(&lP[tri_blk(ai, tj) * kBlk + 4 * lane]), acc);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = 16 * ti + 4 * g4 + r, j = 16 * tj + m16;
-      const float m = PCG ? 1.f : expf(sG[i] - sG[j]);
-      rkk[pr * kBlk + to[r]] = j < i ? -acc[r] * m : 0.f;
-    }
-  }
-  __syncthreads();
-
-  // --- phase D: per key channel ------------------------------------------------
-  if (wave < KB) {
-    const int c = 16 * wave + m16, cc = min(c, d.K - 1);
-    const bool cok = c < d.K;
-    f32x4 k[4], q[4], e[4], G[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int tok = 16 * t + 4 * g4 + r;
-        const size_t row = row0 + size_t(min(tok, rl - 1)) * d.H;
-        const bool ok = cok && tok < rl;
-        const float kx = ld(kp, row * d.K + cc), qx = ld(qp, row * d.K + cc);
-        const float ex = p.erase[EK ? row * d.K + cc : row];
-        const float gx = PCG ? p.g[row * d.K + cc] : 0.f;
-        k[t][r] = ok ? kx : 0.f;
-        q[t][r] = ok ? qx * d.scale : 0.f;
-        e[t][r] = ok ? ex : 0.f;
-        G[t][r] = PCG ? (ok ? gx : 0.f) : sG[tok];
-      }
-    float Gl;
-    if constexpr (PCG) {
-      // Cumulative sums down the channel: within a lane's four rows, over the
-      // four lane groups of a block, then over the blocks.
-      float base = 0.f;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-#pragma unroll
-        for (int r = 1; r < 4; ++r) G[t][r] += G[t][r - 1];
-        float x = G[t][3];
-        float up = __shfl_up(x, 16, 64);
-        if (g4 >= 1) x += up;
-        up = __shfl_up(x, 32, 64);
-        if (g4 >= 2) x += up;
-        const float ex = base + (x - G[t][3]);
-        base += __shfl(x, 48 + m16, 64);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) G[t][r] += ex;
-      }
-      Gl = base;
-    } else {
-      Gl = sG[63];
-    }
-    f32x4 dG[4];
-    float carry = 0.f;
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float eg = expf(G[t][r]), ec = expf(Gl - G[t][r]);
-        const float dkg_ = -dkg[t][r];
-        const float cr = dkc[t][r] * k[t][r] * ec;
-        carry += cr;
-        dG[t][r] = (dqr[t][r] * q[t][r] + dkg_ * k[t][r] * e[t][r]) * eg - cr;
-        dkc[t][r] *= ec;        // → d_k
-        dqr[t][r] *= eg;        // → d_q
-        dkg[t][r] = dkg_ * eg;  // → d(e⊙k)
-      }
-    carry += degl * expf(Gl);
-    carry += __shfl_xor(carry, 16, 64);
-    carry += __shfl_xor(carry, 32, 64);
-    if (g4 == 3) dG[3][3] += carry;
-
-    if constexpr (!PCG) {
-      // head_scores_backward (combined_backward.rs:376-416); the gate's share,
-      // Σ_j of the masked score cotangents against the raw scores, is per row
-      // Σ_c of the products below against ke, q and k.
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        f32x4 a1 = zero4(), a2 = zero4(), a3 = zero4();
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if (j <= t) {
-            a1 = mm(ld4(&rkk[tri_blk(t, j) * kBlk + fo]), k[j], a1);
-            a2 = mm(ld4(&rqk[tri_blk(t, j) * kBlk + fo]), k[j], a2);
-          }
-          if (j >= t) {
-            f32x4 ke;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) ke[r] = k[j][r] * e[j][r];
-            a3 = mm(tr(&rkk[tri_blk(j, t) * kBlk]), ke, a3);
-            a3 = mm(tr(&rqk[tri_blk(j, t) * kBlk]), q[j], a3);
-          }
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          dkg[t][r] += a1[r];
-          dqr[t][r] += a2[r];
-          dkc[t][r] += a3[r];
-          dG[t][r] += k[t][r] * e[t][r] * a1[r] + q[t][r] * a2[r] - k[t][r] * a3[r];
-        }
-      }
-    } else {
-      // channel_scores_backward (combined_backward.rs:421-513): row block pb
-      // through its reference token 8; a clamped exponent passes no gradient.
-#pragma unroll
-      for (int pb = 0; pb < 4; ++pb) {
-        const float Gr = __shfl(G[pb][0], 32 + m16, 64);
-        f32x4 rf, rk, rq, accE = zero4(), accQ = zero4();
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          rf[r] = expf(fminf(G[pb][r] - Gr, kMaxExp));
-          rk[r] = k[pb][r] * e[pb][r] * rf[r];
-          rq[r] = q[pb][r] * rf[r];
-        }
-        float dref = 0.f;
-#pragma unroll
-        for (int jb = 0; jb <= pb; ++jb) {
-          __builtin_amdgcn_sched_barrier(0);  // one block pair's factors at a time
-          f32x4 ce, cb;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            ce[r] = expf(fminf(Gr - G[jb][r], kMaxExp));
-            cb[r] = k[jb][r] * ce[r];
-          }
-          const float *xk = &rkk[tri_blk(pb, jb) * kBlk], *xq = &rqk[tri_blk(pb, jb) * kBlk];
-          accE = mm(ld4(xk + fo), cb, accE);
-          accQ = mm(ld4(xq + fo), cb, accQ);
-          f32x4 dc = mm(tr(xk), rk, zero4());
-          dc = mm(tr(xq), rq, dc);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            dkc[jb][r] += dc[r] * ce[r];
-            const float x = Gr - G[jb][r] >= kMaxExp ? 0.f : dc[r] * cb[r];
-            dG[jb][r] -= x;
-            dref += x;
-          }
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          dkg[pb][r] += accE[r] * rf[r];
-          dqr[pb][r] += accQ[r] * rf[r];
-          const float x =
-              G[pb][r] - Gr >= kMaxExp ? 0.f : accE[r] * rk[r] + accQ[r] * rq[r];
-          dG[pb][r] += x;
-          dref -= x;
-        }
-        dref += __shfl_xor(dref, 16, 64);
-        dref += __shfl_xor(dref, 32, 64);
-        if (g4 == 2) dG[pb][0] += dref;
-        // Left to itself the compiler moves these sums into the stores at the
-        // end, every term of them live until then.
-#pragma unroll
-        for (int t = 0; t <= pb; ++t) asm volatile("" : "+v"(dkc[t]), "+v"(dG[t]));
-        asm volatile("" : "+v"(dkg[pb]), "+v"(dqr[pb]));
-      }
-    }
-    // Front end (combined_backward.rs:153-188).
-    if constexpr (PCG) {
-      // d_g: the reverse of the cumulative sum.
-      float base = 0.f;
-#pragma unroll
-      for (int t = 3; t >= 0; --t) {
-#pragma unroll
-        for (int r = 2; r >= 0; --r) dG[t][r] += dG[t][r + 1];
-        float x = dG[t][0];
-        float dn = __shfl_down(x, 16, 64);
-        if (g4 <= 2) x += dn;
-        dn = __shfl_down(x, 32, 64);
-        if (g4 <= 1) x += dn;
-        const float ex = base + (x - dG[t][0]);
-        base += __shfl(x, m16, 64);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) dG[t][r] += ex;
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int tok = 16 * t + 4 * g4 + r;
-        const size_t at = (row0 + size_t(tok) * d.H) * d.K + c;
-        const float de = dkg[t][r] * k[t][r];
-        if (cok && tok < rl) {
-          st(static_cast<TG*>(p.dq), at, dqr[t][r] * d.scale);
-          st(static_cast<TG*>(p.dk), at, dkc[t][r] + dkg[t][r] * e[t][r]);
-          if constexpr (EK) p.derase[at] = de;
-          if constexpr (PCG)
-            if (p.dg) p.dg[at] = dG[t][r];
-        }
-        // Width-1 gates: sums over the key channels, per token (channels past
-        // head_k_dim hold zeros).
-        if constexpr (!EK || !PCG) {
-          float x = EK ? 0.f : de, y = PCG ? 0.f : dG[t][r];
-#pragma unroll
-          for (int s = 1; s < 16; s *= 2) {
-            if constexpr (!EK) x += __shfl_xor(x, s, 64);
-            if constexpr (!PCG) y += __shfl_xor(y, s, 64);
-          }
-          if (m16 == 0) {
-            red[0][wave][tok] = x;
-            red[1][wave][tok] = y;
-          }
-        }
-      }
-  }
-  if constexpr (!EK || !PCG) {
-    __syncthreads();
-    if (wave == 0) {
-      float x = 0.f, y = 0.f;
-#pragma unroll
-      for (int w = 0; w < KB; ++w) {
-        x += red[0][w][lane];
-        y += red[1][w][lane];
-      }
-      // d_g of a token sums the cumulative gate's cotangents from it on.
-#pragma unroll
-      for (int s = 1; s < 64; s *= 2) {
-        const float dn = __shfl_down(y, s, 64);
-        if (lane + s < 64) y += dn;
-      }
-      if (lane < rl) {
-        const size_t row = row0 + size_t(lane) * d.H;
-        if constexpr (!EK) p.derase[row] = x;
-        if constexpr (!PCG)
-          if (gated && p.dg) p.dg[row] = y;
-      }
-    }
-  }
+  const ChunkTail x{d, row0, rl, p.erase, p.g, p.derase, p.dg};
+  chunk_bwd_tail<KB, NW, PCG, EK>(x, DirectRows<TQ, TG>{x, p.q, p.k, p.dq, p.dk}, lds, red, sG,
+                                  dkc, dqr, dkg, dat, dtt, degl);
 }
 
 hipError_t launch_rev(const FParams& p, int grad_dtype, hipStream_t stream) {

@@ -189,9 +189,7 @@ hipError_t fused_fwd(const Dims& d, int y_dtype, const void* q, const void* k, c
 // MFMA chunk-local kernel reads; where states_g4(d) holds, at head_k_dim
 // 256 (B=8 T=4096 H=16 dv=256: states scan 2543 → 692 µs, reverse scan
 // 3846 → 1623 µs, the chunk-local kernel 5.29 → 5.95 ms, whose key-channel
-// phase reads a row as 16-byte-strided words there). At head_k_dim 128 the
-// scans gained 80 µs each at dv = 256 and the chunk-local kernel lost 260;
-// BASELINE config 5's two-wave scans were slower with it.
+// phase reads a row as 16-byte-strided words there).
 size_t mfma_bwd_workspace(const Dims& d);
 bool states_g4(const Dims& d);
 hipError_t mfma_bwd_scans(const Dims& d, int grad_dtype, const void* dy,
@@ -207,10 +205,20 @@ struct MfmaTiles {
   const float* gc;
 };
 MfmaTiles mfma_bwd_tiles(const Dims& d, void* ws);
-// The chunk-local gradients on MFMA (head_v_dim 64, or a multiple of 128 in
-// passes of 128 value columns, on top of the shapes of mfma_fwd_supported),
-// after mfma_bwd_scans. `partials`: mfma_chunk_bwd_partials(d) bytes of
-// workspace for the value-summed gradients between passes.
+// The chunk-local gradients at head_k_dim 64 and 128, after mfma_bwd_scans:
+// the shapes it has, and those among them that mfma_chunk_bwd does not keep.
+bool local_bwd_supported(const Dims& d);
+bool local_bwd_takes(const Dims& d);
+hipError_t local_bwd(const Dims& d, int grad_dtype, const void* dy, const void* q, const void* k,
+                     const void* v, const float* erase, const float* write, const float* g,
+                     const float* states, const float* ds_after, void* dq, void* dk, void* dv,
+                     float* derase, float* dwrite, float* dg, const MfmaTiles& tiles,
+                     hipStream_t stream);
+// The chunk-local gradients on MFMA, after mfma_bwd_scans: whether either
+// kernel has the call, and the one for per-head gates at head_k_dim 256 (in
+// passes of 128 value columns) or at 64 with head_v_dim 64 or 128.
+// `partials`: mfma_chunk_bwd_partials(d) bytes of workspace for the
+// value-summed gradients between passes.
 bool mfma_chunk_bwd_supported(const Dims& d, int qkv_dtype);
 size_t mfma_chunk_bwd_partials(const Dims& d);
 hipError_t mfma_chunk_bwd(const Dims& d, int grad_dtype, const void* dy, const void* q,
