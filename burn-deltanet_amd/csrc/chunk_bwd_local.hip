@@ -26,9 +26,9 @@
 // 256 the eight steps' products take 36000 and their waits on loads 26000,
 // the fp32 tail 32000. q and k pass through LDS tiles in the tail, and their
 // gradients leave by whole rows: two-byte accesses of a lane's own tokens
-// took 30000 cycles there. All of the kernel with 64 heads of 64 chunks
-// (B=8 T=2048 H=16 dk=128 dv=256, per-head gates): 1190 us in two passes,
-// 715 here; per-channel gates, B=2 T=16384 H=8: 1600 and 1341.
+// took 30000 cycles there. All of the kernel at B=8 T=2048 H=16
+// dk=128 dv=256, per-head gates: 1190 us in two passes, 715 here; at B=2
+// T=16384 H=16 dk=dv=128, per-channel gates: 1600 and 1341.
 #include "chunk_bwd_tail.hpp"
 
 namespace dn {

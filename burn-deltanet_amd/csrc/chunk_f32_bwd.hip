@@ -197,6 +197,9 @@ __global__ __launch_bounds__(64 * (KB < 4 ? 4 : KB)) void f32_chunk_bwd_kernel(F
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m16 = lane & 15, g4 = lane >> 4;
   const int fo = (g4 * 16 + (m16 ^ g4)) * 4;
+  int to[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) to[r] = blk(4 * g4 + r, m16);
   const int rl = min(kC, d.S - n * kC);
   const size_t row0 = (size_t(b) * d.S + size_t(n) * kC) * d.H + h;
   const float* ws = p.ws + size_t(cid) * o.per;
