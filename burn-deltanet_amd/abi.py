@@ -244,7 +244,9 @@ def ptr(t):
 
 
 def stream_handle():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    # torch.cuda.current_stream() builds a Stream object for the same handle
+    # (2.9 us against 0.4, in calls of 15 to 30 us).
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
 
 
 def nan_scale(scale):

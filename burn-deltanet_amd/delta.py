@@ -151,15 +151,16 @@ class DeltaInput:
 
 
 def _expect(t: Tensor, shape, what):
-    if tuple(t.shape) != tuple(shape):
+    if t.shape != shape:
         raise DeltaError(-2, f"{what}: expected shape {list(shape)}, got {list(t.shape)}")
 
 
 def _gate_axis(t: Tensor, lead, full, what):
     n = len(lead)
-    if t.dim() != n + 1 or tuple(t.shape[:n]) != tuple(lead):
+    at = t.shape
+    if len(at) != n + 1 or at[:n] != lead:
         raise DeltaError(-2, f"{what}: expected leading dims {list(lead)}, got {list(t.shape)}")
-    if t.shape[n] not in (1, full):
+    if at[n] != 1 and at[n] != full:
         raise DeltaError(-3, f"{what}: last axis must be 1 or {full}, got {t.shape[n]}")
 
 
@@ -305,13 +306,10 @@ def combined_backward(d_y_bshv, d_final_state_bhkv, q_bshk, k_bshk, v_bshv, eras
     gdt = d_y_bshv.dtype if d_y_bshv.dtype in (torch.float32, torch.bfloat16) else torch.float32
     dy = _dev(d_y_bshv, gdt)
     ds = _dev(d_final_state_bhkv, torch.float32)
-    grads = (torch.empty(q.shape, dtype=gdt, device=q.device),
-             torch.empty(k.shape, dtype=gdt, device=q.device),
-             torch.empty(v.shape, dtype=gdt, device=q.device),
-             torch.empty(e.shape, dtype=torch.float32, device=q.device),
-             torch.empty(w.shape, dtype=torch.float32, device=q.device),
-             None if g is None else torch.empty(g.shape, dtype=torch.float32, device=q.device),
-             torch.empty(s.shape, dtype=torch.float32, device=q.device))
+    new = lambda t, dt=torch.float32: torch.empty_like(t, dtype=dt,
+                                                       memory_format=torch.contiguous_format)
+    grads = (new(q, gdt), new(k, gdt), new(v, gdt), new(e), new(w),
+             None if g is None else new(g), new(s))
     args = abi.chunk_bwd_args(dy, ds, q, k, v, e, w, g, s, grads, chunk_len, scale, algo=algo,
                               check_finite=check_finite)
     _own_workspace(args, abi.lib().dn_chunk_bwd_workspace_bytes(args), q.device)
@@ -327,6 +325,9 @@ class DeltaChunkFunction(torch.autograd.Function):
     def forward(ctx, q, k, v, erase, write, g, state, chunk_len, scale, check_finite):
         y, s_out = delta_chunk_recalculated(q, k, v, erase, write, g, state, g is not None,
                                             chunk_len, scale, check_finite=check_finite)
+        # An output without a gradient arrives as None: no zeros to allocate and
+        # fill for the final state that a training step does not read.
+        ctx.set_materialize_grads(False)
         ctx.save_for_backward(q, k, v, erase, write, g, state)
         ctx.chunk_len, ctx.scale, ctx.check_finite = chunk_len, scale, check_finite
         return y, s_out
