@@ -221,16 +221,16 @@ __global__ __launch_bounds__(256) void f32_intra_kernel(FParams p) {
 // reverse, which evens out the triangular products of the waves that share a
 // SIMD. ST: the state entering each chunk, X and V' go to the workspace, no y.
 template <int KB, int C, bool FOLD, bool ST, class TV, class TY>
-__global__ __launch_bounds__(256 * C) void f32_scan_kernel(FParams p) {
+__global__ __launch_bounds__(256 * C + 256) void f32_scan_kernel(FParams p) {
   constexpr Lay o = lay(KB, FOLD);
-  constexpr int NT = 256 * C;
-  constexpr int kCopy = (ST ? o.q : o.vec) / 4;  // 16-byte words of a chunk's tiles
-  constexpr int NPF = (kCopy + NT - 1) / NT;
-  constexpr int kVec = 4 * kC + 16 * KB;         // xe, ys, gk, G, egl
-  constexpr int NPV = (kVec + NT - 1) / NT;
-  constexpr int NR = (KB + 3) / 4;               // state row blocks per wave
-  __shared__ __attribute__((aligned(16))) float tl[kCopy * 4];
-  __shared__ __attribute__((aligned(16))) float vec[kVec];
+  constexpr int kTile = 4 * KB * kBlk;
+  constexpr int kVec = 4 * kC + 16 * KB;  // xe, ys, gk, G, egl
+  constexpr int NR = (KB + 3) / 4;        // state row blocks per wave
+  // One buffer is enough for what one phase alone reads: a chunk's phases 1, 2
+  // and 3 end at a barrier each, and the other two leave time to replace it.
+  constexpr int kQ = ST ? 16 : kTile, kAt = ST ? 16 : kTri, kU = FOLD ? kTile : 16;
+  __shared__ __attribute__((aligned(16))) float tA[FOLD ? 1 : 2][kTile], tU[kU], tQ[kQ], tT[kTri],
+      tAt[kAt], vecs[2][kVec];
   __shared__ __attribute__((aligned(16))) float Sx[C][KB * kBlk];
   __shared__ __attribute__((aligned(16))) float Xx[C][4 * kBlk], Vx[C][4 * kBlk];
 
@@ -250,6 +250,65 @@ __global__ __launch_bounds__(256 * C) void f32_scan_kernel(FParams p) {
   int to[4];  // the transposed read's words
 #pragma unroll
   for (int r = 0; r < 4; ++r) to[r] = blk(4 * g4 + r, m16);
+  auto chunk = [&](int n) { return (size_t(b) * d.N + n) * d.H + h; };
+  if (__builtin_amdgcn_readfirstlane(wave) >= 4 * C) {
+    // --- the staging waves ---
+    const int t = tid - 256 * C, last = d.N - 1;
+    auto src = [&](int n) { return p.ws + chunk(min(n, last)) * o.per; };
+    Piece<kTile> a;
+    Piece<kU> u;
+    Piece<kQ> q;
+    Piece<kTri> T;
+    Piece<kAt> at;
+    Piece<kVec> v;
+    a.load(src(0) + o.a, t);
+    T.load(src(0) + o.t, t);
+    v.load(src(0) + o.vec, t);
+    if constexpr (!ST) q.load(src(0) + o.q, t);
+    a.store(tA[0], t);
+    T.store(tT, t);
+    v.store(vecs[0], t);
+    if constexpr (!ST) q.store(tQ, t);
+    if constexpr (FOLD) u.load(src(0) + o.u, t);
+    if constexpr (!ST) at.load(src(0) + o.at, t);
+    a.load(src(1) + o.a, t);
+    v.load(src(1) + o.vec, t);
+    if constexpr (!ST) q.load(src(1) + o.q, t);
+    T.load(src(1) + o.t, t);
+    __syncthreads();
+    for (int n = 0; n < d.N; ++n) {
+      // Beside phase 1: what phase 3 reads, and the next chunk's other halves.
+      if constexpr (FOLD) {
+        u.store(tU, t);
+        u.load(src(n + 1) + o.u, t);
+      } else {
+        a.store(tA[(n + 1) & 1], t);
+        a.load(src(n + 2) + o.a, t);
+      }
+      if constexpr (!ST) {
+        at.store(tAt, t);
+        at.load(src(n + 1) + o.at, t);
+      }
+      v.store(vecs[(n + 1) & 1], t);
+      v.load(src(n + 2) + o.vec, t);
+      lds_barrier();
+      // Beside phase 2: the next chunk's operands of phase 1.
+      if constexpr (FOLD) {
+        a.store(tA[0], t);
+        a.load(src(n + 2) + o.a, t);
+      }
+      if constexpr (!ST) {
+        q.store(tQ, t);
+        q.load(src(n + 2) + o.q, t);
+      }
+      lds_barrier();
+      // Beside phase 3: the next chunk's T.
+      T.store(tT, t);
+      T.load(src(n + 2) + o.t, t);
+      lds_barrier();
+    }
+    return;
+  }
   const int ct = tile * C + team, col = 16 * ct + m16;
   const bool live = col < d.V;
   const int cl = min(col, d.V - 1);
@@ -268,24 +327,6 @@ __global__ __launch_bounds__(256 * C) void f32_scan_kernel(FParams p) {
     }
     if (rb < KB) st4(&Sx[team][rb * kBlk + 4 * lane], S[i]);
   }
-  auto chunk = [&](int n) { return (size_t(b) * d.N + n) * d.H + h; };
-  f32x4 pf[NPF];
-  float pv[NPV];
-  auto fetch = [&](int n) {
-    const float* src = p.ws + chunk(n) * o.per;
-#pragma unroll
-    for (int i = 0; i < NPF; ++i) pf[i] = ld4(src + 4 * min(tid + NT * i, kCopy - 1));
-#pragma unroll
-    for (int i = 0; i < NPV; ++i) pv[i] = src[o.vec + min(tid + NT * i, kVec - 1)];
-  };
-  auto stage = [&] {
-#pragma unroll
-    for (int i = 0; i < NPF; ++i)
-      if (NT * (i + 1) <= kCopy || tid + NT * i < kCopy) st4(&tl[4 * (tid + NT * i)], pf[i]);
-#pragma unroll
-    for (int i = 0; i < NPV; ++i)
-      if (tid + NT * i < kVec) vec[tid + NT * i] = pv[i];
-  };
   float vr[4], wr[4];
   auto load_v = [&](int n) {
     const int rl = min(kC, d.S - n * kC);
@@ -300,14 +341,12 @@ __global__ __launch_bounds__(256 * C) void f32_scan_kernel(FParams p) {
       wr[r] = live && t < rl ? w : 0.f;
     }
   };
-  fetch(0);
   load_v(0);
-  stage();
   __syncthreads();
   for (int n = 0; n < d.N; ++n) {
     const int nn = min(n + 1, d.N - 1);
     const size_t cid = chunk(n);
-    fetch(nn);
+    const float *la = tA[FOLD ? 0 : n & 1], *lu = FOLD ? tU : la, *vec = vecs[n & 1];
     if constexpr (ST) {
       if (ct < VB)
 #pragma unroll
@@ -320,11 +359,11 @@ __global__ __launch_bounds__(256 * C) void f32_scan_kernel(FParams p) {
 #pragma unroll
     for (int cb = 0; cb < KB; ++cb) {
       const f32x4 s = ld4(&Sx[team][cb * kBlk + 4 * lane]);
-      const f32x4 a = ld4(&tl[o.a + (tb * KB + cb) * kBlk + fo]);
+      const f32x4 a = ld4(&la[(tb * KB + cb) * kBlk + fo]);
       if constexpr (ST) {
         ks = mm(a, s, ks);
       } else {
-        const f32x4 q = ld4(&tl[o.q + (tb * KB + cb) * kBlk + fo]);
+        const f32x4 q = ld4(&tQ[(tb * KB + cb) * kBlk + fo]);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           ks = mfma_f32(a[r], s[r], ks);
@@ -347,7 +386,7 @@ __global__ __launch_bounds__(256 * C) void f32_scan_kernel(FParams p) {
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       if (j <= tb)
-        Vn = mm(ld4(&tl[o.t + tri_blk(tb, j) * kBlk + fo]),
+        Vn = mm(ld4(&tT[tri_blk(tb, j) * kBlk + fo]),
                 ld4(&Xx[team][j * kBlk + 4 * lane]), Vn);
     st4(&Vx[team][tb * kBlk + 4 * lane], Vn);
     if (ST && ct < VB) st4(p.vn + ((cid * 4 + tb) * VB + ct) * kBlk + 4 * lane, Vn);
@@ -370,7 +409,7 @@ __global__ __launch_bounds__(256 * C) void f32_scan_kernel(FParams p) {
     for (int j = 0; j < 4; ++j) {
       const f32x4 vj = ld4(&Vx[team][j * kBlk + 4 * lane]);
       if constexpr (!ST)
-        if (j <= tb) qs = mm(ld4(&tl[o.at + tri_blk(tb, j) * kBlk + fo]), vj, qs);
+        if (j <= tb) qs = mm(ld4(&tAt[tri_blk(tb, j) * kBlk + fo]), vj, qs);
       f32x4 vk = vj;
       if constexpr (!FOLD) {
         const f32x4 gk = ld4(&vec[128 + 16 * j + 4 * g4]);
@@ -380,7 +419,7 @@ __global__ __launch_bounds__(256 * C) void f32_scan_kernel(FParams p) {
 #pragma unroll
       for (int i = 0; i < NR; ++i)
         if (tw + 4 * i < KB) {
-          const float* ub = &tl[o.u + (j * KB + tw + 4 * i) * kBlk];
+          const float* ub = &lu[(j * KB + tw + 4 * i) * kBlk];
 #pragma unroll
           for (int r = 0; r < 4; ++r) S[i] = mfma_f32(ub[to[r]], vk[r], S[i]);
         }
@@ -398,8 +437,6 @@ __global__ __launch_bounds__(256 * C) void f32_scan_kernel(FParams p) {
           st(static_cast<TY*>(p.y), (row0 + size_t(t) * d.H) * d.V + col, qs[r]);
       }
     }
-    lds_barrier();  // every wave is done with this chunk's tiles
-    stage();
     lds_barrier();
   }
 #pragma unroll
@@ -445,7 +482,7 @@ hipError_t f32_scan(const FParams& p, int qkv_dtype, int y_dtype, bool states,
                     hipStream_t stream) {
   const Dims& d = p.d;
   const int teams = scan_teams(d);
-  const dim3 grid(scan_blocks(d, teams)), block(256 * teams);
+  const dim3 grid(scan_blocks(d, teams)), block(256 * teams + 256);
   const bool b16 = qkv_dtype == DN_BF16, y16 = y_dtype == DN_BF16, fold = folds(d);
   ProfScope ps(states ? "dn_f32_scan_states" : "dn_f32_scan", stream);
 #define DN_S(KB, C, F, ST, TV, TY) \

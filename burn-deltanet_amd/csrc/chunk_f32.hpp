@@ -121,6 +121,23 @@ __device__ inline f32x4 load4(const T* p, size_t at, int n, bool vec) {
   return x;
 }
 
+// W floats of a chunk's tiles on their way to LDS, in the registers of the 256
+// staging threads (t of them).
+template <int W>
+struct Piece {
+  static constexpr int kWords = W / 4, N = (kWords + 255) / 256;
+  f32x4 x[N];
+  __device__ void load(const float* src, int t) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) x[i] = ld4(src + 4 * min(t + 256 * i, kWords - 1));
+  }
+  __device__ void store(float* dst, int t) const {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (256 * (i + 1) <= kWords || t + 256 * i < kWords) st4(dst + 4 * (t + 256 * i), x[i]);
+  }
+};
+
 // Key blocks a launch is compiled for: head_k_dim rounded up to 32, 64, 96 or 128.
 inline int key_blocks(int K) { return 2 * ((K + 31) / 32); }
 inline bool folds(const Dims& d) { return d.ew > 1 || d.dw > 1; }

@@ -15,18 +15,18 @@ namespace {
 //   dV' = attnᵀ·dY + kc·dS,  Z = Tᵀ·dV',  dS ← egl⊙dS + qgᵀ·dY − kgᵀ·Z.
 // Leaves dS (leaving each chunk), dV' and Z in the workspace.
 template <int KB, int C, bool FOLD, class TG>
-__global__ __launch_bounds__(256 * C) void f32_rev_scan_kernel(FParams p) {
+__global__ __launch_bounds__(256 * C + 256) void f32_rev_scan_kernel(FParams p) {
   constexpr Lay o = lay(KB, FOLD);
-  constexpr int NT = 256 * C;
-  constexpr int kCopy = o.vec / 4;
-  constexpr int NPF = (kCopy + NT - 1) / NT;
+  constexpr int kTile = 4 * KB * kBlk;
   constexpr int kVec = 4 * kC + 16 * KB;
-  constexpr int NPV = (kVec + NT - 1) / NT;
   constexpr int NR = (KB + 3) / 4;
-  __shared__ __attribute__((aligned(16))) float tl[kCopy * 4];
-  __shared__ __attribute__((aligned(16))) float vec[kVec];
+  constexpr int kU = FOLD ? kTile : 16;
+  __shared__ __attribute__((aligned(16))) float tA[FOLD ? 1 : 2][kTile], tU[kU], tQ[kTile], tT[kTri],
+      tAt[kTri], vecs[2][kVec];
   __shared__ __attribute__((aligned(16))) float Sx[C][KB * kBlk];
-  __shared__ __attribute__((aligned(16))) float Yx[C][4 * kBlk], Vx[C][4 * kBlk], Zx[C][4 * kBlk];
+  // dY and dV' change places from chunk to chunk: dV' is dead when the next
+  // chunk's dY arrives.
+  __shared__ __attribute__((aligned(16))) float YVx[2][C][4 * kBlk], Zx[C][4 * kBlk];
 
   const Dims& d = p.d;
   const int BH = d.B * d.H, VB = (d.V + 15) / 16, ntile = (VB + C - 1) / C;
@@ -42,6 +42,65 @@ __global__ __launch_bounds__(256 * C) void f32_rev_scan_kernel(FParams p) {
   int to[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) to[r] = blk(4 * g4 + r, m16);
+  auto chunk = [&](int n) { return (size_t(b) * d.N + n) * d.H + h; };
+  if (__builtin_amdgcn_readfirstlane(wave) >= 4 * C) {
+    // --- the staging waves (the forward scan's, for this walk's phases) ---
+    const int t = tid - 256 * C;
+    auto src = [&](int n) { return p.ws + chunk(max(n, 0)) * o.per; };
+    const int N1 = d.N - 1;
+    Piece<kTile> a, q;
+    Piece<kU> u;
+    Piece<kTri> T, at;
+    Piece<kVec> v;
+    at.load(src(N1) + o.at, t);
+    T.load(src(N1) + o.t, t);
+    v.load(src(N1) + o.vec, t);
+    a.load(src(N1) + o.a, t);
+    if constexpr (FOLD) u.load(src(N1) + o.u, t);
+    at.store(tAt, t);
+    T.store(tT, t);
+    v.store(vecs[N1 & 1], t);
+    if constexpr (FOLD) {
+      u.store(tU, t);
+    } else {
+      a.store(tA[N1 & 1], t);
+      a.load(src(N1 - 1) + o.a, t);
+    }
+    q.load(src(N1) + o.q, t);
+    v.load(src(N1 - 1) + o.vec, t);
+    at.load(src(N1 - 1) + o.at, t);
+    if constexpr (FOLD) u.load(src(N1 - 1) + o.u, t);
+    T.load(src(N1 - 1) + o.t, t);
+    __syncthreads();
+    for (int n = N1; n >= 0; --n) {
+      // Beside phase 1: phase 3's operands.
+      q.store(tQ, t);
+      q.load(src(n - 1) + o.q, t);
+      if constexpr (FOLD) {
+        a.store(tA[0], t);
+        a.load(src(n - 1) + o.a, t);
+      }
+      v.store(vecs[(n + 1) & 1], t);
+      v.load(src(n - 2) + o.vec, t);
+      lds_barrier();
+      // Beside phase 2: the next chunk's operands of phase 1.
+      at.store(tAt, t);
+      at.load(src(n - 2) + o.at, t);
+      if constexpr (FOLD) {
+        u.store(tU, t);
+        u.load(src(n - 2) + o.u, t);
+      } else {
+        a.store(tA[(n + 1) & 1], t);
+        a.load(src(n - 2) + o.a, t);
+      }
+      lds_barrier();
+      // Beside phase 3: the next chunk's T.
+      T.store(tT, t);
+      T.load(src(n - 2) + o.t, t);
+      lds_barrier();
+    }
+    return;
+  }
   const int ct = tile * C + team, col = 16 * ct + m16;
   const bool live = col < d.V;
   const int cl = min(col, d.V - 1);
@@ -62,15 +121,8 @@ __global__ __launch_bounds__(256 * C) void f32_rev_scan_kernel(FParams p) {
     }
     if (rb < KB) st4(&Sx[team][rb * kBlk + 4 * lane], S[i]);
   }
-  auto chunk = [&](int n) { return (size_t(b) * d.N + n) * d.H + h; };
-  f32x4 pf[NPF], py;
-  float pv[NPV];
+  f32x4 py;
   auto fetch = [&](int n) {
-    const float* src = p.ws + chunk(n) * o.per;
-#pragma unroll
-    for (int i = 0; i < NPF; ++i) pf[i] = ld4(src + 4 * min(tid + NT * i, kCopy - 1));
-#pragma unroll
-    for (int i = 0; i < NPV; ++i) pv[i] = src[o.vec + min(tid + NT * i, kVec - 1)];
     const int rl = min(kC, d.S - n * kC);
     const size_t row0 = (size_t(b) * d.S + size_t(n) * kC) * d.H + h;
 #pragma unroll
@@ -80,20 +132,14 @@ __global__ __launch_bounds__(256 * C) void f32_rev_scan_kernel(FParams p) {
       py[r] = live && t < rl ? x : 0.f;
     }
   };
-  auto stage = [&] {
-#pragma unroll
-    for (int i = 0; i < NPF; ++i)
-      if (NT * (i + 1) <= kCopy || tid + NT * i < kCopy) st4(&tl[4 * (tid + NT * i)], pf[i]);
-#pragma unroll
-    for (int i = 0; i < NPV; ++i)
-      if (tid + NT * i < kVec) vec[tid + NT * i] = pv[i];
-    st4(&Yx[team][tb * kBlk + 4 * lane], py);
-  };
   fetch(d.N - 1);
-  stage();
+  st4(&YVx[(d.N - 1) & 1][team][tb * kBlk + 4 * lane], py);
   __syncthreads();
   for (int n = d.N - 1; n >= 0; --n) {
     const size_t cid = chunk(n);
+    const float *la = tA[FOLD ? 0 : n & 1], *lu = FOLD ? tU : la, *vec = vecs[n & 1];
+    const float* Yx = YVx[n & 1][team];
+    float* Vx = YVx[(n + 1) & 1][team];
     fetch(max(n - 1, 0));
     if (ct < VB)
 #pragma unroll
@@ -103,27 +149,27 @@ __global__ __launch_bounds__(256 * C) void f32_rev_scan_kernel(FParams p) {
     f32x4 dv = zero4(), av = zero4();
 #pragma unroll
     for (int cb = 0; cb < KB; ++cb)
-      dv = mm(ld4(&tl[o.u + (tb * KB + cb) * kBlk + fo]), ld4(&Sx[team][cb * kBlk + 4 * lane]),
+      dv = mm(ld4(&lu[(tb * KB + cb) * kBlk + fo]), ld4(&Sx[team][cb * kBlk + 4 * lane]),
               dv);
     // A transposed block's operand: its four words in column order.
     auto tr = [&](const float* x) { return f32x4{x[to[0]], x[to[1]], x[to[2]], x[to[3]]}; };
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       if (j >= tb)
-        av = mm(tr(&tl[o.at + tri_blk(j, tb) * kBlk]), ld4(&Yx[team][j * kBlk + 4 * lane]), av);
+        av = mm(tr(&tAt[tri_blk(j, tb) * kBlk]), ld4(&Yx[j * kBlk + 4 * lane]), av);
     {
       const f32x4 gk = ld4(&vec[128 + 16 * tb + 4 * g4]);
 #pragma unroll
       for (int r = 0; r < 4; ++r) dv[r] = av[r] + (FOLD ? dv[r] : gk[r] * dv[r]);
     }
-    st4(&Vx[team][tb * kBlk + 4 * lane], dv);
+    st4(&Vx[tb * kBlk + 4 * lane], dv);
     if (ct < VB) st4(p.dvn + ((cid * 4 + tb) * VB + ct) * kBlk + 4 * lane, dv);
     lds_barrier();
     f32x4 z = zero4();
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       if (j >= tb)
-        z = mm(tr(&tl[o.t + tri_blk(j, tb) * kBlk]), ld4(&Vx[team][j * kBlk + 4 * lane]), z);
+        z = mm(tr(&tT[tri_blk(j, tb) * kBlk]), ld4(&Vx[j * kBlk + 4 * lane]), z);
     st4(&Zx[team][tb * kBlk + 4 * lane], z);
     if (ct < VB) st4(p.z + ((cid * 4 + tb) * VB + ct) * kBlk + 4 * lane, z);
     lds_barrier();
@@ -136,7 +182,7 @@ __global__ __launch_bounds__(256 * C) void f32_rev_scan_kernel(FParams p) {
       }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      f32x4 y = ld4(&Yx[team][j * kBlk + 4 * lane]), zj = ld4(&Zx[team][j * kBlk + 4 * lane]);
+      f32x4 y = ld4(&Yx[j * kBlk + 4 * lane]), zj = ld4(&Zx[team][j * kBlk + 4 * lane]);
       const f32x4 xe = ld4(&vec[16 * j + 4 * g4]), ys = ld4(&vec[64 + 16 * j + 4 * g4]);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -147,15 +193,14 @@ __global__ __launch_bounds__(256 * C) void f32_rev_scan_kernel(FParams p) {
       for (int i = 0; i < NR; ++i)
         if (tw + 4 * i < KB) {
           const int at = (j * KB + tw + 4 * i) * kBlk;
-          S[i] = mm(tr(&tl[o.q + at]), y, S[i]);
-          S[i] = mm(tr(&tl[o.a + at]), zj, S[i]);
+          S[i] = mm(tr(&tQ[at]), y, S[i]);
+          S[i] = mm(tr(&la[at]), zj, S[i]);
         }
     }
 #pragma unroll
     for (int i = 0; i < NR; ++i)
       if (tw + 4 * i < KB) st4(&Sx[team][(tw + 4 * i) * kBlk + 4 * lane], S[i]);
-    lds_barrier();
-    stage();
+    st4(&Vx[tb * kBlk + 4 * lane], py);  // the next chunk's dY
     lds_barrier();
   }
 #pragma unroll
@@ -331,7 +376,7 @@ __global__ __launch_bounds__(64 * (KB < 4 ? 4 : KB)) void f32_chunk_bwd_kernel(F
 hipError_t launch_rev(const FParams& p, int grad_dtype, hipStream_t stream) {
   const Dims& d = p.d;
   const int teams = scan_teams(d);
-  const dim3 grid(scan_blocks(d, teams)), block(256 * teams);
+  const dim3 grid(scan_blocks(d, teams)), block(256 * teams + 256);
   const bool g16 = grad_dtype == DN_BF16, fold = folds(d);
   ProfScope ps("dn_f32_rev_scan", stream);
 #define DN_R(KB, C, F)                                                                       \
