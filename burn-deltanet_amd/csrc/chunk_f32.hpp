@@ -17,8 +17,8 @@
 // kernels that ran these calls before, whose scores and inverse were scalar
 // loops over HBM: intra 769 -> 25 us, scan 605 -> 75, states scan 404 -> 63
 // beside the reverse scan 661 -> 124, chunk_bwd 1601 -> 90; forward and
-// backward through autograd 4812 -> 353 us. B=1 S=512 H=4 K=V=64: forward
-// 592 -> 34 us.
+// backward through autograd 4812 -> 324 us. B=1 S=512 H=4 K=V=64: forward
+// 592 -> 31 us.
 //
 // Tiles. Every operand is kept as 16×16 blocks of 256 floats. Element (i, j)
 // of a block sits at blk(i, j): float4s along j in the order of the MFMA
