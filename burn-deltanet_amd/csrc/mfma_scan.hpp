@@ -145,7 +145,7 @@ __global__ __launch_bounds__(64 * WAVES) void mfma_scan_kernel(MfmaParams p) {
   // one is consumed, so one barrier per chunk suffices. The per-channel
   // tiles with y, and head_k_dim 256's (88 KB a chunk), do not fit twice in
   // LDS: they are staged between two barriers. (Without y the per-channel
-  // tiles take 64 KB; double-buffered, config 5's two-wave states scan ran
+  // tiles take 64 KB; double-buffered, the two-wave states scan of 32 heads ran
   // slower, 861 → 1057 µs.) (A head_k_dim 256 variant that
   // kept the K and [64][64] tiles double-buffered and restaged a single Q
   // tile after a barrier behind phase 1 measured slower, 487 → 652 µs at
@@ -602,16 +602,16 @@ __global__ __launch_bounds__(64 * WAVES) void mfma_scan_kernel(MfmaParams p) {
     const uint16_t* tl = tiles[cur];
     const float egl = PC ? 1.f : gegl[cur];
     // The next chunk's tiles are fetched at the top, so the loads have all
-    // three phases to land before stage() writes them to LDS (config 2 scan
-    // 392 → 376 µs, config 5's per-channel scan 1165 → 870 µs). The
+    // three phases to land before stage() writes them to LDS (128 heads, dv 256:
+    // 392 → 376 µs, 32 heads' per-channel scan 1165 → 870 µs). The
     // per-channel states mode (the backward's recompute) measured slower so
     // (1055 → 1105 µs): its fetch stays after phase 1.
     constexpr bool kFetchTop = !(PC && ST);
     // Eight-wave double-buffered scans: the next chunk's tiles in two
     // halves, the first staged after phase 1 (the other buffer is free all
-    // chunk), which halves the registers holding them (config 2 scan 339 →
+    // chunk), which halves the registers holding them (128 heads' scan 339 →
     // 312 µs). The two-wave scan (36 rounds per lane) and the states mode
-    // measured slower so (config 4 1.09 → 1.24 ms).
+    // measured slower so (64 heads of 256 chunks, 1.09 → 1.24 ms).
     constexpr bool kHalf = NBUF == 2 && WAVES == 8 && !ST;
     constexpr int NH = kHalf ? (NPF + 1) / 2 : NPF;
     if constexpr (kFetchTop) fetch(nn, 0, NH);
@@ -640,10 +640,10 @@ __global__ __launch_bounds__(64 * WAVES) void mfma_scan_kernel(MfmaParams p) {
     // Two-wave per-head scans (one wave per SIMD) interleave VALU work with
     // independent MFMAs by hand: in phase 1 the next k-step's S fragments
     // are split while this one's MFMAs run, one MFMA to two VALU
-    // instructions (config 4 1.09 → 1.05 ms). With two waves per SIMD the
+    // instructions (64 heads, 1.09 → 1.05 ms). With two waves per SIMD the
     // other wave covers the split, and so interleaved the eight-wave scan
     // measured slower (315 → 345 µs), as did the per-channel states mode;
-    // S's gate products placed under phase 3's attn MFMAs likewise (config 4
+    // S's gate products placed under phase 3's attn MFMAs likewise (64 heads
     // 1.05 → 1.20 ms), and X's second k-step split under phase 2's first
     // nine MFMAs (1.05 → 1.14 ms).
     constexpr bool kPipe = WAVES == 2 && !PC && !ST;

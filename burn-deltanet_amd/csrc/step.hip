@@ -209,7 +209,7 @@ __global__ __launch_bounds__(kRowThreads) void step_row_kernel(StepParams p) {
 
   // The state streams through once per step: non-temporal loads and stores
   // keep it from displacing anything in L2 / Infinity Cache. (Issuing these
-  // loads before the gate set-up above measured slower on config 3.)
+  // loads before the gate set-up above measured slower with 4096 heads.)
   const bool colok = j0 + C - 1 < V;
   const float* sin = p.s_in + bh * size_t(K) * V + j0;
   vec s[RPT];
