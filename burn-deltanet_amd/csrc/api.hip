@@ -391,8 +391,9 @@ int dn_chunk_fwd(const dn_chunk_fwd_args* a, hipStream_t stream) {
   d = run_dims(d, algo);
   const size_t need = fwd_workspace(d, algo);
   void* ws = a->workspace;
+  const size_t ws_bytes = ws ? a->workspace_bytes : need;
   if (ws) {
-    if (a->workspace_bytes < need)
+    if (ws_bytes < need)
       return fail(DN_ERR_WORKSPACE, "workspace too small: need " + std::to_string(need) +
                                         " bytes");
   } else if (need) {
@@ -413,8 +414,8 @@ int dn_chunk_fwd(const dn_chunk_fwd_args* a, hipStream_t stream) {
   hipError_t e;
   if (algo != DN_ALGO_GENERIC)
     e = mfma_fwd(d, a->y_dtype, a->q, a->k, a->v, a->erase, a->write,
-                 a->has_gate ? a->g : nullptr, a->state_in, a->y, a->state_out, ws, stream,
-                 algo == DN_ALGO_MFMA_FUSED);
+                 a->has_gate ? a->g : nullptr, a->state_in, a->y, a->state_out, ws, ws_bytes,
+                 stream, algo == DN_ALGO_MFMA_FUSED);
   else
     e = generic_fwd(d, a->qkv_dtype, a->y_dtype, a->q, a->k, a->v, a->erase, a->write,
                     a->has_gate ? a->g : nullptr, a->state_in, a->y, a->state_out, ws, stream);
@@ -454,8 +455,8 @@ int dn_chunk_fwd_noalloc(const dn_chunk_fwd_args* a, hipStream_t stream) {
   // same call (no counters or partial sums), so nothing is cleared first.
   if (algo != DN_ALGO_GENERIC)
     e = mfma_fwd(d, a->y_dtype, a->q, a->k, a->v, a->erase, a->write,
-                 a->has_gate ? a->g : nullptr, a->state_in, a->y, a->state_out, ws, stream,
-                 algo == DN_ALGO_MFMA_FUSED);
+                 a->has_gate ? a->g : nullptr, a->state_in, a->y, a->state_out, ws,
+                 DN_NOALLOC_SCRATCH_BYTES, stream, algo == DN_ALGO_MFMA_FUSED);
   else
     e = generic_fwd(d, a->qkv_dtype, a->y_dtype, a->q, a->k, a->v, a->erase, a->write,
                     a->has_gate ? a->g : nullptr, a->state_in, a->y, a->state_out, ws, stream);
@@ -523,8 +524,9 @@ int dn_chunk_fwd_out_norm(const dn_chunk_fwd_out_norm_args* a, hipStream_t strea
   const bool in_scan = a->in_scan && algo == DN_ALGO_MFMA && norm_fusable(a);
   const size_t need = in_scan ? mfma_fwd_norm_workspace(d) : fwd_workspace(d, algo);
   void* ws = f->workspace;
+  const size_t ws_bytes = ws ? f->workspace_bytes : need;
   if (ws) {
-    if (f->workspace_bytes < need)
+    if (ws_bytes < need)
       return fail(DN_ERR_WORKSPACE, "workspace too small: need " + std::to_string(need) +
                                         " bytes");
   } else if (need) {
@@ -556,7 +558,7 @@ int dn_chunk_fwd_out_norm(const dn_chunk_fwd_out_norm_args* a, hipStream_t strea
     // The forward, then the norm in place on y.
     if (algo != DN_ALGO_GENERIC)
       e = mfma_fwd(d, f->y_dtype, f->q, f->k, f->v, f->erase, f->write, g, f->state_in, f->y,
-                   f->state_out, ws, stream, algo == DN_ALGO_MFMA_FUSED);
+                   f->state_out, ws, ws_bytes, stream, algo == DN_ALGO_MFMA_FUSED);
     else
       e = generic_fwd(d, f->qkv_dtype, f->y_dtype, f->q, f->k, f->v, f->erase, f->write, g,
                       f->state_in, f->y, f->state_out, ws, stream);
@@ -842,8 +844,9 @@ int dn_frontend_chunk_fwd(const dn_frontend_chunk_fwd_args* a, hipStream_t strea
   d = run_dims(d, algo);
   const size_t need = fwd_workspace(d, algo);
   void* ws = f->workspace;
+  const size_t ws_bytes = ws ? f->workspace_bytes : need;
   if (ws) {
-    if (f->workspace_bytes < need)
+    if (ws_bytes < need)
       return fail(DN_ERR_WORKSPACE, "workspace too small: need " + std::to_string(need) +
                                         " bytes");
   } else if (need) {
@@ -865,8 +868,8 @@ int dn_frontend_chunk_fwd(const dn_frontend_chunk_fwd_args* a, hipStream_t strea
   fp.q = static_cast<uint16_t*>(fe.q);
   fp.k = static_cast<uint16_t*>(fe.k);
   e = mfma_fwd(d, f->y_dtype, f->q, f->k, f->v, f->erase, f->write,
-               f->has_gate ? f->g : nullptr, f->state_in, f->y, f->state_out, ws, stream, false,
-               &fp);
+               f->has_gate ? f->g : nullptr, f->state_in, f->y, f->state_out, ws, ws_bytes, stream,
+               false, &fp);
   if (e != hipSuccess) return hip_fail(e, "dn_frontend_chunk_fwd launch");
   e = launch_frontend(fe, stream, kFrontWindow);
   if (e != hipSuccess) return hip_fail(e, "dn_frontend_chunk_fwd window launch");

@@ -1483,8 +1483,9 @@ int norm_scan_waves(const Dims& d) {
 // less than one scan by a twelfth: a pass is its chunks and about 4 us, the
 // carry 3 us a segment (1.3 at head_k_dim 64), two more launches 5. Sequences
 // of 32 whole chunks or more, in segments of 8 or more; the last may be shorter. The
-// segments' buffers must not take a call past the fixed scratch of
-// dn_chunk_fwd_noalloc that its tiles fit. Calls, us, whole and segmented:
+// segments' buffers must fit `room` bytes of workspace behind the tiles, and
+// must not take a call past the fixed scratch of dn_chunk_fwd_noalloc that its
+// tiles fit. Calls, us, whole and segmented:
 // S=8192 dk=dv=128, 1 head, per channel 190 and 90; 4 heads, per-head gates,
 // dv 256: S=16384 323 and 197, S=8192 166 and 122; dk 64, 2 heads: S=16384 258
 // and 75. 32 heads at S=16384 per channel, 596 us of scans in segments of
@@ -1513,15 +1514,15 @@ size_t seg_bytes(const Dims& d, int P) {
   const size_t bh = size_t(d.B) * P * d.H, K = size_t(d.K);
   return P == 1 ? 0 : region(bh * K * K * 4) + 2 * region(bh * K * d.V * 4);
 }
-int seg_parts(const Dims& d) {
+int seg_parts(const Dims& d, size_t room) {
   if (d.K > 128 || d.N < 32 || size_t(d.S) != size_t(d.N) * d.L) return 1;
   const ScanShape w = scan_shape(d, false);
   float least = chunk_us(d, w) * float(d.N) *
                     float(scan_rounds(d, w.teams ? 16 * w.teams : 16 * w.waves, 1)) + 4.f;
   int best = 1;
   for (int P = 2; d.N >= 8 * P && P <= 64; P *= 2) {
-    const size_t tiles = tiles_workspace(d);
-    if (tiles <= DN_NOALLOC_SCRATCH_BYTES && tiles + seg_bytes(d, P) > DN_NOALLOC_SCRATCH_BYTES)
+    const size_t tiles = tiles_workspace(d), bytes = tiles + seg_bytes(d, P);
+    if (bytes > room || (tiles <= DN_NOALLOC_SCRATCH_BYTES && bytes > DN_NOALLOC_SCRATCH_BYTES))
       break;
     const float n = float((d.N + P - 1) / P);
     const float cut = n * (teams_us(d, d.V + d.K, P) + teams_us(d, d.V, P)) +
@@ -1741,19 +1742,19 @@ bool mfma_bwd_supported(const Dims& d, int qkv_dtype) {
 }
 
 size_t mfma_fwd_workspace(const Dims& d, bool fused) {
-  return fused ? fused_fwd_workspace(d) : tiles_workspace(d) + seg_bytes(d, seg_parts(d));
+  return fused ? fused_fwd_workspace(d) : tiles_workspace(d) + seg_bytes(d, seg_parts(d, SIZE_MAX));
 }
 
 hipError_t mfma_fwd(const Dims& d, int y_dtype, const void* q, const void* k, const void* v,
                     const float* erase, const float* write, const float* g,
-                    const float* state_in, void* y, float* state_out, void* ws,
+                    const float* state_in, void* y, float* state_out, void* ws, size_t ws_bytes,
                     hipStream_t stream, bool fused, const FeParams* fe) {
   if (fused)
     return fused_fwd(d, y_dtype, q, k, v, erase, write, g, state_in, y, state_out, ws, stream);
   MfmaParams p = make_params(d, q, k, v, erase, write, g, state_in, y, state_out, ws);
   hipError_t e = launch_intra(p, d, stream, nullptr, fe);
   if (e != hipSuccess) return e;
-  const int P = seg_parts(d);
+  const int P = seg_parts(d, ws_bytes);
   const bool yb = y_dtype == DN_BF16, pc = pc_path(d);
   if (P == 1) return launch_scan<false>(p, d, yb, stream);
   // Segmented: the segments' transitions, the carry, then the outputs.

@@ -131,7 +131,10 @@ bool mfma_fwd_supported(const Dims& d, int qkv_dtype, int y_dtype);
 bool mfma_bwd_supported(const Dims& d, int qkv_dtype);
 // The MFMA forward: the intra kernel and the scan as two launches with their
 // tiles in the workspace, or with `fused` (where fused_fwd_supported holds)
-// the one kernel of chunk_fwd_fused.hip.
+// the one kernel of chunk_fwd_fused.hip. mfma_fwd plans by the `ws_bytes` it
+// is given, which need not be what mfma_fwd_workspace says for its arguments
+// (a caller may hold another entry point's workspace): it cuts the sequences
+// into no more segments than fit there.
 size_t mfma_fwd_workspace(const Dims& d, bool fused = false);
 // The projection front-end's q/k formed in the intra kernel's load stage
 // (dn_frontend_chunk_fwd): the raw projection columns, the conv of length 4
@@ -150,7 +153,7 @@ struct FeParams {
 };
 hipError_t mfma_fwd(const Dims& d, int y_dtype, const void* q, const void* k, const void* v,
                     const float* erase, const float* write, const float* g,
-                    const float* state_in, void* y, float* state_out, void* ws,
+                    const float* state_in, void* y, float* state_out, void* ws, size_t ws_bytes,
                     hipStream_t stream, bool fused = false, const FeParams* fe = nullptr);
 // The MFMA forward with the output norm applied in the scan's y write
 // (OutNorm::forward, norm.rs:106-144): y receives the normalised output.

@@ -1,0 +1,165 @@
+// What the library's host code launches and where it points the kernels, on
+// the CPU: this program stands in for the HIP runtime (its definitions come
+// before libamdhip64's), records every launch with a copy of the kernel's
+// parameters and runs none of them. Device pointers are addresses nobody reads.
+//
+// Prints "ok <case>" per case; exits nonzero at the first failure.
+
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <string>
+#include <vector>
+
+#include "dn_common.hpp"
+#include "mfma_scan.hpp"
+
+namespace {
+
+struct Launch {
+  std::string kernel;
+  const void* params;  // valid until the next launch
+};
+
+std::map<const void*, std::string>& kernels() {
+  static auto* m = new std::map<const void*, std::string>();  // filled before main
+  return *m;
+}
+
+int device = 0;  // current device: how many CUs it has
+const int kCus[] = {256, 128, 64, 32};
+int blocks_per_cu = 0;  // what the occupancy query answers
+void (*on_launch)(const Launch&) = nullptr;
+
+void fail(const std::string& what) {
+  std::fprintf(stderr, "FAIL %s\n", what.c_str());
+  std::exit(1);
+}
+
+hipError_t record(const void* f, void** args) {
+  const auto it = kernels().find(f);
+  if (it == kernels().end()) fail("launch of an unregistered kernel");
+  if (on_launch) on_launch({it->second, args[0]});
+  return hipSuccess;
+}
+
+}  // namespace
+
+extern "C" {
+void** __hipRegisterFatBinary(const void*) {
+  static void* handle = nullptr;
+  return &handle;
+}
+void __hipUnregisterFatBinary(void**) {}
+void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, uint3*,
+                           uint3*, dim3*, dim3*, int*) {
+  kernels()[host] = name;
+}
+void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
+hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3*, dim3*, size_t*, hipStream_t*) { return hipSuccess; }
+hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t) {
+  return record(f, args);
+}
+hipError_t hipLaunchCooperativeKernel(const void* f, dim3, dim3, void** args, unsigned,
+                                      hipStream_t) {
+  return record(f, args);
+}
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetDevice(int* d) {
+  *d = device;
+  return hipSuccess;
+}
+hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int d) {
+  *v = kCus[d];
+  return hipSuccess;
+}
+hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int, size_t) {
+  *n = blocks_per_cu;
+  return hipSuccess;
+}
+hipError_t hipMalloc(void** p, size_t) {
+  *p = reinterpret_cast<void*>(uintptr_t(1) << 20);
+  return hipSuccess;
+}
+hipError_t hipMemset(void*, int, size_t) { return hipSuccess; }
+}
+
+namespace {
+
+char* const kWorkspace = reinterpret_cast<char*>(uintptr_t(1) << 44);
+const void* const kTensor = reinterpret_cast<const void*>(uintptr_t(1) << 30);
+
+dn_chunk_fwd_args forward(int B, int S, int H, int K, int V, bool channel) {
+  dn_chunk_fwd_args a{};
+  a.batch = B, a.sequence = S, a.nheads = H, a.head_k_dim = K, a.head_v_dim = V;
+  a.erase_width = channel ? K : 1, a.write_width = channel ? V : 1;
+  a.decay_width = channel ? K : 1;
+  a.has_gate = 1, a.chunk_len = 64, a.scale = std::nan("");
+  a.qkv_dtype = a.y_dtype = DN_BF16;
+  a.q = a.k = a.v = kTensor;
+  a.erase = a.write = a.g = a.state_in = static_cast<const float*>(kTensor);
+  a.y = const_cast<void*>(kTensor);
+  a.state_out = static_cast<float*>(const_cast<void*>(kTensor));
+  a.workspace = kWorkspace;
+  return a;
+}
+
+// The end of the segmented scan's buffers, as its carry kernel is given them.
+struct Segments {
+  int parts = 0;
+  const char* end = nullptr;
+} segments;
+
+void see_segments(const Launch& l) {
+  if (l.kernel.find("seg_carry_kernel") == std::string::npos) return;
+  const auto& p = *static_cast<const dn::MfmaParams*>(l.params);
+  const int K = l.kernel.find("Li128E") != std::string::npos ? 128 : 64;
+  segments.parts = p.seg_p;
+  segments.end = reinterpret_cast<const char*>(p.seg_start + size_t(p.B) * p.seg_p * p.H * K * p.V);
+}
+
+// dn_chunk_fwd_out_norm with the norm in the scan, on devices where its
+// cooperative launch never fits: the plain forward runs in its workspace.
+void out_norm_fallback() {
+  on_launch = see_segments;
+  blocks_per_cu = 0;
+  int cut = 0;
+  for (device = 0; device < 4; ++device)
+    for (int K : {64, 128})
+      for (int V = 64; V <= 1024; V += 64)
+        for (int chunks : {32, 64, 100, 256})
+          for (int heads : {1, 2, 3, 5})
+            for (bool channel : {false, true}) {
+              dn_chunk_fwd_out_norm_args a{};
+              a.fwd = forward(1, 64 * chunks, heads, K, V, channel);
+              a.weight = static_cast<const float*>(kTensor);
+              a.eps = 1e-5;
+              a.in_scan = 1;
+              a.fwd.workspace_bytes = dn_chunk_fwd_out_norm_workspace_bytes(&a);
+              segments = {};
+              if (dn_chunk_fwd_out_norm(&a, nullptr) != DN_OK) fail(dn_last_error());
+              cut += segments.parts > 1;
+              if (segments.end > kWorkspace + a.fwd.workspace_bytes)
+                fail("out norm fallback: " + std::to_string(segments.parts) + " segments of K " +
+                     std::to_string(K) + " V " + std::to_string(V) + " chunks " +
+                     std::to_string(chunks) + " heads " + std::to_string(heads) + " end " +
+                     std::to_string(segments.end - kWorkspace - a.fwd.workspace_bytes) +
+                     " bytes past the workspace");
+            }
+  device = 0;
+  if (!cut) fail("out norm fallback: no call was segmented");
+  std::printf("ok out_norm_fallback (%d segmented calls)\n", cut);
+}
+
+}  // namespace
+
+int main() {
+  out_norm_fallback();
+  std::printf("all passed\n");
+  return 0;
+}
