@@ -35,7 +35,7 @@ namespace dn {
 namespace {
 
 // Accesses to the caller's gates and gradients, which are aligned to their
-// elements and no further (q, k, v and dO are to 16 bytes).
+// elements and no further, and to v, which is to 4 bytes (q, k and dO are to 16).
 typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u2_any __attribute__((ext_vector_type(2), aligned(2)));
 typedef uint32_t u4_any __attribute__((ext_vector_type(4), aligned(2)));
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(4 * K) void local_bwd_kernel(LocalParams p) {
   f32x4 ps[2], pd[2];
   uint4 py;
   f32x4 pyf[kYlo ? 2 : 1];
-  uint2 pv[TPW];
+  u2_any pv[TPW];
   f32x4 pw[PCG ? TPW : 1];
   auto load = [&](int v0) {
 #pragma unroll
@@ -145,7 +145,7 @@ __global__ __launch_bounds__(4 * K) void local_bwd_kernel(LocalParams p) {
 #pragma unroll
     for (int u = 0; u < TPW; ++u) {
       const int v = v0 + 16 * ((wave + NW * u) >> 2) + 4 * g4;
-      pv[u] = *reinterpret_cast<const uint2*>(p.v + trow * V + v);
+      pv[u] = *reinterpret_cast<const u2_any*>(p.v + trow * V + v);
       if constexpr (PCG)
         if (d.ww != 1) pw[u] = *reinterpret_cast<const f4_any*>(p.write + trow * V + v);
     }
@@ -301,7 +301,7 @@ __global__ __launch_bounds__(4 * K) void local_bwd_kernel(LocalParams p) {
     f32x4 w4[TPW];
 #pragma unroll
     for (int u = 0; u < TPW; ++u) {
-      v4[u] = pv[u];
+      v4[u] = make_uint2(pv[u].x, pv[u].y);
       w4[u] = f32x4{wt1, wt1, wt1, wt1};
       if constexpr (PCG)
         if (d.ww != 1) w4[u] = tok_ok ? pw[u] : zero4();

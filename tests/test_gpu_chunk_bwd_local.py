@@ -47,3 +47,22 @@ def test_chunk_bwd_local(rng, S, K, V, widths, dtype):
         if want is not None:
             scale = max(np.abs(np_of(want)).max(), least if i == 5 else 0.0)
             assert np.abs(np_of(got) - np_of(want)).max() / scale < 2e-2, i
+
+
+@pytest.mark.parametrize("K,V,gates", [(128, 192, "head"), (64, 192, "none"), (64, 64, "channel"),
+                                       (128, 64, "channel")])
+def test_v_four_bytes_past_a_boundary(rng, K, V, gates):
+    """v is owed 4 bytes of alignment: a view that starts there takes the same
+    kernels to the same bits."""
+    announce(f"v at a four-byte offset K {K} V {V} {gates}")
+    raw = random_raw(rng, 1, 70, 2, K, V, gated=gates != "none", channel=gates == "channel")
+    args = to_gpu(raw, torch.bfloat16)
+    dy = torch.tensor(rng.standard_normal(raw[2].shape), device=args[0].device).bfloat16()
+    flat = torch.empty(args[2].numel() + 2, dtype=torch.bfloat16, device=args[0].device)
+    flat[2:] = args[2].flatten()
+    off = list(args)
+    off[2] = flat[2:].view(args[2].shape)
+    assert off[2].data_ptr() % 8 == 4
+    for a, b in zip(*[vars(pkg.combined_backward(dy, None, *x, 64, 1.0 / np.sqrt(K), algo=MFMA)).values()
+                      for x in (args, off)]):
+        assert (a is None and b is None) or torch.equal(a, b)
