@@ -1,8 +1,8 @@
 // The chunkwise WY forward and its backward in fp32 arithmetic, for any
 // shape, gate width and chunk length: what the fp32 matrix-core kernels
-// (chunk_f32.hpp) do not take, that is head_k_dim above 128, a per-channel
-// forget gate at a chunk length other than 64, and calls so small that
-// 64-token chunks would need more workspace than their own.
+// (chunk_f32.hpp) do not take: head_k_dim above 128, chunks of fewer than 64
+// tokens, a per-channel forget gate at any length but 64, and calls so small
+// that 64-token chunks would need more workspace than longer ones.
 //
 // Same three stages as the reference (src/delta/chunk_recalculated/forward.rs):
 //   intra   one workgroup per chunk-head (b, n, h), fully parallel:
@@ -875,15 +875,19 @@ static size_t own_bwd_workspace(const Dims& d) {
 }
 
 // Whether the matrix-core kernels run a call, and the dims they run it with:
-// 64-token chunks, which without a per-channel forget gate order the
-// roundings and nothing else (with one, the block decay's clamp depends on
-// where chunks start, so another length keeps its kernels). They take every
-// such call whose workspace they do not enlarge, so that a caller's fixed
-// scratch holds what it held; short chunks of small heads are the exception
-// (S = 64 in chunks of 16 with K = V = 4: 38 KB a head against 23).
+// 64-token chunks. A request for longer ones runs at 64 where the gates are
+// per head (per channel, the block decay's clamp depends on where chunks
+// start). A request for shorter ones keeps its length and these kernels: the
+// cumulative gate and the inverse round by the length of their sums, so short
+// chunks are what a caller picks for accuracy (y against float64, 256 tokens,
+// K = 64, chunks of 16 and of 64: no gate 2.0e-7 and 2.6e-7, log gates of -1
+// to -5 a token 1.6e-7 and 5.3e-7, one token in ten at -200 9e-6 and 3.6e-5,
+// in a model of the two sums). They take only calls whose workspace they do
+// not enlarge, so that a caller's fixed scratch holds what it held (one chunk
+// of 65 tokens at K = V = 4: 62720 bytes, as two of 64 76032).
 static Dims f32_dims(const Dims& d) {
   Dims f = d;
-  if (d.dw <= 1 || d.K == 1) {
+  if (d.L > 64 && (d.dw <= 1 || d.K == 1)) {
     f.L = 64;
     f.N = (d.S + 63) / 64;
   }

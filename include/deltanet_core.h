@@ -69,7 +69,9 @@ typedef enum {
 typedef enum {
   DN_ALGO_AUTO = 0,
   DN_ALGO_GENERIC = 1, /* fp32 arithmetic, any shape (fp32 matrix cores up to
-                          head_k_dim 128) */
+                          head_k_dim 128 where chunk_len is 64, or longer and run
+                          at 64 without a per-channel forget gate; a shorter
+                          chunk_len keeps its length and its accuracy) */
   DN_ALGO_MFMA = 2,    /* bf16 MFMA tiles; DN_ERR_UNSUPPORTED if the shape does not fit.
                           The forward runs two kernels (intra-chunk tiles through the
                           workspace, then the scan). */

@@ -41,20 +41,20 @@ CASES = [
     (1, 128, 2, 128, 40, 64, (1, 1, 1)),
     (1, 96, 2, 128, 130, 64, (128, 130, 128)),
     (3, 70, 1, 96, 33, 100, (1, 33, 1)),
-    (1, 200, 2, 66, 32, 32, (66, 1, None)),
+    (1, 200, 2, 66, 32, 64, (66, 1, None)),
     # 288 column tiles: more than the device's CUs, so two-team workgroups
     (9, 66, 16, 64, 24, 64, (1, 1, 1)),
     (9, 66, 16, 128, 24, 64, (128, 24, 128)),
 ]
 
 
-def profiled(f):
+def profiled(f, kernels="dn_f32"):
     pkg.abi.profile_enable(True)
     out = f()
     torch.cuda.synchronize()
     names = pkg.abi.profile_read()
     pkg.abi.profile_enable(False)
-    assert names and all(n.startswith("dn_f32") for n in names), names
+    assert names and all(n.startswith(kernels) for n in names), names
     return out
 
 
@@ -89,12 +89,36 @@ def test_f32_forward_and_backward_match_oracle(rng, case, dtype):
 
 
 def test_f32_kernels_do_not_enlarge_a_workspace(rng):
-    """Short chunks of small heads keep kernels of their own: 64-token tiles
-    would need more scratch than a caller held for them."""
-    args = to_gpu(inputs(rng, 1, 64, 1, 4, 4, 1, 1, 1))
-    pkg.abi.profile_enable(True)
-    pkg.delta_chunk_recalculated(*args, True, 16, 0.5, algo=GENERIC)
-    torch.cuda.synchronize()
-    names = pkg.abi.profile_read()
-    pkg.abi.profile_enable(False)
-    assert all(n.startswith("dn_generic") for n in names), names
+    """One chunk of 65 tokens of a small head: two 64-token chunks' tiles would
+    need more scratch than a caller held for it, so it keeps its kernels."""
+    args = to_gpu(inputs(rng, 1, 65, 1, 4, 4, 1, 1, 1))
+    y, s = torch.empty_like(args[2]), torch.empty_like(args[6])
+    held = [pkg.abi.lib().dn_chunk_fwd_workspace_bytes(
+        pkg.abi.chunk_fwd_args(*args, y, s, L, 0.5, algo=GENERIC)) for L in (65, 64)]
+    assert 0 < held[0] < held[1]
+    for L, kernels in ((65, "dn_generic"), (64, "dn_f32")):
+        profiled(lambda: pkg.delta_chunk_recalculated(*args, True, L, 0.5, algo=GENERIC), kernels)
+
+
+@pytest.mark.parametrize("K", [32, 128])
+@pytest.mark.parametrize("L", [16, 32])
+def test_short_chunks_are_as_accurate_as_their_length(rng, L, K):
+    """The state is cleared by a log gate of -3e4 at the last token of every
+    second short chunk, which leaves no sum that the gate enters beside others;
+    carried on in a longer chunk, a cumulative gate of -3e4 (2^-9 its last bit)
+    would cost the tokens after it three digits."""
+    B, S, H, V = 1, 200, 2, 24
+    announce(f"short chunks L {L} K {K}")
+    args = inputs(rng, B, S, H, K, V, 1, 1, 1)
+    args[5][:, L - 1::2 * L] = -3e4
+    g_args = to_gpu(args)
+    ref = as_oracle_inputs(g_args)
+    y, s = pkg.delta_chunk_recalculated(*g_args, True, L, 0.5, algo=GENERIC)
+    want = O.chunk_fwd(*ref, chunk_len=L, scale=0.5)
+    assert rel_err(np_of(y), want[0]) < bar(K) and rel_err(np_of(s), want[1]) < bar(K)
+    dy = torch.tensor(rng.standard_normal((B, S, H, V)), dtype=torch.float32, device=DEV)
+    got = pkg.combined_backward(dy, None, *g_args, L, 0.5, algo=GENERIC)
+    want = O.chunk_bwd(np_of(dy), np.zeros(want[1].shape), *ref, chunk_len=L, scale=0.5)
+    for i, name in enumerate(("d_q_bshk", "d_k_bshk", "d_v_bshv", "d_erase_bshK",
+                              "d_write_bshV")):
+        assert rel_err(np_of(getattr(got, name)), want[i]) < bar(K), name
