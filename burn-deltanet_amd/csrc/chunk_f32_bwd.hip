@@ -483,11 +483,10 @@ hipError_t f32_bwd(const Dims& d, int qkv_dtype, int grad_dtype, const void* dy,
   if (e != hipSuccess) return e;
   // The two scans need nothing from each other: the reverse one runs on the
   // calling stream's second stream.
-  hipStream_t side = nullptr;
-  if ((e = side_fork(stream, &side)) != hipSuccess) return e;
-  if ((e = launch_rev(p, grad_dtype, side)) != hipSuccess) return e;
-  if ((e = f32_scan(p, qkv_dtype, DN_F32, true, stream)) != hipSuccess) return e;
-  if ((e = side_join(stream)) != hipSuccess) return e;
+  e = side_by_side(
+      stream, [&](hipStream_t side) { return launch_rev(p, grad_dtype, side); },
+      [&] { return f32_scan(p, qkv_dtype, DN_F32, true, stream); });
+  if (e != hipSuccess) return e;
   return launch_chunk_bwd(p, qkv_dtype, grad_dtype, stream);
 }
 

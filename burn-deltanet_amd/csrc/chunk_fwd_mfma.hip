@@ -1656,6 +1656,52 @@ hipError_t launch_scan(const MfmaParams& p, const Dims& d, bool yb, hipStream_t 
   return hipGetLastError();
 }
 
+hipError_t launch_rev(const RevParams& p, const Dims& d, int grad_dtype, hipStream_t stream,
+                      bool g4) {
+  // head_k_dim 256: eight waves with ds_after in row groups of four (the
+  // generic kernels' row-major layout: four, whose single wave per SIMD has
+  // the register file for 256 dS rows beside the next chunk's 120 KB of
+  // tiles; eight waves spilled there). At B=8 T=4096 H=16 dv=256: eight
+  // waves row-major 5.05 ms, four 3.85, four in row groups 1.61, eight in
+  // row groups 1.36.
+  const ScanShape shape = scan_shape(d, true);
+  const int waves = d.K == 256 && !g4 ? 4 : shape.waves;
+  ProfScope ps("dn_mfma_rev_scan", stream);
+  if (shape.teams)
+    return g4 ? hipErrorInvalidValue
+              : launch_team_rev(p, d.K, grad_dtype == DN_BF16, shape.teams, stream);
+  const unsigned blocks = unsigned(((d.B * d.H + 7) / 8) * 8 * (d.V / (16 * waves)));
+#define DN_REV(KD, TG, W) \
+  hipLaunchKernelGGL((mfma_rev_scan_kernel<KD, TG, W>), dim3(blocks), dim3(64 * W), 0, stream, p)
+#define DN_REV4(KD, TG, W)                                                                     \
+  hipLaunchKernelGGL((mfma_rev_scan_kernel<KD, TG, W, true>), dim3(blocks), dim3(64 * W), 0,  \
+                     stream, p)
+#define DN_REV_W(KD, TG) \
+  do { if (waves == 8) DN_REV(KD, TG, 8); else DN_REV(KD, TG, 4); } while (0)
+  if (g4 && waves != 8 && d.K != 256) return hipErrorInvalidValue;
+  if (d.K == 256) {
+    if (g4) {
+      if (grad_dtype == DN_BF16) DN_REV4(256, bf16, 8); else DN_REV4(256, float, 8);
+    } else {
+      if (grad_dtype == DN_BF16) DN_REV(256, bf16, 4); else DN_REV(256, float, 4);
+    }
+  } else if (g4) {
+    if (d.K == 128) {
+      if (grad_dtype == DN_BF16) DN_REV4(128, bf16, 8); else DN_REV4(128, float, 8);
+    } else {
+      if (grad_dtype == DN_BF16) DN_REV4(64, bf16, 8); else DN_REV4(64, float, 8);
+    }
+  } else if (d.K == 128) {
+    if (grad_dtype == DN_BF16) DN_REV_W(128, bf16); else DN_REV_W(128, float);
+  } else {
+    if (grad_dtype == DN_BF16) DN_REV_W(64, bf16); else DN_REV_W(64, float);
+  }
+#undef DN_REV_W
+#undef DN_REV4
+#undef DN_REV
+  return hipGetLastError();
+}
+
 // Clears the output norm's exchange words (a fill kernel: the launch may be
 // captured into a HIP graph, where memset nodes are avoided).
 __global__ __launch_bounds__(256) void zero_words_kernel(unsigned long long* w, size_t n) {
@@ -1864,58 +1910,10 @@ hipError_t mfma_bwd_scans(const Dims& d, int grad_dtype, const void* dy,
   // The intra kernel writes the reverse scan's transposed tiles too.
   hipError_t e = launch_intra(p, d, stream, &bt);
   if (e != hipSuccess) return e;
-  hipStream_t side = nullptr;
-  if ((e = side_fork(stream, &side)) != hipSuccess) return e;
-  RevParams rp{d.B, d.S, d.H, d.V, d.N, dy, dstate_final, ds_after, dstate, bt};
-  // head_k_dim 256: eight waves with ds_after in row groups of four (the
-  // generic kernels' row-major layout: four, whose single wave per SIMD has
-  // the register file for 256 dS rows beside the next chunk's 120 KB of
-  // tiles; eight waves spilled there). At B=8 T=4096 H=16 dv=256: eight
-  // waves row-major 5.05 ms, four 3.85, four in row groups 1.61, eight in
-  // row groups 1.36.
-  const ScanShape shape = scan_shape(d, true);
-  const int waves = d.K == 256 && !g4 ? 4 : shape.waves;
-  {
-  ProfScope ps("dn_mfma_rev_scan", side);
-  if (shape.teams) {
-    if (g4) return hipErrorInvalidValue;
-    if ((e = launch_team_rev(rp, d.K, grad_dtype == DN_BF16, shape.teams, side)) != hipSuccess)
-      return e;
-  } else {
-  const unsigned blocks = unsigned(((d.B * d.H + 7) / 8) * 8 * (d.V / (16 * waves)));
-#define DN_REV(KD, TG, W) \
-  hipLaunchKernelGGL((mfma_rev_scan_kernel<KD, TG, W>), dim3(blocks), dim3(64 * W), 0, side, rp)
-#define DN_REV4(KD, TG, W)                                                                     \
-  hipLaunchKernelGGL((mfma_rev_scan_kernel<KD, TG, W, true>), dim3(blocks), dim3(64 * W), 0,  \
-                     side, rp)
-#define DN_REV_W(KD, TG) \
-  do { if (waves == 8) DN_REV(KD, TG, 8); else DN_REV(KD, TG, 4); } while (0)
-  if (g4 && waves != 8 && d.K != 256) return hipErrorInvalidValue;
-  if (d.K == 256) {
-    if (g4) {
-      if (grad_dtype == DN_BF16) DN_REV4(256, bf16, 8); else DN_REV4(256, float, 8);
-    } else {
-      if (grad_dtype == DN_BF16) DN_REV(256, bf16, 4); else DN_REV(256, float, 4);
-    }
-  } else if (g4) {
-    if (d.K == 128) {
-      if (grad_dtype == DN_BF16) DN_REV4(128, bf16, 8); else DN_REV4(128, float, 8);
-    } else {
-      if (grad_dtype == DN_BF16) DN_REV4(64, bf16, 8); else DN_REV4(64, float, 8);
-    }
-  } else if (d.K == 128) {
-    if (grad_dtype == DN_BF16) DN_REV_W(128, bf16); else DN_REV_W(128, float);
-  } else {
-    if (grad_dtype == DN_BF16) DN_REV_W(64, bf16); else DN_REV_W(64, float);
-  }
-#undef DN_REV_W
-#undef DN_REV4
-#undef DN_REV
-  }
-  }
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  if ((e = launch_scan<true>(p, d, false, stream, g4)) != hipSuccess) return e;
-  return side_join(stream);
+  const RevParams rp{d.B, d.S, d.H, d.V, d.N, dy, dstate_final, ds_after, dstate, bt};
+  return side_by_side(
+      stream, [&](hipStream_t side) { return launch_rev(rp, d, grad_dtype, side, g4); },
+      [&] { return launch_scan<true>(p, d, false, stream, g4); });
 }
 
 }  // namespace dn

@@ -247,6 +247,20 @@ int device_cu_count();
 // may overlap what `main` gets next; side_join(main) makes `main` wait for it.
 hipError_t side_fork(hipStream_t main, hipStream_t* side);
 hipError_t side_join(hipStream_t main);
+// on_side(side) on the second stream beside on_main() on `main`, joined
+// whatever either returns: what was launched on the second stream would
+// otherwise run on after the call, in memory that its caller has back, or
+// stay unjoined in a capture.
+template <class Side, class Main>
+hipError_t side_by_side(hipStream_t main, Side on_side, Main on_main) {
+  hipStream_t side = nullptr;
+  hipError_t e = side_fork(main, &side);
+  if (e != hipSuccess) return e;
+  e = on_side(side);
+  if (e == hipSuccess) e = on_main();
+  const hipError_t joined = side_join(main);
+  return e != hipSuccess ? e : joined;
+}
 
 // NaN/Inf guard: sets *flag (device int) to 1 if any element is not finite.
 hipError_t launch_nonfinite_scan(const void* p, size_t n, int dtype, int* flag,

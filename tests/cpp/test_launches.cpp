@@ -34,6 +34,10 @@ int device = 0;  // current device: how many CUs it has
 const int kCus[] = {256, 128, 64, 32};
 int blocks_per_cu = 0;  // what the occupancy query answers
 void (*on_launch)(const Launch&) = nullptr;
+int launches = 0, failing = 0;  // the launch whose check reports an error, from 1; 0: none
+// Waits of the second stream for the caller's, and of the caller's for it.
+int forks = 0, joins = 0;
+const hipStream_t kSide = reinterpret_cast<hipStream_t>(uintptr_t(1) << 12);
 
 void fail(const std::string& what) {
   std::fprintf(stderr, "FAIL %s\n", what.c_str());
@@ -44,6 +48,7 @@ hipError_t record(const void* f, void** args) {
   const auto it = kernels().find(f);
   if (it == kernels().end()) fail("launch of an unregistered kernel");
   if (on_launch) on_launch({it->second, args[0]});
+  ++launches;
   return hipSuccess;
 }
 
@@ -69,7 +74,19 @@ hipError_t hipLaunchCooperativeKernel(const void* f, dim3, dim3, void** args, un
                                       hipStream_t) {
   return record(f, args);
 }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+  return failing && launches == failing ? hipErrorLaunchFailure : hipSuccess;
+}
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
+  *s = kSide;
+  return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t*, unsigned) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t, unsigned) {
+  ++(s == kSide ? forks : joins);
+  return hipSuccess;
+}
 hipError_t hipGetDevice(int* d) {
   *d = device;
   return hipSuccess;
@@ -156,10 +173,55 @@ void out_norm_fallback() {
   std::printf("ok out_norm_fallback (%d segmented calls)\n", cut);
 }
 
+// dn_chunk_bwd where its launches fail one by one: what it left on the second
+// stream is joined whenever it returns.
+void backward_joins() {
+  on_launch = nullptr;
+  const struct {
+    int dtype, S, H, K, V;
+    bool channel;
+  } cases[] = {{DN_F32, 130, 2, 64, 64, false},     {DN_BF16, 130, 2, 128, 128, false},
+               {DN_BF16, 130, 2, 128, 128, true},   {DN_BF16, 130, 2, 256, 128, false},
+               {DN_BF16, 130, 96, 128, 256, false}, {DN_BF16, 130, 2, 64, 64, false}};
+  for (const auto& c : cases) {
+    dn_chunk_bwd_args a{};
+    a.batch = 1, a.sequence = c.S, a.nheads = c.H, a.head_k_dim = c.K, a.head_v_dim = c.V;
+    a.erase_width = a.decay_width = c.channel ? c.K : 1;
+    a.write_width = c.channel ? c.V : 1;
+    a.has_gate = 1, a.chunk_len = 64, a.scale = std::nan("");
+    a.qkv_dtype = a.grad_dtype = c.dtype;
+    void* const t = const_cast<void*>(kTensor);
+    float* const f = static_cast<float*>(t);
+    a.d_y = a.q = a.k = a.v = t;
+    a.erase = a.write = a.g = a.state_in = f;
+    a.d_q = a.d_k = a.d_v = t;
+    a.d_erase = a.d_write = a.d_g = a.d_state = f;
+    a.workspace = kWorkspace;
+    a.workspace_bytes = dn_chunk_bwd_workspace_bytes(&a);
+    launches = failing = forks = joins = 0;
+    if (dn_chunk_bwd(&a, nullptr) != DN_OK) fail(dn_last_error());
+    const int all = launches;
+    if (all < 4 || forks != 1 || joins != 1) fail("backward: one fork and one join");
+    for (int n = 1; n <= all; ++n) {
+      launches = forks = joins = 0;
+      failing = n;
+      if (dn_chunk_bwd(&a, nullptr) != DN_ERR_HIP) fail("backward: a failed launch is reported");
+      if (launches != n) fail("backward: nothing is launched after a failure");
+      if (forks != joins)
+        fail("backward of K " + std::to_string(c.K) + " dtype " + std::to_string(c.dtype) +
+             ": launch " + std::to_string(n) + " of " + std::to_string(all) +
+             " failed, and the second stream was not joined");
+    }
+    failing = 0;
+  }
+  std::printf("ok backward_joins\n");
+}
+
 }  // namespace
 
 int main() {
   out_norm_fallback();
+  backward_joins();
   std::printf("all passed\n");
   return 0;
 }
