@@ -316,6 +316,12 @@ size_t fwd_workspace(const Dims& d, int algo) {
   return mfma_fwd_workspace(d, algo == DN_ALGO_MFMA_FUSED);
 }
 
+// The least a caller's workspace must hold.
+size_t fwd_least_workspace(const Dims& d, int algo) {
+  if (algo == DN_ALGO_GENERIC) return generic_fwd_workspace(d);
+  return mfma_fwd_least_workspace(d, algo == DN_ALGO_MFMA_FUSED);
+}
+
 Dims bwd_dims(const dn_chunk_bwd_args* a) {
   return make_dims(a->batch, a->sequence, a->nheads, a->head_k_dim, a->head_v_dim,
                    a->erase_width, a->write_width, a->decay_width, a->has_gate, a->chunk_len,
@@ -393,7 +399,7 @@ int dn_chunk_fwd(const dn_chunk_fwd_args* a, hipStream_t stream) {
   void* ws = a->workspace;
   const size_t ws_bytes = ws ? a->workspace_bytes : need;
   if (ws) {
-    if (ws_bytes < need)
+    if (ws_bytes < fwd_least_workspace(d, algo))
       return fail(DN_ERR_WORKSPACE, "workspace too small: need " + std::to_string(need) +
                                         " bytes");
   } else if (need) {
@@ -526,7 +532,7 @@ int dn_chunk_fwd_out_norm(const dn_chunk_fwd_out_norm_args* a, hipStream_t strea
   void* ws = f->workspace;
   const size_t ws_bytes = ws ? f->workspace_bytes : need;
   if (ws) {
-    if (ws_bytes < need)
+    if (ws_bytes < (in_scan ? need : fwd_least_workspace(d, algo)))
       return fail(DN_ERR_WORKSPACE, "workspace too small: need " + std::to_string(need) +
                                         " bytes");
   } else if (need) {
@@ -846,7 +852,7 @@ int dn_frontend_chunk_fwd(const dn_frontend_chunk_fwd_args* a, hipStream_t strea
   void* ws = f->workspace;
   const size_t ws_bytes = ws ? f->workspace_bytes : need;
   if (ws) {
-    if (ws_bytes < need)
+    if (ws_bytes < fwd_least_workspace(d, algo))
       return fail(DN_ERR_WORKSPACE, "workspace too small: need " + std::to_string(need) +
                                         " bytes");
   } else if (need) {

@@ -1791,6 +1791,13 @@ size_t mfma_fwd_workspace(const Dims& d, bool fused) {
   return fused ? fused_fwd_workspace(d) : tiles_workspace(d) + seg_bytes(d, seg_parts(d, SIZE_MAX));
 }
 
+// Callers with a fixed buffer hold what the segments of norm_seg_parts take:
+// seg_parts finds some faster with more of them, and uses those that fit.
+size_t mfma_fwd_least_workspace(const Dims& d, bool fused) {
+  const size_t all = mfma_fwd_workspace(d, fused);
+  return fused ? all : std::min(all, tiles_workspace(d) + seg_bytes(d, norm_seg_parts(d)));
+}
+
 hipError_t mfma_fwd(const Dims& d, int y_dtype, const void* q, const void* k, const void* v,
                     const float* erase, const float* write, const float* g,
                     const float* state_in, void* y, float* state_out, void* ws, size_t ws_bytes,

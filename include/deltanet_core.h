@@ -95,7 +95,7 @@ typedef enum {
   DN_ERR_NONFINITE = -5,   /* NaN/Inf guard on inputs or outputs (sanity, path.rs:198-207) */
   DN_ERR_NULL = -6,        /* a required pointer is NULL */
   DN_ERR_DTYPE = -7,       /* unknown dtype tag */
-  DN_ERR_WORKSPACE = -8,   /* caller workspace smaller than dn_*_workspace_bytes() */
+  DN_ERR_WORKSPACE = -8,   /* caller workspace too small (dn_*_workspace_bytes()) */
   DN_ERR_UNSUPPORTED = -9, /* DN_ALGO_MFMA requested for a shape it does not cover */
   DN_ERR_HIP = -10,        /* a HIP runtime call failed */
 } dn_status;
@@ -445,7 +445,12 @@ int dn_unit_lower_inverse(const dn_tri_args *args, hipStream_t stream);
  * first call at a new largest size is not asynchronous; under HIP graph
  * capture growth is refused (DN_ERR_HIP, hipErrorStreamCaptureUnsupported).
  * Callers that capture graphs, use several streams, or must not allocate in
- * the call pass their own workspace of at least these many bytes. */
+ * the call pass their own workspace of at least these many bytes. For a
+ * forward on the MFMA path over few long sequences, they include the buffers
+ * of the segments that it cuts those into for speed. Such a call is also served
+ * from a smaller workspace, with the segments that fit there: one that holds
+ * its tiles and, at head_k_dim 128 with head_v_dim a multiple of 128, segments
+ * for one 128-column workgroup per CU. */
 size_t dn_chunk_fwd_workspace_bytes(const dn_chunk_fwd_args *args);
 size_t dn_chunk_bwd_workspace_bytes(const dn_chunk_bwd_args *args);
 

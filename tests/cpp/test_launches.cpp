@@ -173,6 +173,32 @@ void out_norm_fallback() {
   std::printf("ok out_norm_fallback (%d segmented calls)\n", cut);
 }
 
+// A workspace of the size that fewer segments, or none, took serves the call,
+// which keeps to it; a smaller one is refused.
+void smaller_workspaces() {
+  on_launch = see_segments;
+  const struct {
+    int S, K, V;
+    size_t bytes;
+  } cases[] = {{4096, 64, 128, 1589760}, {4096, 128, 576, 1591552}, {8192, 128, 192, 3179264},
+               {16384, 64, 576, 6359296}, {2048, 64, 64, 794880}};
+  for (const auto& c : cases) {
+    dn_chunk_fwd_args a = forward(1, c.S, 1, c.K, c.V, false);
+    if (dn_chunk_fwd_workspace_bytes(&a) <= c.bytes) fail("smaller workspace: not smaller");
+    for (size_t more : {size_t(0), size_t(1) << 19, size_t(1) << 26}) {
+      a.workspace_bytes = c.bytes + more;
+      segments = {};
+      if (dn_chunk_fwd(&a, nullptr) != DN_OK) fail(dn_last_error());
+      if (segments.end > kWorkspace + a.workspace_bytes) fail("smaller workspace: left");
+      if (more > dn_chunk_fwd_workspace_bytes(&a) && segments.parts < 2)
+        fail("smaller workspace: a large one is not cut");
+    }
+    a.workspace_bytes = c.bytes - 1;
+    if (dn_chunk_fwd(&a, nullptr) != DN_ERR_WORKSPACE) fail("smaller workspace: accepted");
+  }
+  std::printf("ok smaller_workspaces\n");
+}
+
 // dn_chunk_bwd where its launches fail one by one: what it left on the second
 // stream is joined whenever it returns.
 void backward_joins() {
@@ -221,6 +247,7 @@ void backward_joins() {
 
 int main() {
   out_norm_fallback();
+  smaller_workspaces();
   backward_joins();
   std::printf("all passed\n");
   return 0;

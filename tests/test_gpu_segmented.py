@@ -97,3 +97,23 @@ def test_short_or_ragged_sequences_are_not_segmented(rng):
     for S in (1024, 4000):
         g_args = to_gpu(inputs(rng, 1, S, 1, 128, 128, "head", 0.0), torch.bfloat16)
         assert "dn_mfma_seg_carry" not in run(g_args)[2]
+
+
+@pytest.mark.parametrize("S,K,V,held", [(4096, 64, 128, 1589760),    # the tiles alone
+                                        (4096, 64, 128, 2000000),    # fewer segments than asked
+                                        (4096, 128, 576, 1591552)])
+def test_smaller_workspaces(rng, S, K, V, held):
+    """A workspace below the query's serves the call, which stays inside it."""
+    announce(f"segmented scan: workspace of {held} for S {S} K {K} V {V}")
+    g_args = to_gpu(inputs(rng, 1, S, 1, K, V, "head", 0.1), torch.bfloat16)
+    y = torch.empty(g_args[2].shape, dtype=torch.float32, device=DEV)
+    s = torch.empty_like(g_args[6])
+    a = abi.chunk_fwd_args(*g_args, y, s, 64, None)
+    most = abi.lib().dn_chunk_fwd_workspace_bytes(a)
+    assert most > held
+    ws = torch.full((most + 256,), 77, dtype=torch.uint8, device=DEV)
+    a.workspace, a.workspace_bytes = ws.data_ptr(), held
+    abi.run_chunk_fwd(a)
+    y0, s0 = O.chunk_fwd(*as_oracle_inputs(g_args), chunk_len=64, dtype=np.float64)
+    assert rel_err(np_of(y), y0) < TOL and rel_err(np_of(s), s0) < TOL
+    assert bool((ws[held:] == 77).all())
