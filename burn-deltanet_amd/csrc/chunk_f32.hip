@@ -124,12 +124,12 @@ __global__ __launch_bounds__(256) void f32_intra_kernel(FParams p) {
         uu[r] = kr[i][r] * expf(Gl[r] - G[r]);
         qq[r] = q[r] * eg;
       }
-      st4(&ws[o.a + at], a);
-      st4(&ws[o.u + at], uu);
-      st4(&ws[o.q + at], qq);
+      stw(&ws[o.a + at], a);
+      stw(&ws[o.u + at], uu);
+      stw(&ws[o.q + at], qq);
     } else {
-      st4(&ws[o.a + at], kr[i]);
-      st4(&ws[o.q + at], q);
+      stw(&ws[o.a + at], kr[i]);
+      stw(&ws[o.q + at], q);
     }
   }
   if (tid < kC) {
@@ -360,7 +360,7 @@ __global__ __launch_bounds__(256 * C + 256) void f32_scan_kernel(FParams p) {
 #pragma unroll
         for (int i = 0; i < NR; ++i)
           if (tw + 4 * i < KB)
-            st4(p.states + ((cid * KB + tw + 4 * i) * VB + ct) * kBlk + 4 * lane, S[i]);
+            stw(p.states + ((cid * KB + tw + 4 * i) * VB + ct) * kBlk + 4 * lane, S[i]);
     }
     // K·S and Q·S of this wave's token block.
     f32x4 ks = zero4(), qs = zero4();
@@ -387,7 +387,7 @@ __global__ __launch_bounds__(256 * C + 256) void f32_scan_kernel(FParams p) {
     }
     load_v(nn);
     st4(&Xx[team][tb * kBlk + 4 * lane], X);
-    if (ST && ct < VB) st4(p.xs + ((cid * 4 + tb) * VB + ct) * kBlk + 4 * lane, X);
+    if (ST && ct < VB) stw(p.xs + ((cid * 4 + tb) * VB + ct) * kBlk + 4 * lane, X);
     lds_barrier();
     // V' = T·X
     f32x4 Vn = zero4();
@@ -397,7 +397,7 @@ __global__ __launch_bounds__(256 * C + 256) void f32_scan_kernel(FParams p) {
         Vn = mm(ld4(&tT[tri_blk(tb, j) * kBlk + fo]),
                 ld4(&Xx[team][j * kBlk + 4 * lane]), Vn);
     st4(&Vx[team][tb * kBlk + 4 * lane], Vn);
-    if (ST && ct < VB) st4(p.vn + ((cid * 4 + tb) * VB + ct) * kBlk + 4 * lane, Vn);
+    if (ST && ct < VB) stw(p.vn + ((cid * 4 + tb) * VB + ct) * kBlk + 4 * lane, Vn);
     lds_barrier();
     // y = ys⊙(Q·S) + attn·V' and S ← egl⊙S + Uᵀ·V'.
     if constexpr (!ST) {

@@ -95,6 +95,10 @@ namespace {
 __device__ inline f32x4 zero4() { return f32x4{0.f, 0.f, 0.f, 0.f}; }
 __device__ inline f32x4 ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 __device__ inline void st4(float* p, const f32x4& v) { *reinterpret_cast<f32x4*>(p) = v; }
+// The workspace, which the caller aligns to its elements and no further.
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+__device__ inline f32x4 ldw(const float* p) { return *reinterpret_cast<const f32x4_any*>(p); }
+__device__ inline void stw(float* p, const f32x4& v) { *reinterpret_cast<f32x4_any*>(p) = v; }
 
 // acc += A·B over a 16-deep contraction from the two operands' lane values.
 __device__ inline f32x4 mm(const f32x4& a, const f32x4& b, f32x4 acc) {
@@ -129,7 +133,7 @@ struct Piece {
   f32x4 x[N];
   __device__ void load(const float* src, int t) {
 #pragma unroll
-    for (int i = 0; i < N; ++i) x[i] = ld4(src + 4 * min(t + 256 * i, kWords - 1));
+    for (int i = 0; i < N; ++i) x[i] = ldw(src + 4 * min(t + 256 * i, kWords - 1));
   }
   __device__ void store(float* dst, int t) const {
 #pragma unroll

@@ -145,7 +145,7 @@ __global__ __launch_bounds__(256 * C + 256) void f32_rev_scan_kernel(FParams p) 
 #pragma unroll
       for (int i = 0; i < NR; ++i)
         if (tw + 4 * i < KB)
-          st4(p.ds_after + ((cid * KB + tw + 4 * i) * VB + ct) * kBlk + 4 * lane, S[i]);
+          stw(p.ds_after + ((cid * KB + tw + 4 * i) * VB + ct) * kBlk + 4 * lane, S[i]);
     f32x4 dv = zero4(), av = zero4();
 #pragma unroll
     for (int cb = 0; cb < KB; ++cb)
@@ -163,7 +163,7 @@ __global__ __launch_bounds__(256 * C + 256) void f32_rev_scan_kernel(FParams p) 
       for (int r = 0; r < 4; ++r) dv[r] = av[r] + (FOLD ? dv[r] : gk[r] * dv[r]);
     }
     st4(&Vx[tb * kBlk + 4 * lane], dv);
-    if (ct < VB) st4(p.dvn + ((cid * 4 + tb) * VB + ct) * kBlk + 4 * lane, dv);
+    if (ct < VB) stw(p.dvn + ((cid * 4 + tb) * VB + ct) * kBlk + 4 * lane, dv);
     lds_barrier();
     f32x4 z = zero4();
 #pragma unroll
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(256 * C + 256) void f32_rev_scan_kernel(FParams p) 
       if (j >= tb)
         z = mm(tr(&tT[tri_blk(j, tb) * kBlk]), ld4(&Vx[j * kBlk + 4 * lane]), z);
     st4(&Zx[team][tb * kBlk + 4 * lane], z);
-    if (ct < VB) st4(p.z + ((cid * 4 + tb) * VB + ct) * kBlk + 4 * lane, z);
+    if (ct < VB) stw(p.z + ((cid * 4 + tb) * VB + ct) * kBlk + 4 * lane, z);
     lds_barrier();
 #pragma unroll
     for (int i = 0; i < NR; ++i)
@@ -276,10 +276,10 @@ __global__ __launch_bounds__(64 * (KB < 4 ? 4 : KB)) void f32_chunk_bwd_kernel(F
     at4[r] = (row0 + size_t(min(16 * (wave & 3) + 4 * g4 + r, rl - 1)) * d.H) * d.V;
   auto load = [&](int vt) {
 #pragma unroll
-    for (int i = 0; i < NPT; ++i) pf[i] = ld4(src[i] + size_t(vt) * kBlk + 4 * lane);
+    for (int i = 0; i < NPT; ++i) pf[i] = ldw(src[i] + size_t(vt) * kBlk + 4 * lane);
     if (wave < 4) {
       const int col = 16 * vt + m16, cl = min(col, d.V - 1);
-      pz = ld4(zsrc + size_t(vt) * kBlk + 4 * lane);
+      pz = ldw(zsrc + size_t(vt) * kBlk + 4 * lane);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         py[r] = ld(dyp, at4[r] + cl);
@@ -367,7 +367,7 @@ __global__ __launch_bounds__(64 * (KB < 4 ? 4 : KB)) void f32_chunk_bwd_kernel(F
   __syncthreads();
 
   float *lT = lds;
-  for (int i = tid; i < kTri / 4; i += 64 * NW) st4(&lT[4 * i], ld4(ws + o.t + 4 * i));
+  for (int i = tid; i < kTri / 4; i += 64 * NW) st4(&lT[4 * i], ldw(ws + o.t + 4 * i));
   const ChunkTail x{d, row0, rl, p.erase, p.g, p.derase, p.dg};
   chunk_bwd_tail<KB, NW, PCG, EK>(x, DirectRows<TQ, TG>{x, p.q, p.k, p.dq, p.dk}, lds, red, sG,
                                   dkc, dqr, dkg, dat, dtt, degl);

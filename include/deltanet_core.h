@@ -450,7 +450,8 @@ int dn_unit_lower_inverse(const dn_tri_args *args, hipStream_t stream);
  * of the segments that it cuts those into for speed. Such a call is also served
  * from a smaller workspace, with the segments that fit there: one that holds
  * its tiles and, at head_k_dim 128 with head_v_dim a multiple of 128, segments
- * for one 128-column workgroup per CU. */
+ * for one 128-column workgroup per CU. A caller's workspace starts at a 16-byte
+ * boundary, where the call runs DN_ALGO_GENERIC at a 4-byte one. */
 size_t dn_chunk_fwd_workspace_bytes(const dn_chunk_fwd_args *args);
 size_t dn_chunk_bwd_workspace_bytes(const dn_chunk_bwd_args *args);
 

@@ -122,3 +122,26 @@ def test_short_chunks_are_as_accurate_as_their_length(rng, L, K):
     for i, name in enumerate(("d_q_bshk", "d_k_bshk", "d_v_bshv", "d_erase_bshK",
                               "d_write_bshV")):
         assert rel_err(np_of(getattr(got, name)), want[i]) < bar(K), name
+
+
+@pytest.mark.parametrize("V,widths", [(40, (1, 1, 1)), (24, (64, 24, 64))])
+def test_workspace_at_a_four_byte_boundary(rng, V, widths):
+    """The generic path's workspace is owed the alignment of its floats: one
+    that starts four bytes past a boundary holds the same bits."""
+    announce(f"f32 kernels: workspace off a 16-byte boundary V {V} {widths}")
+    B, S, H, K = 1, 130, 2, 64
+    args = to_gpu(inputs(rng, B, S, H, K, V, *widths))
+    dy = torch.tensor(rng.standard_normal((B, S, H, V)), dtype=torch.float32, device=DEV)
+    lib, out = pkg.abi.lib(), []
+    for off in (0, 4):
+        y, s = torch.empty_like(args[2]), torch.empty_like(args[6])
+        grads = [torch.empty_like(t) for t in args]
+        fwd = pkg.abi.chunk_fwd_args(*args, y, s, 64, 0.5, algo=GENERIC)
+        bwd = pkg.abi.chunk_bwd_args(dy, None, *args, grads, 64, 0.5, algo=GENERIC)
+        for a, size, run in ((fwd, lib.dn_chunk_fwd_workspace_bytes, pkg.abi.run_chunk_fwd),
+                             (bwd, lib.dn_chunk_bwd_workspace_bytes, pkg.abi.run_chunk_bwd)):
+            ws = torch.empty(size(a) + off, dtype=torch.uint8, device=DEV)
+            a.workspace, a.workspace_bytes = ws.data_ptr() + off, size(a)
+            profiled(lambda: run(a))
+        out.append([y, s] + grads)
+    assert all(torch.equal(a, b) for a, b in zip(*out))
