@@ -311,15 +311,11 @@ int fwd_algo(const dn_chunk_fwd_args* a, const Dims& d0) {
   return fits ? DN_ALGO_MFMA : DN_ALGO_GENERIC;
 }
 
-size_t fwd_workspace(const Dims& d, int algo) {
+// What the forward uses of `room` bytes of workspace, or needs where that is
+// more.
+size_t fwd_workspace(const Dims& d, int algo, size_t room = SIZE_MAX) {
   if (algo == DN_ALGO_GENERIC) return generic_fwd_workspace(d);
-  return mfma_fwd_workspace(d, algo == DN_ALGO_MFMA_FUSED);
-}
-
-// The least a caller's workspace must hold.
-size_t fwd_least_workspace(const Dims& d, int algo) {
-  if (algo == DN_ALGO_GENERIC) return generic_fwd_workspace(d);
-  return mfma_fwd_least_workspace(d, algo == DN_ALGO_MFMA_FUSED);
+  return mfma_fwd_workspace(d, algo == DN_ALGO_MFMA_FUSED, room);
 }
 
 Dims bwd_dims(const dn_chunk_bwd_args* a) {
@@ -399,7 +395,7 @@ int dn_chunk_fwd(const dn_chunk_fwd_args* a, hipStream_t stream) {
   void* ws = a->workspace;
   const size_t ws_bytes = ws ? a->workspace_bytes : need;
   if (ws) {
-    if (ws_bytes < fwd_least_workspace(d, algo))
+    if (ws_bytes < need && ws_bytes < fwd_workspace(d, algo, ws_bytes))
       return fail(DN_ERR_WORKSPACE, "workspace too small: need " + std::to_string(need) +
                                         " bytes");
   } else if (need) {
@@ -447,7 +443,7 @@ int dn_chunk_fwd_noalloc(const dn_chunk_fwd_args* a, hipStream_t stream) {
   if (algo < 0)
     return fail(DN_ERR_UNSUPPORTED, "the requested MFMA path does not cover this shape/dtype");
   d = run_dims(d, algo);
-  const size_t need = fwd_workspace(d, algo);
+  const size_t need = fwd_workspace(d, algo, DN_NOALLOC_SCRATCH_BYTES);
   if (need > size_t(DN_NOALLOC_SCRATCH_BYTES))
     return fail(DN_ERR_WORKSPACE,
                 "dn_chunk_fwd_noalloc: these arguments need " + std::to_string(need) +
@@ -532,7 +528,7 @@ int dn_chunk_fwd_out_norm(const dn_chunk_fwd_out_norm_args* a, hipStream_t strea
   void* ws = f->workspace;
   const size_t ws_bytes = ws ? f->workspace_bytes : need;
   if (ws) {
-    if (ws_bytes < (in_scan ? need : fwd_least_workspace(d, algo)))
+    if (ws_bytes < need && (in_scan || ws_bytes < fwd_workspace(d, algo, ws_bytes)))
       return fail(DN_ERR_WORKSPACE, "workspace too small: need " + std::to_string(need) +
                                         " bytes");
   } else if (need) {
@@ -852,7 +848,7 @@ int dn_frontend_chunk_fwd(const dn_frontend_chunk_fwd_args* a, hipStream_t strea
   void* ws = f->workspace;
   const size_t ws_bytes = ws ? f->workspace_bytes : need;
   if (ws) {
-    if (ws_bytes < fwd_least_workspace(d, algo))
+    if (ws_bytes < need && ws_bytes < fwd_workspace(d, algo, ws_bytes))
       return fail(DN_ERR_WORKSPACE, "workspace too small: need " + std::to_string(need) +
                                         " bytes");
   } else if (need) {

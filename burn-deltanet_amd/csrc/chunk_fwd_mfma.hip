@@ -1478,18 +1478,13 @@ int norm_scan_waves(const Dims& d) {
   return best;
 }
 
-// Segments per sequence for a scan by teams, where its three passes (the
-// transitions cover K extra columns; then the carry; then the outputs) cost
-// less than one scan by a twelfth: a pass is its chunks and about 4 us, the
-// carry 3 us a segment (1.3 at head_k_dim 64), two more launches 5. Sequences
-// of 32 whole chunks or more, in segments of 8 or more; the last may be shorter. The
-// segments' buffers must fit `room` bytes of workspace behind the tiles, and
-// must not take a call past the fixed scratch of dn_chunk_fwd_noalloc that its
-// tiles fit. Calls, us, whole and segmented:
-// S=8192 dk=dv=128, 1 head, per channel 190 and 90; 4 heads, per-head gates,
-// dv 256: S=16384 323 and 197, S=8192 166 and 122; dk 64, 2 heads: S=16384 258
-// and 75. 32 heads at S=16384 per channel, 596 us of scans in segments of
-// eight-wave workgroups before, take 514 whole.
+// How the segmented scan covers a sequence: `parts` segments (1: not cut), its
+// two passes by teams or by lone workgroups of eight waves.
+struct SegPlan {
+  int parts;
+  bool lone;
+};
+
 float teams_us(const Dims& d, int V, int P) {
   Dims s = d;
   s.B = d.B * P;
@@ -1514,33 +1509,21 @@ size_t seg_bytes(const Dims& d, int P) {
   const size_t bh = size_t(d.B) * P * d.H, K = size_t(d.K);
   return P == 1 ? 0 : region(bh * K * K * 4) + 2 * region(bh * K * d.V * 4);
 }
-int seg_parts(const Dims& d, size_t room) {
-  if (d.K > 128 || d.N < 32 || size_t(d.S) != size_t(d.N) * d.L) return 1;
-  const ScanShape w = scan_shape(d, false);
-  float least = chunk_us(d, w) * float(d.N) *
-                    float(scan_rounds(d, w.teams ? 16 * w.teams : 16 * w.waves, 1)) + 4.f;
-  int best = 1;
-  for (int P = 2; d.N >= 8 * P && P <= 64; P *= 2) {
-    const size_t tiles = tiles_workspace(d), bytes = tiles + seg_bytes(d, P);
-    if (bytes > room || (tiles <= DN_NOALLOC_SCRATCH_BYTES && bytes > DN_NOALLOC_SCRATCH_BYTES))
-      break;
-    const float n = float((d.N + P - 1) / P);
-    const float cut = n * (teams_us(d, d.V + d.K, P) + teams_us(d, d.V, P)) +
-                      (d.K == 128 ? 3.05f : 1.3f) * float(P) + 13.f;
-    if (cut < 0.92f * least) {
-      best = P;
-      least = cut;
-    }
-  }
-  return best;
+// The dims of segments by lone waves: batch b·P + s runs segment s of batch b.
+Dims seg_dims(const Dims& d, int P) {
+  Dims s = d;
+  s.B = d.B * P;
+  s.S = d.S / P;
+  s.N = d.N / P;
+  return s;
 }
 
-// Segments for the scan with the output norm in its y write, which has
-// 8-wave workgroups in both passes: enough to fill the device with them, of
+// Segments for passes by 8-wave workgroups: enough to fill the device with them, of
 // at least 16 whole chunks each (head_k_dim 128, head_v_dim a multiple of
 // 128, a sequence of whole chunks), where even 2-wave workgroups would leave
-// half the device idle, since segmenting triples the scans' work.
-int norm_seg_parts(const Dims& d) {
+// half the device idle, since segmenting triples the scans' work. The scan with
+// the output norm in its y write has no others.
+int lone_seg_parts(const Dims& d) {
   if (d.K != 128 || d.V % 128 != 0 || size_t(d.S) != size_t(d.N) * d.L) return 1;
   const size_t cus = size_t(device_cu_count());
   if (size_t(d.B) * d.H * (d.V / 32) * 2 > cus) return 1;
@@ -1548,6 +1531,49 @@ int norm_seg_parts(const Dims& d) {
   int P = 1;
   while (wgs * P * 2 <= cus && d.N % (P * 2) == 0 && d.N / (P * 2) >= 16) P *= 2;
   return P;
+}
+
+// The segments whose three passes (the transitions cover K extra columns; then
+// the carry; then the outputs) cost less than one scan. By teams, of 8 chunks
+// or more, the last of which may be shorter: less by a twelfth, and again for
+// each doubling, with a pass its chunks and about 4 us, the carry 3 us a segment
+// (1.3 at head_k_dim 64), two more launches 5. Calls, us, whole and cut: S=8192
+// dk=dv=128, 1 head, per channel 190 and 90; 4 heads, per-head gates, dv 256:
+// S=16384 323 and 197, S=8192 166 and 122; dk 64, 2 heads: S=16384 258 and 75.
+// Or by 8-wave workgroups (lone_seg_parts), which cover 128 columns with one
+// staging: less than that by a twentieth, at 4.1 us a chunk (5.1 per channel)
+// and 5 a segment, fitted to 448 calls of 1 to 16 heads, dv 128 to 512 and 32
+// to 512 chunks, of which it leaves 11 on their slower side, all past dv 256 or
+// 256 chunks: by 3 to 7%, and 3 heads of dv 512 by 4 to 15%. Calls, us, by teams
+// and by 8 waves: S=16384 dv 256, 8 heads 339 and 265 (per channel 459 and 397),
+// 4 heads 187 and 185 (233 and 242); S=12288 dv 256, 4 heads 152 and 205; whole
+// and by 8 waves: S=16384 dv 128, 16 heads 402 and 316 (644 and 527).
+// Sequences of 32 whole chunks or more. The segments' buffers must fit `room`
+// bytes of workspace behind the tiles.
+SegPlan seg_plan(const Dims& d, size_t room) {
+  SegPlan best{1, false};
+  if (d.K > 128 || d.N < 32 || size_t(d.S) != size_t(d.N) * d.L) return best;
+  auto fits = [&](int P) { return tiles_workspace(d) + seg_bytes(d, P) <= room; };
+  const ScanShape w = scan_shape(d, false);
+  float least = chunk_us(d, w) * float(d.N) *
+                    float(scan_rounds(d, w.teams ? 16 * w.teams : 16 * w.waves, 1)) + 4.f;
+  for (int P = 2; d.N >= 8 * P && P <= 64 && fits(P); P *= 2) {
+    const float n = float((d.N + P - 1) / P);
+    const float cut = n * (teams_us(d, d.V + d.K, P) + teams_us(d, d.V, P)) +
+                      (d.K == 128 ? 3.05f : 1.3f) * float(P) + 13.f;
+    if (cut < 0.92f * least) {
+      best = {P, false};
+      least = cut;
+    }
+  }
+  const int P = lone_seg_parts(d);
+  if (P == 1 || !fits(P)) return best;
+  const Dims s = seg_dims(d, P);
+  Dims m = s;
+  m.V = d.V + d.K;
+  const float us = (pc_path(d) ? 5.1f : 4.1f) * float(s.N) *
+                       float(scan_rounds(m, 128, 1) + scan_rounds(s, 128, 1)) + 5.f * float(P);
+  return us < 0.95f * least ? SegPlan{P, true} : best;
 }
 
 // The segmented scan's buffers, after the tiles in the workspace.
@@ -1571,13 +1597,27 @@ hipError_t launch_carry(const MfmaParams& p, const Dims& d, hipStream_t stream) 
   return hipGetLastError();
 }
 
-// The dims of the segmented scans: batch b·P + s runs segment s of batch b.
-Dims seg_dims(const Dims& d, int P) {
-  Dims s = d;
-  s.B = d.B * P;
-  s.S = d.S / P;
-  s.N = d.N / P;
-  return s;
+// Of a segmented call's parameters p, those of the segments' transitions by
+// lone waves (dims ds), and of the pass that writes the outputs from the
+// carried starts.
+MfmaParams lone_segs(const MfmaParams& p, const Dims& d, const Dims& ds) {
+  MfmaParams a = p;
+  a.B = ds.B;
+  a.S = ds.S;
+  a.N = ds.N;
+  a.seg = 1;
+  a.vx = d.V + d.K;
+  a.y = nullptr;
+  return a;
+}
+MfmaParams lone_outputs(const MfmaParams& segs, const MfmaParams& p) {
+  MfmaParams a = segs;
+  a.seg = 2;
+  a.vx = p.V;
+  a.s_in = p.seg_start;
+  a.y = p.y;
+  a.seg_final = p.s_out;
+  return a;
 }
 
 // g4 (ST): write the states in row groups of four (states_g4).
@@ -1587,16 +1627,27 @@ hipError_t launch_scan(const MfmaParams& p, const Dims& d, bool yb, hipStream_t 
   const bool pc = pc_path(d);
   if constexpr (!ST) {
     if (p.seg) {
-      // The transitions of the output norm's segmented scan: 8-wave
-      // workgroups, head_k_dim 128.
+      // The segmented scans: 8-wave workgroups, head_k_dim 128.
       const unsigned blocks = unsigned(((d.B * d.H + 7) / 8) * 8 * (p.vx / 128));
-      ProfScope ps(pc ? "dn_mfma_scan_pc_segs" : "dn_mfma_scan_segs", stream);
-      if (pc)
-        hipLaunchKernelGGL((mfma_scan_kernel<128, float, 8, true, false, 1>), dim3(blocks),
-                           dim3(512), 0, stream, p);
+      ProfScope ps(p.seg == 1 ? (pc ? "dn_mfma_scan_pc_segs" : "dn_mfma_scan_segs")
+                              : (pc ? "dn_mfma_scan_pc" : "dn_mfma_scan"),
+                   stream);
+#define DN_SEG(TY, SG)                                                                     \
+  do {                                                                                     \
+    if (pc)                                                                                \
+      hipLaunchKernelGGL((mfma_scan_kernel<128, TY, 8, true, false, SG>), dim3(blocks),    \
+                         dim3(512), 0, stream, p);                                         \
+    else                                                                                   \
+      hipLaunchKernelGGL((mfma_scan_kernel<128, TY, 8, false, false, SG>), dim3(blocks),   \
+                         dim3(512), 0, stream, p);                                         \
+  } while (0)
+      if (p.seg == 1)
+        DN_SEG(float, 1);  // no y
+      else if (yb)
+        DN_SEG(bf16, 2);
       else
-        hipLaunchKernelGGL((mfma_scan_kernel<128, float, 8, false, false, 1>), dim3(blocks),
-                           dim3(512), 0, stream, p);
+        DN_SEG(float, 2);
+#undef DN_SEG
       return hipGetLastError();
     }
   }
@@ -1715,7 +1766,7 @@ __global__ __launch_bounds__(256) void zero_words_kernel(unsigned long long* w, 
 size_t norm_words(const Dims& d, int P, int waves) {
   return size_t(d.B) * P * d.H * (d.V / (16 * waves)) * 4 * kL;
 }
-size_t norm_exchange_bytes(const Dims& d) { return region(norm_words(d, norm_seg_parts(d), 2) * 8); }
+size_t norm_exchange_bytes(const Dims& d) { return region(norm_words(d, lone_seg_parts(d), 2) * 8); }
 
 // The output-norm scan's launch geometry for dims `d` (the segmented output
 // pass's dims when seg): workgroup waves and column workgroups per head.
@@ -1787,15 +1838,9 @@ bool mfma_bwd_supported(const Dims& d, int qkv_dtype) {
   return d.K <= 128 && (per_channel(d) || (d.ew == 1 && d.ww == 1));
 }
 
-size_t mfma_fwd_workspace(const Dims& d, bool fused) {
-  return fused ? fused_fwd_workspace(d) : tiles_workspace(d) + seg_bytes(d, seg_parts(d, SIZE_MAX));
-}
-
-// Callers with a fixed buffer hold what the segments of norm_seg_parts take:
-// seg_parts finds some faster with more of them, and uses those that fit.
-size_t mfma_fwd_least_workspace(const Dims& d, bool fused) {
-  const size_t all = mfma_fwd_workspace(d, fused);
-  return fused ? all : std::min(all, tiles_workspace(d) + seg_bytes(d, norm_seg_parts(d)));
+size_t mfma_fwd_workspace(const Dims& d, bool fused, size_t room) {
+  if (fused) return fused_fwd_workspace(d);
+  return tiles_workspace(d) + seg_bytes(d, seg_plan(d, room).parts);
 }
 
 hipError_t mfma_fwd(const Dims& d, int y_dtype, const void* q, const void* k, const void* v,
@@ -1807,12 +1852,19 @@ hipError_t mfma_fwd(const Dims& d, int y_dtype, const void* q, const void* k, co
   MfmaParams p = make_params(d, q, k, v, erase, write, g, state_in, y, state_out, ws);
   hipError_t e = launch_intra(p, d, stream, nullptr, fe);
   if (e != hipSuccess) return e;
-  const int P = seg_parts(d, ws_bytes);
+  const SegPlan plan = seg_plan(d, ws_bytes);
+  const int P = plan.parts;
   const bool yb = y_dtype == DN_BF16, pc = pc_path(d);
   if (P == 1) return launch_scan<false>(p, d, yb, stream);
-  // Segmented: the segments' transitions, the carry, then the outputs.
   carve_seg(p, d, P, static_cast<char*>(ws) + tiles_workspace(d));
   p.seg_p = P;
+  if (plan.lone) {
+    const Dims ds = seg_dims(d, P);
+    const MfmaParams pa = lone_segs(p, d, ds);
+    if ((e = launch_scan<false>(pa, ds, yb, stream)) != hipSuccess) return e;
+    if ((e = launch_carry(p, d, stream)) != hipSuccess) return e;
+    return launch_scan<false>(lone_outputs(pa, p), ds, yb, stream);
+  }
   p.seg_n = (d.N + P - 1) / P;
   MfmaParams pa = p;
   pa.seg = 1;
@@ -1830,7 +1882,7 @@ hipError_t mfma_fwd(const Dims& d, int y_dtype, const void* q, const void* k, co
 }
 
 size_t mfma_fwd_norm_workspace(const Dims& d) {
-  return tiles_workspace(d) + seg_bytes(d, norm_seg_parts(d)) + norm_exchange_bytes(d);
+  return tiles_workspace(d) + seg_bytes(d, lone_seg_parts(d)) + norm_exchange_bytes(d);
 }
 
 hipError_t mfma_fwd_norm(const Dims& d, int y_dtype, const void* q, const void* k, const void* v,
@@ -1842,7 +1894,7 @@ hipError_t mfma_fwd_norm(const Dims& d, int y_dtype, const void* q, const void* 
   p.ng_stride = nm.gate_stride;
   p.nw = nm.weight;
   p.neps = nm.eps;
-  const int P = norm_seg_parts(d);
+  const int P = lone_seg_parts(d);
   p.nx = reinterpret_cast<unsigned long long*>(static_cast<char*>(ws) + tiles_workspace(d) +
                                                seg_bytes(d, P));
   p.nfault = nm.fault;
@@ -1858,26 +1910,12 @@ hipError_t mfma_fwd_norm(const Dims& d, int y_dtype, const void* q, const void* 
   if (e != hipSuccess) return e;
   if (P == 1) return launch_scan_norm(p, d, y_dtype == DN_BF16, stream);
   carve_seg(p, d, P, static_cast<char*>(ws) + tiles_workspace(d));
+  p.seg_p = P;
   const Dims ds = seg_dims(d, P);
-  MfmaParams pa = p;
-  pa.B = ds.B;
-  pa.S = ds.S;
-  pa.N = ds.N;
-  pa.seg = 1;
-  pa.seg_p = P;
-  pa.vx = d.V + d.K;
-  pa.y = nullptr;
+  const MfmaParams pa = lone_segs(p, d, ds);
   if ((e = launch_scan<false>(pa, ds, y_dtype == DN_BF16, stream)) != hipSuccess) return e;
-  MfmaParams pb = p;
-  pb.seg_p = P;
-  if ((e = launch_carry(pb, d, stream)) != hipSuccess) return e;
-  MfmaParams pc = pa;
-  pc.seg = 2;
-  pc.vx = d.V;
-  pc.s_in = p.seg_start;
-  pc.y = y;
-  pc.seg_final = state_out;
-  return launch_scan_norm(pc, ds, y_dtype == DN_BF16, stream);
+  if ((e = launch_carry(p, d, stream)) != hipSuccess) return e;
+  return launch_scan_norm(lone_outputs(pa, p), ds, y_dtype == DN_BF16, stream);
 }
 
 MfmaTiles mfma_bwd_tiles(const Dims& d, void* ws) {

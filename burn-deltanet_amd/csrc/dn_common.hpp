@@ -132,12 +132,9 @@ bool mfma_bwd_supported(const Dims& d, int qkv_dtype);
 // The MFMA forward: the intra kernel and the scan as two launches with their
 // tiles in the workspace, or with `fused` (where fused_fwd_supported holds)
 // the one kernel of chunk_fwd_fused.hip. mfma_fwd plans by the `ws_bytes` it
-// is given, which need not be what mfma_fwd_workspace says for its arguments
-// (a caller may hold another entry point's workspace, or a smaller one, down
-// to mfma_fwd_least_workspace): it cuts the sequences into no more segments
-// than fit there.
-size_t mfma_fwd_workspace(const Dims& d, bool fused = false);
-size_t mfma_fwd_least_workspace(const Dims& d, bool fused);
+// is given: it cuts the sequences into no more segments than fit there.
+// mfma_fwd_workspace: what it uses of `room` bytes, or needs where that is more.
+size_t mfma_fwd_workspace(const Dims& d, bool fused, size_t room);
 // The projection front-end's q/k formed in the intra kernel's load stage
 // (dn_frontend_chunk_fwd): the raw projection columns, the conv of length 4
 // with its window and SiLU (the reference's default activations), the L2

@@ -448,26 +448,24 @@ int dn_unit_lower_inverse(const dn_tri_args *args, hipStream_t stream);
  * the call pass their own workspace of at least these many bytes. For a
  * forward on the MFMA path over few long sequences, they include the buffers
  * of the segments that it cuts those into for speed. Such a call is also served
- * from a smaller workspace, with the segments that fit there: one that holds
- * its tiles and, at head_k_dim 128 with head_v_dim a multiple of 128, segments
- * for one 128-column workgroup per CU. A caller's workspace starts at a 16-byte
- * boundary, where the call runs DN_ALGO_GENERIC at a 4-byte one. */
+ * from a smaller workspace, as long as that holds its tiles, with the segments
+ * that fit there. A caller's workspace starts at a 16-byte boundary, where the
+ * call runs DN_ALGO_GENERIC at a 4-byte one. */
 size_t dn_chunk_fwd_workspace_bytes(const dn_chunk_fwd_args *args);
 size_t dn_chunk_bwd_workspace_bytes(const dn_chunk_bwd_args *args);
 
 /* dn_chunk_fwd for callers that cannot allocate: code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc. No counterpart in the
  * reference, whose Burn backend allocates every tensor. It takes the same
- * arguments and gives the same results as dn_chunk_fwd, but ignores
- * `workspace` and runs on a fixed scratch array of DN_NOALLOC_SCRATCH_BYTES
- * that the library holds on each device it runs on until the process ends
- * (the array is part of the loaded code object). It calls no hipMalloc,
- * hipFree or other allocating routine. Limits:
- *   - arguments whose dn_chunk_fwd_workspace_bytes() exceeds
- *     DN_NOALLOC_SCRATCH_BYTES return DN_ERR_WORKSPACE (the MFMA path needs
- *     24.25 KiB per (batch, head, chunk of 64 tokens) with per-head gates,
- *     so 64 MiB covers 2700 of them, e.g. batch 1 x 16 heads x 10,700
- *     tokens);
+ * arguments as dn_chunk_fwd, ignores `workspace` and gives the results of
+ * dn_chunk_fwd from one of DN_NOALLOC_SCRATCH_BYTES: it runs on a fixed scratch
+ * array of that size, which the library holds on each device it runs on until
+ * the process ends (the array is part of the loaded code object). It calls no
+ * hipMalloc, hipFree or other allocating routine. Limits:
+ *   - arguments that a workspace of that size does not serve return
+ *     DN_ERR_WORKSPACE (the MFMA path needs 24.25 KiB per (batch, head, chunk
+ *     of 64 tokens) with per-head gates, so 64 MiB covers 2700 of them, e.g.
+ *     batch 1 x 16 heads x 10,700 tokens);
  *   - check_finite is refused (DN_ERR_UNSUPPORTED): the guard allocates its
  *     flag and synchronises;
  *   - every call on one device shares that device's array, so calls that

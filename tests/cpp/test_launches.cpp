@@ -181,7 +181,8 @@ void smaller_workspaces() {
     int S, K, V;
     size_t bytes;
   } cases[] = {{4096, 64, 128, 1589760}, {4096, 128, 576, 1591552}, {8192, 128, 192, 3179264},
-               {16384, 64, 576, 6359296}, {2048, 64, 64, 794880}};
+               {16384, 64, 576, 6359296}, {2048, 64, 64, 794880},
+               {8192, 128, 256, 3179520}};
   for (const auto& c : cases) {
     dn_chunk_fwd_args a = forward(1, c.S, 1, c.K, c.V, false);
     if (dn_chunk_fwd_workspace_bytes(&a) <= c.bytes) fail("smaller workspace: not smaller");
@@ -197,6 +198,36 @@ void smaller_workspaces() {
     if (dn_chunk_fwd(&a, nullptr) != DN_ERR_WORKSPACE) fail("smaller workspace: accepted");
   }
   std::printf("ok smaller_workspaces\n");
+}
+
+// Which kernels walk the segments: teams where a round of the device holds
+// them, 8-wave workgroups where it does not, or the sequence whole.
+void segment_kernels() {
+  static int teams, lone, carries;
+  on_launch = [](const Launch& l) {
+    teams += l.kernel.find("team_scan_kernel") != std::string::npos;
+    lone += l.kernel.find("mfma_scan_kernel") != std::string::npos;
+    carries += l.kernel.find("seg_carry_kernel") != std::string::npos;
+  };
+  const struct {
+    int S, H, V;
+    bool channel;
+    int teams, lone, carries;
+  } cases[] = {{12288, 4, 256, false, 2, 0, 1}, {16384, 8, 256, false, 0, 2, 1},
+               {16384, 8, 256, true, 0, 2, 1},  {16384, 4, 256, true, 2, 0, 1},
+               {16384, 16, 128, false, 0, 2, 1}, {16384, 6, 192, false, 2, 0, 1},
+               {16352, 8, 256, false, 1, 0, 0}, {2048, 16, 256, false, 1, 0, 0}};
+  for (const auto& c : cases) {
+    dn_chunk_fwd_args a = forward(1, c.S, c.H, 128, c.V, c.channel);
+    a.workspace_bytes = dn_chunk_fwd_workspace_bytes(&a);
+    teams = lone = carries = 0;
+    if (dn_chunk_fwd(&a, nullptr) != DN_OK) fail(dn_last_error());
+    if (teams != c.teams || lone != c.lone || carries != c.carries)
+      fail("segment kernels of S " + std::to_string(c.S) + " H " + std::to_string(c.H) + " V " +
+           std::to_string(c.V) + ": teams " + std::to_string(teams) + " lone " +
+           std::to_string(lone) + " carries " + std::to_string(carries));
+  }
+  std::printf("ok segment_kernels\n");
 }
 
 // dn_chunk_bwd where its launches fail one by one: what it left on the second
@@ -248,6 +279,7 @@ void backward_joins() {
 int main() {
   out_norm_fallback();
   smaller_workspaces();
+  segment_kernels();
   backward_joins();
   std::printf("all passed\n");
   return 0;

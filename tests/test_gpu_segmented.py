@@ -62,6 +62,8 @@ CASES = [
     (1, 2048, 1, 128, 256, "head", 0.0),       # P = 2, two 128-column tiles
     (2, 4096, 1, 128, 128, None, 0.02),        # P = 4, ungated
     (1, 4096, 1, 128, 128, "channel", 0.5),    # P = 4, a large initial state
+    (1, 8192, 12, 128, 128, "head", 0.02),     # P = 8, by eight-wave workgroups
+    (1, 8192, 16, 128, 128, "channel", 0.02),  # P = 8, by eight-wave workgroups
 ]
 
 

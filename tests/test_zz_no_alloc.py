@@ -77,6 +77,23 @@ def test_noalloc_forward_equals_dn_chunk_fwd_on_two_calls_in_a_row(case, fused):
         assert torch.equal(ref[0], got[0]) and torch.equal(ref[1], got[1])
 
 
+def test_noalloc_keeps_to_its_scratch():
+    """A call that dn_chunk_fwd would cut into more segments than the scratch
+    holds: the results of dn_chunk_fwd from a workspace of the scratch's size."""
+    announce("dn_chunk_fwd_noalloc: fewer segments than dn_chunk_fwd")
+    args = inputs(44, 1, 16384, 8, 128, 256, torch.bfloat16)
+    out = []
+    for run in (abi.run_chunk_fwd, abi.run_chunk_fwd_noalloc):
+        y, s1 = torch.empty_like(args[2]), torch.empty_like(args[6])
+        a = abi.chunk_fwd_args(*args, y, s1, 64, None)
+        assert abi.lib().dn_chunk_fwd_workspace_bytes(a) > abi.NOALLOC_SCRATCH_BYTES
+        ws = torch.empty(abi.NOALLOC_SCRATCH_BYTES, dtype=torch.uint8, device=DEV)
+        a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+        run(a)
+        out.append((y, s1))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
 def test_noalloc_refuses_arguments_above_its_scratch():
     announce("dn_chunk_fwd_noalloc: too large for the scratch array")
     # BASELINE config 5 (GDN-2 per-channel gates): 737 MB of workspace.
