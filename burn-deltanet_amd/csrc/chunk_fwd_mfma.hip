@@ -1428,10 +1428,12 @@ inline float chunk_us(const Dims& d, ScanShape s) {
          : s.waves == 4 ? (pc ? 2.6f : 2.55f)
                         : (pc ? 3.8f : 2.65f);
 }
+inline size_t scan_wgs(const Dims& d, int columns, int copies) {
+  return size_t(d.B) * d.H * ((d.V + columns - 1) / columns) * copies;
+}
 inline size_t scan_rounds(const Dims& d, int columns, int copies) {
-  const size_t wgs = size_t(d.B) * d.H * ((d.V + columns - 1) / columns) * copies;
   const size_t cus = size_t(device_cu_count());
-  return (wgs + cus - 1) / cus;
+  return (scan_wgs(d, columns, copies) + cus - 1) / cus;
 }
 
 // The shape whose rounds cost least. In the backward at head_k_dim 128 the
@@ -1440,7 +1442,14 @@ inline size_t scan_rounds(const Dims& d, int columns, int copies) {
 // (backward) at 16 chunks, the narrowest of 2, 4 and 8 lone waves that fills
 // the device -> this choice: forward dv 256, 16 heads 3.3 -> 1.7, 32 heads
 // 3.2 -> 2.1, 48 heads 6.05 -> 3.7, 96 heads 7.1 -> 4.3; per channel, dv 256,
-// 16 heads 3.5 -> 1.85. Backward dv 256, 16 heads 171 -> 144, 48 heads
+// 16 heads 3.5 -> 1.85. At head_k_dim 64 two workgroups of teams fit a CU (63 and
+// 76 KB of LDS with y) and share its time, so the count of rounds holds in the
+// choices it decides but one: two teams in three rounds or 4 lone waves in two
+// (`shared`, in the forward past 2.5 rounds). S=2048, us a call, teams and lone
+// waves: backward, dv 64, 350 heads 1521 and 1450, dv 192, 96 heads 757 and 721,
+// 128 heads 982 and 882; forward, dv 192, 86 heads 157 and 181, 96 heads 179 and
+// 186, 128 heads, per channel 298 and 285, dv 64, 260 heads 265 and 257 (S=1024
+// 116 and 125), 350 heads 296 and 285. Backward dv 256, 16 heads 171 -> 144, 48 heads
 // 452 -> 382; per channel, dv 128, 32 heads 221 -> 199.
 ScanShape scan_shape(const Dims& d, bool backward) {
   // head_k_dim 256: eight waves, whose staging registers (11 per lane) fit
@@ -1453,7 +1462,10 @@ ScanShape scan_shape(const Dims& d, bool backward) {
   for (const ScanShape& s : shapes) {
     const int columns = s.teams ? 16 * s.teams : 16 * s.waves;
     if (!s.teams && d.V % columns != 0) continue;
-    const float cost = chunk_us(d, s) * float(scan_rounds(d, columns, copies));
+    const size_t rounds = scan_rounds(d, columns, copies);
+    const bool late = 2 * scan_wgs(d, columns, 1) > 5 * size_t(device_cu_count());
+    const float shared = d.K == 64 && s.teams && rounds > 2 && (backward || late) ? 1.1f : 1.f;
+    const float cost = chunk_us(d, s) * shared * float(rounds);
     if (least == 0.f || cost < least) {
       best = s;
       least = cost;

@@ -23,6 +23,7 @@ namespace {
 struct Launch {
   std::string kernel;
   const void* params;  // valid until the next launch
+  int threads;
 };
 
 std::map<const void*, std::string>& kernels() {
@@ -44,10 +45,10 @@ void fail(const std::string& what) {
   std::exit(1);
 }
 
-hipError_t record(const void* f, void** args) {
+hipError_t record(const void* f, dim3 block, void** args) {
   const auto it = kernels().find(f);
   if (it == kernels().end()) fail("launch of an unregistered kernel");
-  if (on_launch) on_launch({it->second, args[0]});
+  if (on_launch) on_launch({it->second, args[0], int(block.x)});
   ++launches;
   return hipSuccess;
 }
@@ -65,14 +66,21 @@ void __hipRegisterFunction(void**, const void* host, char*, const char* name, un
   kernels()[host] = name;
 }
 void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
-hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
-hipError_t __hipPopCallConfiguration(dim3*, dim3*, size_t*, hipStream_t*) { return hipSuccess; }
-hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t) {
-  return record(f, args);
+static dim3 pushed;  // the block of the launch under way
+hipError_t __hipPushCallConfiguration(dim3, dim3 block, size_t, hipStream_t) {
+  pushed = block;
+  return hipSuccess;
 }
-hipError_t hipLaunchCooperativeKernel(const void* f, dim3, dim3, void** args, unsigned,
+hipError_t __hipPopCallConfiguration(dim3*, dim3* block, size_t*, hipStream_t*) {
+  *block = pushed;
+  return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void* f, dim3, dim3 block, void** args, size_t, hipStream_t) {
+  return record(f, block, args);
+}
+hipError_t hipLaunchCooperativeKernel(const void* f, dim3, dim3 block, void** args, unsigned,
                                       hipStream_t) {
-  return record(f, args);
+  return record(f, block, args);
 }
 hipError_t hipGetLastError() {
   return failing && launches == failing ? hipErrorLaunchFailure : hipSuccess;
@@ -230,6 +238,34 @@ void segment_kernels() {
   std::printf("ok segment_kernels\n");
 }
 
+// The workgroups a whole scan is given, by how many of them the device holds:
+// threads of teams (4 waves a team and 4 that stage) or of lone waves.
+void scan_shapes() {
+  static int team_threads, lone_threads;
+  on_launch = [](const Launch& l) {
+    if (l.kernel.find("team_scan_kernel") != std::string::npos) team_threads = l.threads;
+    if (l.kernel.find("mfma_scan_kernel") != std::string::npos) lone_threads = l.threads;
+  };
+  const struct {
+    int H, K, V, teams, waves;
+  } cases[] = {{16, 128, 256, 1, 0}, {17, 128, 256, 2, 0}, {32, 128, 256, 2, 0}, {48, 128, 256, 0, 4},
+               {65, 128, 256, 0, 8}, {96, 128, 256, 0, 8}, {64, 64, 64, 1, 0},   {65, 64, 64, 2, 0},
+               {129, 64, 64, 0, 4},  {300, 64, 64, 2, 0},  {350, 64, 64, 0, 4},  {129, 64, 128, 0, 8}, {96, 64, 192, 2, 0},
+               {128, 64, 192, 0, 4},
+               {4, 256, 128, 0, 8}};
+  for (const auto& c : cases) {
+    dn_chunk_fwd_args a = forward(1, 100, c.H, c.K, c.V, false);
+    a.workspace_bytes = dn_chunk_fwd_workspace_bytes(&a);
+    team_threads = lone_threads = 0;
+    if (dn_chunk_fwd(&a, nullptr) != DN_OK) fail(dn_last_error());
+    if (team_threads != (c.teams ? 256 * c.teams + 256 : 0) || lone_threads != 64 * c.waves)
+      fail("scan shape of H " + std::to_string(c.H) + " K " + std::to_string(c.K) + " V " +
+           std::to_string(c.V) + ": team threads " + std::to_string(team_threads) +
+           ", lone threads " + std::to_string(lone_threads));
+  }
+  std::printf("ok scan_shapes\n");
+}
+
 // dn_chunk_bwd where its launches fail one by one: what it left on the second
 // stream is joined whenever it returns.
 void backward_joins() {
@@ -280,6 +316,7 @@ int main() {
   out_norm_fallback();
   smaller_workspaces();
   segment_kernels();
+  scan_shapes();
   backward_joins();
   std::printf("all passed\n");
   return 0;
