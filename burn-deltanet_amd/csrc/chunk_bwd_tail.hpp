@@ -97,7 +97,8 @@ __device__ void chunk_bwd_tail(const ChunkTail& x, const Rows& rows, float* lds,
     for (int r = 0; r < 4; ++r) {
       const int i = 16 * ti + 4 * g4 + r, j = 16 * tj + m16;
       const float m = PCG ? 1.f : expf(sG[i] - sG[j]);
-      lD[pr * kBlk + to[r]] = dtt[u][r];
+      // (What lies on and above the diagonal reaches no result but as 0 × it.)
+      lD[pr * kBlk + to[r]] = j < i ? dtt[u][r] : 0.f;
       rqk[pr * kBlk + to[r]] = j <= i ? dat[u][r] * m : 0.f;
     }
   }

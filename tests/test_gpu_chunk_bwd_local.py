@@ -66,3 +66,19 @@ def test_v_four_bytes_past_a_boundary(rng, K, V, gates):
     for a, b in zip(*[vars(pkg.combined_backward(dy, None, *x, 64, 1.0 / np.sqrt(K), algo=MFMA)).values()
                       for x in (args, off)]):
         assert (a is None and b is None) or torch.equal(a, b)
+
+
+@pytest.mark.parametrize("K,gates", [(128, "head"), (64, "channel"), (128, "channel")])
+def test_infinite_value_of_the_last_token(rng, K, gates):
+    """The erase gates before a token do not meet its value, whatever that is:
+    their gradients are those of a finite one, to the bit."""
+    announce(f"chunk-local backward: an infinite value K {K} {gates}")
+    S, V = 128, 64
+    args = to_gpu(random_raw(rng, 1, S, 2, K, V, channel=gates == "channel"), torch.bfloat16)
+    dy = torch.tensor(rng.standard_normal((1, S, 2, V)), device=args[0].device).bfloat16()
+    out = []
+    for value in (1.0, float("inf")):
+        args[2][:, -1, :, 3] = value
+        out.append(pkg.combined_backward(dy, None, *args, 64, 1.0 / np.sqrt(K),
+                                         algo=MFMA).d_erase_bshK[:, :-1])
+    assert bool(torch.isfinite(out[1]).all()) and torch.equal(*out)
