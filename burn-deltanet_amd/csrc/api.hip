@@ -324,9 +324,8 @@ Dims bwd_dims(const dn_chunk_bwd_args* a) {
                    a->scale);
 }
 
-// MFMA: the two scans of the backward on bf16 MFMA (the forward MFMA path's
-// shapes, bf16 q/k/v), and for head_v_dim 64 or 128 the chunk-local
-// gradients too; otherwise those stay on the generic fp32 kernel.
+// MFMA: the backward's scans and chunk-local gradients on bf16 MFMA, for the
+// forward MFMA path's shapes (mfma_bwd_supported) and bf16 q/k/v.
 // The backward's MFMA kernels also read d_y in 16-byte words.
 int bwd_algo(const dn_chunk_bwd_args* a, const Dims& d0) {
   if (a->algo == DN_ALGO_GENERIC) return DN_ALGO_GENERIC;
@@ -337,17 +336,13 @@ int bwd_algo(const dn_chunk_bwd_args* a, const Dims& d0) {
   return fits ? DN_ALGO_MFMA : DN_ALGO_GENERIC;
 }
 
-bool bwd_all_mfma(const Dims& d, int qkv_dtype, int algo) {
-  return algo == DN_ALGO_MFMA && mfma_chunk_bwd_supported(d, qkv_dtype);
-}
-
 // Per-chunk states and state cotangents, fp32 [G][K][V] each.
 size_t bwd_state_bytes(const Dims& d) {
   return align_up(size_t(d.B) * d.N * d.H * d.K * d.V * sizeof(float), 256);
 }
 
-size_t bwd_workspace(const Dims& d, int algo, int qkv_dtype) {
-  if (bwd_all_mfma(d, qkv_dtype, algo))
+size_t bwd_workspace(const Dims& d, int algo) {
+  if (algo == DN_ALGO_MFMA)
     return 2 * bwd_state_bytes(d) + align_up(mfma_bwd_workspace(d), 256) +
            mfma_chunk_bwd_partials(d);
   return align_up(generic_bwd_workspace(d), 256);
@@ -607,7 +602,7 @@ size_t dn_chunk_bwd_workspace_bytes(const dn_chunk_bwd_args* a) {
   if (check_bwd(a)) return 0;
   const Dims d = bwd_dims(a);
   const int algo = bwd_algo(a, d);
-  return algo < 0 ? 0 : bwd_workspace(run_dims(d, algo), algo, a->qkv_dtype);
+  return algo < 0 ? 0 : bwd_workspace(run_dims(d, algo), algo);
 }
 
 int dn_chunk_bwd(const dn_chunk_bwd_args* a, hipStream_t stream) {
@@ -620,7 +615,7 @@ int dn_chunk_bwd(const dn_chunk_bwd_args* a, hipStream_t stream) {
                                     "of 128), head_v_dim a multiple of 64, and chunk_len 64 "
                                     "with a per-channel forget gate");
   const Dims d = run_dims(bwd_dims(a), algo);
-  const size_t need = bwd_workspace(d, algo, a->qkv_dtype);
+  const size_t need = bwd_workspace(d, algo);
   void* ws = a->workspace;
   if (ws) {
     if (a->workspace_bytes < need)
@@ -645,14 +640,13 @@ int dn_chunk_bwd(const dn_chunk_bwd_args* a, hipStream_t stream) {
   }
   hipError_t e;
   const float* g = a->has_gate ? a->g : nullptr;
-  if (bwd_all_mfma(d, a->qkv_dtype, algo)) {
+  if (algo == DN_ALGO_MFMA) {
     char* base = static_cast<char*>(ws);
     float* states = reinterpret_cast<float*>(base);
     float* ds_after = reinterpret_cast<float*>(base + bwd_state_bytes(d));
     void* mws = base + 2 * bwd_state_bytes(d);
-    const bool g4 = states_g4(d);
     e = mfma_bwd_scans(d, a->grad_dtype, a->d_y, a->d_state_final, a->q, a->k, a->v, a->erase,
-                       a->write, g, a->state_in, states, ds_after, a->d_state, mws, stream, g4);
+                       a->write, g, a->state_in, states, ds_after, a->d_state, mws, stream);
     if (e == hipSuccess && local_bwd_takes(d))
       e = local_bwd(d, a->grad_dtype, a->d_y, a->q, a->k, a->v, a->erase, a->write, g, states,
                     ds_after, a->d_q, a->d_k, a->d_v, a->d_erase, a->d_write,
@@ -666,7 +660,7 @@ int dn_chunk_bwd(const dn_chunk_bwd_args* a, hipStream_t stream) {
               ? reinterpret_cast<float*>(static_cast<char*>(mws) +
                                          align_up(mfma_bwd_workspace(d), 256))
               : nullptr,
-          stream, g4);
+          stream);
   } else {
     e = generic_bwd(d, a->qkv_dtype, a->grad_dtype, a->d_y, a->d_state_final, a->q, a->k, a->v,
                     a->erase, a->write, g, a->state_in, a->d_q, a->d_k, a->d_v, a->d_erase,

@@ -57,9 +57,6 @@ struct LocalParams {
 __device__ inline int rows_slot(int m, int g) { return 16 * g + (m ^ (2 * g)); }
 __device__ inline int cols_slot(int m, int g) { return 16 * g + (m ^ (4 * g)); }
 
-// Steps of a triangular 64×64 tile's six nonzero 16×32 blocks.
-__device__ inline int upper_step(int tb, int kk) { return tb < 2 ? 2 * tb + kk : tb + 2; }
-
 // q and k of the chunk in LDS tiles ([64][K] of 16 × 32 blocks), which their
 // gradients replace where they are bf16; fp32 ones go to memory.
 template <int K, class TG>
@@ -186,8 +183,8 @@ __global__ __launch_bounds__(4 * K) void local_bwd_kernel(LocalParams p) {
     for (int i = 0; i < NS; ++i) {
       const int u = min(tid + NT * i, 5 * kTri6 - 1), which = u / kTri6, w = u % kTri6, st = w >> 6;
       const bool up = which >= 2;  // T, T lo below; Tᵀ, Tᵀ lo, attnᵀ above the diagonal
-      const int rb = up ? (st < 4 ? st >> 1 : st - 2) : tril_tb(st);
-      const int kk = up ? (st < 4 ? st & 1 : 1) : tril_kk(st);
+      const int rb = up ? triu_tb(st) : tril_tb(st);
+      const int kk = up ? triu_kk(st) : tril_kk(st);
       const uint16_t* x = which == 0   ? p.t.T
                           : which == 1 ? p.t.Tlo
                           : which == 2 ? p.t.Tt
@@ -333,7 +330,7 @@ __global__ __launch_bounds__(4 * K) void local_bwd_kernel(LocalParams p) {
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
         if (kk < (tb >> 1)) continue;
-        const bf16x8 af = frag(tA, upper_step(tb, kk));
+        const bf16x8 af = frag(tA, triu_step(tb, kk));
         ya = mfma16(trans(Yt, kk, ct, false), af, ya);
         if constexpr (kYlo) ya = mfma16(trans(Yt + 256, kk, ct, false), af, ya);
       }
@@ -364,7 +361,7 @@ __global__ __launch_bounds__(4 * K) void local_bwd_kernel(LocalParams p) {
           vb = mfma16(trans(Xt + 256, kk, ct, false), th, vb);
         }
         if (kk >= (tb >> 1)) {
-          const bf16x8 uh = frag(tU[0], upper_step(tb, kk)), ul = frag(tU[1], upper_step(tb, kk));
+          const bf16x8 uh = frag(tU[0], triu_step(tb, kk)), ul = frag(tU[1], triu_step(tb, kk));
           const bf16x8 dh = trans(Dt, kk, ct, false);
           za = mfma16(dh, uh, za);
           zb = mfma16(dh, ul, zb);
@@ -495,13 +492,6 @@ __global__ __launch_bounds__(4 * K) void local_bwd_kernel(LocalParams p) {
 }
 
 }  // namespace
-
-bool local_bwd_supported(const Dims& d) {
-  const bool pc = d.dw == d.K && d.K > 1;
-  return (d.K == 64 || d.K == 128) && d.V % 32 == 0 &&
-         (pc ? (d.ew == 1 || d.ew == d.K) && (d.ww == 1 || d.ww == d.V)
-             : d.dw <= 1 && d.ew == 1 && d.ww == 1);
-}
 
 hipError_t local_bwd(const Dims& d, int grad_dtype, const void* dy, const void* q, const void* k,
                      const void* v, const float* erase, const float* write, const float* g,

@@ -102,23 +102,6 @@ __device__ inline void split4(const float* f, uint2& h, uint2& l) {
                  pk_bf16(f[2] - lo_f(h.y), f[3] - hi_f(h.y)));
 }
 
-// v[0..15] summed over the 16 lanes that share lane/16; lane l receives the
-// total of index l%16 (a halving exchange: 15 shuffles instead of 64).
-__device__ inline float reduce16(const float (&v)[16], int lane) {
-  float a[8], b[4], c[2];
-  const bool u8 = lane & 8, u4 = lane & 4, u2 = lane & 2, u1 = lane & 1;
-#pragma unroll
-  for (int j = 0; j < 8; ++j)
-    a[j] = (u8 ? v[8 + j] : v[j]) + __shfl_xor(u8 ? v[j] : v[8 + j], 8);
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    b[j] = (u4 ? a[4 + j] : a[j]) + __shfl_xor(u4 ? a[j] : a[4 + j], 4);
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-    c[j] = (u2 ? b[2 + j] : b[j]) + __shfl_xor(u2 ? b[j] : b[2 + j], 2);
-  return (u1 ? c[1] : c[0]) + __shfl_xor(u1 ? c[0] : c[1], 1);
-}
-
 // A 64×64 bf16 tile (global, row-major) → LDS with the permuted column order:
 // thread tid loads 16-byte chunk tid (512 threads, one each), then stores it.
 __device__ inline uint4 load_perm(const uint16_t* src, int tid) {
@@ -154,7 +137,7 @@ __global__ __launch_bounds__(kNT) void mfma_chunk_bwd_kernel(CbParams p) {
   static_assert(KA == K || KA == 2 * K, "all keys, or one of their halves");
   constexpr int KS = KA;  // row stride of q, k, the states and the key-channel outputs
   // The states and state cotangents in row groups of four, [G][K/4][V][4]
-  // (mfma_bwd_scans' g4, at head_k_dim 256), else [G][K][V].
+  // at head_k_dim 256 (mfma_bwd_scans), else [G][K][V].
   constexpr bool G4 = KA == 256;
   static_assert(!(EARLY && LASTP), "partial score sums: not the last pass");
   constexpr bool F32DY = std::is_same<TG, float>::value;
@@ -210,7 +193,7 @@ __global__ __launch_bounds__(kNT) void mfma_chunk_bwd_kernel(CbParams p) {
   const TG* dy = static_cast<const TG*>(p.dy);
   const bool gated = p.gated;
   auto rowi = [&](int ib, int r) { return 16 * ib + 4 * g4 + r; };
-  // Row of the value reduce16 leaves in this lane (index 4·ib + r).
+  // Row of the value sum16 leaves in this lane (index 4·ib + r).
   const int red_row = 16 * (r16 >> 2) + 4 * g4 + (r16 & 3);
 
   // ---- staging -----------------------------------------------------------
@@ -443,7 +426,7 @@ __global__ __launch_bounds__(kNT) void mfma_chunk_bwd_kernel(CbParams p) {
         if (store_a && i < valid) st(gv, row_of(i) * VS + vo + col, dW[ib][r] * wv[ib][r]);
         rs[4 * ib + r] = dW[ib][r] * vv[ib][r];
       }
-    atomicAdd(&racc[0][red_row], reduce16(rs, lane));
+    atomicAdd(&racc[0][red_row], sum16(rs, lane));
   }
   // dY rows for LDS, then phase B's global operands: S₀ and dS rows of this
   // lane's key channel.
@@ -832,7 +815,7 @@ __global__ __launch_bounds__(kNT) void mfma_chunk_bwd_kernel(CbParams p) {
           rowv[4 * ib + r] = val;
         }
       }
-      atomicAdd(&racc[2][red_row], reduce16(rowv, lane));
+      atomicAdd(&racc[2][red_row], sum16(rowv, lane));
       // d(G_last) of the whole head: Σ d_carry + Σ_channels (dS⊙S₀)·e^{G_last}.
       float tot = carry + (g4 == 0 ? degl * eg_s[kL - 1] : 0.f);
 #pragma unroll
@@ -890,7 +873,7 @@ __global__ __launch_bounds__(kNT) void mfma_chunk_bwd_kernel(CbParams p) {
                              kv[r] * (SK2[ib][r] + SQ2[ib][r]);
         }
       }
-      if (gated) atomicAdd(&racc[2][red_row], reduce16(rowv, lane));
+      if (gated) atomicAdd(&racc[2][red_row], sum16(rowv, lane));
     }
     // Front end (combined_backward.rs:153-188) and the stores.
     float rde[16];
@@ -916,7 +899,7 @@ __global__ __launch_bounds__(kNT) void mfma_chunk_bwd_kernel(CbParams p) {
         rde[4 * ib + r] = dkeA[ib][r] * kv[r];
       }
     }
-    atomicAdd(&racc[1][red_row], reduce16(rde, lane));
+    atomicAdd(&racc[1][red_row], sum16(rde, lane));
   }
   __syncthreads();
   if (gated && wave == 0) {
@@ -951,11 +934,7 @@ static bool own_shape(const Dims& d) {
   return d.dw <= 1 && d.ew == 1 && d.ww == 1 && (d.K == 256 || (d.K == 64 && d.V <= 128));
 }
 
-bool mfma_chunk_bwd_supported(const Dims& d, int qkv_dtype) {
-  return mfma_fwd_supported(d, qkv_dtype, DN_BF16) && (own_shape(d) || local_bwd_supported(d));
-}
-
-bool local_bwd_takes(const Dims& d) { return local_bwd_supported(d) && !own_shape(d); }
+bool local_bwd_takes(const Dims& d) { return !own_shape(d); }
 
 // The fp32 partial sums of the value-summed gradients across head_k_dim 256's
 // launches: per (token, head) d_q, d_k (K each), d_erase, d_g and d_write,
@@ -971,9 +950,8 @@ hipError_t mfma_chunk_bwd(const Dims& d, int grad_dtype, const void* dy, const v
                           const void* k, const void* v, const float* erase, const float* write,
                           const float* g, const float* states, const float* ds_after, void* dq,
                           void* dk, void* dv, float* derase, float* dwrite, float* dg,
-                          const MfmaTiles& tiles, float* partials, hipStream_t stream, bool g4) {
+                          const MfmaTiles& tiles, float* partials, hipStream_t stream) {
   // The chunk-local kernels read the row-group layout exactly at head_k_dim 256.
-  if (g4 != (d.K == 256)) return hipErrorInvalidValue;
   CbParams p;
   p.S = d.S;
   p.H = d.H;

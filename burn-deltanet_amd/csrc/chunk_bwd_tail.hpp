@@ -18,23 +18,6 @@ struct ChunkTail {
   float *derase, *dg;
 };
 
-// v[0..15] summed over the 16 lanes that share lane/16; lane l receives the
-// total of index l%16 (a halving exchange: 15 shuffles instead of 64).
-__device__ inline float sum16(const float (&v)[16], int lane) {
-  float a[8], b[4], c[2];
-  const bool u8 = lane & 8, u4 = lane & 4, u2 = lane & 2, u1 = lane & 1;
-#pragma unroll
-  for (int j = 0; j < 8; ++j)
-    a[j] = (u8 ? v[8 + j] : v[j]) + __shfl_xor(u8 ? v[j] : v[8 + j], 8);
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    b[j] = (u4 ? a[4 + j] : a[j]) + __shfl_xor(u4 ? a[j] : a[4 + j], 4);
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-    c[j] = (u2 ? b[2 + j] : b[j]) + __shfl_xor(u2 ? b[j] : b[2 + j], 2);
-  return (u1 ? c[1] : c[0]) + __shfl_xor(u1 ? c[0] : c[1], 1);
-}
-
 // q, k and their gradients straight from and to memory, an element at a time.
 template <class TQ, class TG>
 struct DirectRows {

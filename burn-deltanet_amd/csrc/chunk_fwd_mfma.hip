@@ -969,8 +969,8 @@ __global__ __launch_bounds__(256) void seg_carry_kernel(MfmaParams p) {
 // once in double-buffered LDS with the same k-permutation (head_k_dim 256:
 // 120 KB a chunk, single-buffered between two barriers). dS is read as bf16
 // hi + lo parts, dV' likewise for Tᵀ·dV'.
-// G4: ds_after in row groups of four ([G][K/4][V][4], states_g4).
-template <int K, class TG, int WAVES, bool G4 = false>
+// head_k_dim 256: ds_after in row groups of four ([G][K/4][V][4], mfma_bwd_scans).
+template <int K, class TG, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void mfma_rev_scan_kernel(RevParams p) {
   constexpr int KK = K / 32;
   constexpr int RBK = K / 16;
@@ -1110,7 +1110,7 @@ __global__ __launch_bounds__(64 * WAVES) void mfma_rev_scan_kernel(RevParams p) 
     const int cur = NBUF == 1 ? 0 : (it & 1);
     const int nn = n > 0 ? n - 1 : n;  // the first chunk prefetches itself again
     const uint16_t* tl = tiles[cur];
-    if constexpr (G4) {
+    if constexpr (K == 256) {
       float4* dst = reinterpret_cast<float4*>(p.ds_after + chunk_of(n) * K * p.V) + jl;
 #pragma unroll
       for (int rb = 0; rb < RBK; ++rb)
@@ -1632,10 +1632,8 @@ MfmaParams lone_outputs(const MfmaParams& segs, const MfmaParams& p) {
   return a;
 }
 
-// g4 (ST): write the states in row groups of four (states_g4).
 template <bool ST>
-hipError_t launch_scan(const MfmaParams& p, const Dims& d, bool yb, hipStream_t stream,
-                       bool g4 = false) {
+hipError_t launch_scan(const MfmaParams& p, const Dims& d, bool yb, hipStream_t stream) {
   const bool pc = pc_path(d);
   if constexpr (!ST) {
     if (p.seg) {
@@ -1667,7 +1665,7 @@ hipError_t launch_scan(const MfmaParams& p, const Dims& d, bool yb, hipStream_t 
   ProfScope ps(ST ? (pc ? "dn_mfma_scan_pc_states" : "dn_mfma_scan_states")
                   : (pc ? "dn_mfma_scan_pc" : "dn_mfma_scan"),
                stream);
-  if (shape.teams && !g4) return launch_team_scan(p, d.K, pc, ST, yb, shape.teams, stream);
+  if (shape.teams) return launch_team_scan(p, d.K, pc, ST, yb, shape.teams, stream);
   const int waves = shape.waves;
   const unsigned blocks = unsigned(((d.B * d.H + 7) / 8) * 8 * (d.V / (16 * waves)));
 #define DN_SCAN(KD, TY, W)                                                                        \
@@ -1681,20 +1679,6 @@ hipError_t launch_scan(const MfmaParams& p, const Dims& d, bool yb, hipStream_t 
   } while (0)
 #define DN_SCAN_W(KD, TY) \
   do { if (waves == 8) DN_SCAN(KD, TY, 8); else DN_SCAN(KD, TY, 4); } while (0)
-  if constexpr (ST) {
-    if (g4) {
-      // Eight-wave workgroups (head_k_dim 64, 128, 256).
-      if (waves != 8 || (pc && d.K == 256)) return hipErrorInvalidValue;
-#define DN_SCAN_G4(KD, PCV)                                                                    \
-  hipLaunchKernelGGL((mfma_scan_kernel<KD, float, 8, PCV, true, 0, 0, true>), dim3(blocks),     \
-                     dim3(512), 0, stream, p)
-      if (d.K == 256) DN_SCAN_G4(256, false);
-      else if (d.K == 128) { if (pc) DN_SCAN_G4(128, true); else DN_SCAN_G4(128, false); }
-      else { if (pc) DN_SCAN_G4(64, true); else DN_SCAN_G4(64, false); }
-#undef DN_SCAN_G4
-      return hipGetLastError();
-    }
-  }
   if (d.K == 256) {
     // head_k_dim 256: per-head gates, eight-wave workgroups.
     if (pc || waves != 8) return hipErrorInvalidValue;
@@ -1719,48 +1703,26 @@ hipError_t launch_scan(const MfmaParams& p, const Dims& d, bool yb, hipStream_t 
   return hipGetLastError();
 }
 
-hipError_t launch_rev(const RevParams& p, const Dims& d, int grad_dtype, hipStream_t stream,
-                      bool g4) {
-  // head_k_dim 256: eight waves with ds_after in row groups of four (the
-  // generic kernels' row-major layout: four, whose single wave per SIMD has
-  // the register file for 256 dS rows beside the next chunk's 120 KB of
-  // tiles; eight waves spilled there). At B=8 T=4096 H=16 dv=256: eight
-  // waves row-major 5.05 ms, four 3.85, four in row groups 1.61, eight in
-  // row groups 1.36.
+hipError_t launch_rev(const RevParams& p, const Dims& d, int grad_dtype, hipStream_t stream) {
+  // head_k_dim 256 in eight waves (B=8 T=4096 H=16 dv=256, with ds_after in row
+  // groups of four: four waves 1.61 ms, eight 1.36).
   const ScanShape shape = scan_shape(d, true);
-  const int waves = d.K == 256 && !g4 ? 4 : shape.waves;
   ProfScope ps("dn_mfma_rev_scan", stream);
-  if (shape.teams)
-    return g4 ? hipErrorInvalidValue
-              : launch_team_rev(p, d.K, grad_dtype == DN_BF16, shape.teams, stream);
-  const unsigned blocks = unsigned(((d.B * d.H + 7) / 8) * 8 * (d.V / (16 * waves)));
-#define DN_REV(KD, TG, W) \
-  hipLaunchKernelGGL((mfma_rev_scan_kernel<KD, TG, W>), dim3(blocks), dim3(64 * W), 0, stream, p)
-#define DN_REV4(KD, TG, W)                                                                     \
-  hipLaunchKernelGGL((mfma_rev_scan_kernel<KD, TG, W, true>), dim3(blocks), dim3(64 * W), 0,  \
-                     stream, p)
-#define DN_REV_W(KD, TG) \
-  do { if (waves == 8) DN_REV(KD, TG, 8); else DN_REV(KD, TG, 4); } while (0)
-  if (g4 && waves != 8 && d.K != 256) return hipErrorInvalidValue;
-  if (d.K == 256) {
-    if (g4) {
-      if (grad_dtype == DN_BF16) DN_REV4(256, bf16, 8); else DN_REV4(256, float, 8);
-    } else {
-      if (grad_dtype == DN_BF16) DN_REV(256, bf16, 4); else DN_REV(256, float, 4);
-    }
-  } else if (g4) {
-    if (d.K == 128) {
-      if (grad_dtype == DN_BF16) DN_REV4(128, bf16, 8); else DN_REV4(128, float, 8);
-    } else {
-      if (grad_dtype == DN_BF16) DN_REV4(64, bf16, 8); else DN_REV4(64, float, 8);
-    }
-  } else if (d.K == 128) {
-    if (grad_dtype == DN_BF16) DN_REV_W(128, bf16); else DN_REV_W(128, float);
-  } else {
-    if (grad_dtype == DN_BF16) DN_REV_W(64, bf16); else DN_REV_W(64, float);
-  }
-#undef DN_REV_W
-#undef DN_REV4
+  const bool g16 = grad_dtype == DN_BF16;
+  if (shape.teams) return launch_team_rev(p, d.K, g16, shape.teams, stream);
+  const unsigned blocks = unsigned(((d.B * d.H + 7) / 8) * 8 * (d.V / (16 * shape.waves)));
+#define DN_REV(KD, W)                                                                       \
+  do {                                                                                      \
+    if (g16)                                                                                \
+      hipLaunchKernelGGL((mfma_rev_scan_kernel<KD, bf16, W>), dim3(blocks), dim3(64 * W),   \
+                         0, stream, p);                                                     \
+    else                                                                                    \
+      hipLaunchKernelGGL((mfma_rev_scan_kernel<KD, float, W>), dim3(blocks), dim3(64 * W),  \
+                         0, stream, p);                                                     \
+  } while (0)
+  if (d.K == 256) DN_REV(256, 8);
+  else if (d.K == 128) { if (shape.waves == 8) DN_REV(128, 8); else DN_REV(128, 4); }
+  else { if (shape.waves == 8) DN_REV(64, 8); else DN_REV(64, 4); }
 #undef DN_REV
   return hipGetLastError();
 }
@@ -1944,13 +1906,11 @@ size_t mfma_bwd_workspace(const Dims& d) {
          region(size_t(d.B) * d.H * K * d.V * 4);  // the recompute's final state (unused)
 }
 
-bool states_g4(const Dims& d) { return d.K == 256; }
-
 hipError_t mfma_bwd_scans(const Dims& d, int grad_dtype, const void* dy,
                           const float* dstate_final, const void* q, const void* k, const void* v,
                           const float* erase, const float* write, const float* g,
                           const float* state_in, float* states, float* ds_after, float* dstate,
-                          void* ws, hipStream_t stream, bool g4) {
+                          void* ws, hipStream_t stream) {
   const size_t G = size_t(d.B) * d.N * d.H, K = size_t(d.K);
   // The forward recompute (states mode) and the reverse scan need nothing
   // from each other: after the intra kernel, the reverse scan and its tiles
@@ -1969,8 +1929,8 @@ hipError_t mfma_bwd_scans(const Dims& d, int grad_dtype, const void* dy,
   if (e != hipSuccess) return e;
   const RevParams rp{d.B, d.S, d.H, d.V, d.N, dy, dstate_final, ds_after, dstate, bt};
   return side_by_side(
-      stream, [&](hipStream_t side) { return launch_rev(rp, d, grad_dtype, side, g4); },
-      [&] { return launch_scan<true>(p, d, false, stream, g4); });
+      stream, [&](hipStream_t side) { return launch_rev(rp, d, grad_dtype, side); },
+      [&] { return launch_scan<true>(p, d, false, stream); });
 }
 
 }  // namespace dn

@@ -6,7 +6,7 @@ namespace dn {
 
 hipError_t launch_team_scan(const MfmaParams& p, int K, bool pc, bool states, bool yb, int teams,
                             hipStream_t stream) {
-  const int vb = (p.seg == 1 ? p.V + K : p.V) / 16, ntile = (vb + teams - 1) / teams;
+  const int ntile = (p.seg == 1 ? p.V + K : p.V) / (16 * teams);  // V and K: multiples of 64
   const int seqs = p.B * (p.seg ? p.seg_p : 1) * p.H;
   const dim3 grid(unsigned(((seqs + 7) / 8) * 8 * ntile)), block(256 * teams + 256);
 #define DN_T(KD, TY, C, PCV, STV, SG) \
@@ -38,7 +38,7 @@ hipError_t launch_team_scan(const MfmaParams& p, int K, bool pc, bool states, bo
 
 hipError_t launch_team_rev(const RevParams& p, int K, bool grad_bf16, int teams,
                            hipStream_t stream) {
-  const int ntile = (p.V / 16 + teams - 1) / teams;
+  const int ntile = p.V / (16 * teams);
   const dim3 grid(unsigned(((p.B * p.H + 7) / 8) * 8 * ntile)), block(256 * teams + 256);
 #define DN_R(KD, C)                                                                       \
   do {                                                                                    \

@@ -185,20 +185,18 @@ hipError_t fused_fwd(const Dims& d, int y_dtype, const void* q, const void* k, c
                      hipStream_t stream);
 // The backward's two scans on MFMA (bf16 q/k/v, the shapes mfma_fwd_supported
 // accepts): the states entering each chunk and the state cotangents leaving
-// each chunk, fp32 [G][K][V], plus the initial state's cotangent. g4: both
-// per-chunk arrays in row groups of four instead, [G][K/4][V][4] (a lane's
-// four accumulator rows of its column are one 16-byte store), which the
-// MFMA chunk-local kernel reads; where states_g4(d) holds, at head_k_dim
-// 256 (B=8 T=4096 H=16 dv=256: states scan 2543 → 692 µs, reverse scan
-// 3846 → 1623 µs, the chunk-local kernel 5.29 → 5.95 ms, whose key-channel
-// phase reads a row as 16-byte-strided words there).
+// each chunk, fp32 [G][K][V], plus the initial state's cotangent. At head_k_dim
+// 256 both per-chunk arrays in row groups of four instead, [G][K/4][V][4] (a
+// lane's four accumulator rows of its column are one 16-byte store; B=8 T=4096
+// H=16 dv=256: states scan 2543 → 692 µs, reverse scan 3846 → 1623 µs, the
+// chunk-local kernel 5.29 → 5.95 ms, whose key-channel phase reads a row as
+// 16-byte-strided words there).
 size_t mfma_bwd_workspace(const Dims& d);
-bool states_g4(const Dims& d);
 hipError_t mfma_bwd_scans(const Dims& d, int grad_dtype, const void* dy,
                           const float* dstate_final, const void* q, const void* k, const void* v,
                           const float* erase, const float* write, const float* g,
                           const float* state_in, float* states, float* ds_after, float* dstate,
-                          void* ws, hipStream_t stream, bool g4);
+                          void* ws, hipStream_t stream);
 // The per-chunk tiles mfma_bwd_scans leaves in its workspace: T (hi, lo) and
 // Tᵀ (hi, lo), attnᵀ [G][64][64]; kc = e^{G_last−G}⊙K [G][64][K]; per-channel
 // decay: kg = e⊙e^G⊙K hi, lo [G][64][K]; per-head: the cumulative gate [G][64].
@@ -207,27 +205,24 @@ struct MfmaTiles {
   const float* gc;
 };
 MfmaTiles mfma_bwd_tiles(const Dims& d, void* ws);
-// The chunk-local gradients at head_k_dim 64 and 128, after mfma_bwd_scans:
-// the shapes it has, and those among them that mfma_chunk_bwd does not keep.
-bool local_bwd_supported(const Dims& d);
+// The chunk-local gradients after mfma_bwd_scans at head_k_dim 64 and 128, in
+// the shapes that mfma_chunk_bwd does not keep.
 bool local_bwd_takes(const Dims& d);
 hipError_t local_bwd(const Dims& d, int grad_dtype, const void* dy, const void* q, const void* k,
                      const void* v, const float* erase, const float* write, const float* g,
                      const float* states, const float* ds_after, void* dq, void* dk, void* dv,
                      float* derase, float* dwrite, float* dg, const MfmaTiles& tiles,
                      hipStream_t stream);
-// The chunk-local gradients on MFMA, after mfma_bwd_scans: whether either
-// kernel has the call, and the one for per-head gates at head_k_dim 256 (in
-// passes of 128 value columns) or at 64 with head_v_dim 64 or 128.
-// `partials`: mfma_chunk_bwd_partials(d) bytes of workspace for the
+// The chunk-local gradients after mfma_bwd_scans for per-head gates at
+// head_k_dim 256 (in passes of 128 value columns) or at 64 with head_v_dim 64 or
+// 128. `partials`: mfma_chunk_bwd_partials(d) bytes of workspace for the
 // value-summed gradients between passes.
-bool mfma_chunk_bwd_supported(const Dims& d, int qkv_dtype);
 size_t mfma_chunk_bwd_partials(const Dims& d);
 hipError_t mfma_chunk_bwd(const Dims& d, int grad_dtype, const void* dy, const void* q,
                           const void* k, const void* v, const float* erase, const float* write,
                           const float* g, const float* states, const float* ds_after, void* dq,
                           void* dk, void* dv, float* derase, float* dwrite, float* dg,
-                          const MfmaTiles& tiles, float* partials, hipStream_t stream, bool g4);
+                          const MfmaTiles& tiles, float* partials, hipStream_t stream);
 
 // Per-kernel HIP-event timing (dn_profile_enable): a scope records a start
 // event on construction and a stop event on destruction, on `stream`.

@@ -51,12 +51,6 @@ __device__ inline uint2 pack4_lo(const f32x4& a, const uint2& h) {
                     pk_bf16(a[2] - lo_f(h.y), a[3] - hi_f(h.y)));
 }
 
-// The six nonzero 16×32 blocks of an upper-triangular 64×64 tile, in row
-// block order: row blocks 2 and 3 have no k-step 0.
-__host__ __device__ constexpr int triu_tb(int s) { return s < 4 ? s >> 1 : s - 2; }
-__host__ __device__ constexpr int triu_kk(int s) { return s < 4 ? s & 1 : 1; }
-__device__ inline int triu_step(int tb, int kk) { return tb < 2 ? 2 * tb + kk : tb + 2; }
-
 // Forward (ST = false) and states scan (ST). C teams per workgroup.
 // Tiles by the phase that last reads them, each staged for the next chunk as
 // soon as that phase's barrier has passed:
@@ -85,7 +79,7 @@ __global__ __launch_bounds__(256 * C + 256) void team_scan_kernel(MfmaParams p) 
   __shared__ __attribute__((aligned(16))) float ge[2][PC ? K : 1];       // e^{G_last}
 
   const int P = SEG ? p.seg_p : 1, VB = (SEG == 1 ? p.V + K : p.V) / 16;
-  const int ntile = (VB + C - 1) / C, BH = p.B * P * p.H;
+  const int ntile = VB / C, BH = p.B * P * p.H;
   const int group = blockIdx.x / (8 * ntile), within = blockIdx.x % (8 * ntile);
   const int tile = within / 8, bh = group * 8 + within % 8;
   if (bh >= BH) return;
@@ -254,9 +248,7 @@ __global__ __launch_bounds__(256 * C + 256) void team_scan_kernel(MfmaParams p) 
   // Odd teams take the token blocks in reverse: the triangular products of
   // the waves that share a SIMD then add up alike.
   const int tb = (team & 1) ? 3 - tw : tw;
-  // A last workgroup's spare team repeats the last column tile, unwritten.
-  const int ct = min(tile * C + team, VB - 1);
-  const bool live = tile * C + team < VB;
+  const int ct = tile * C + team;
   const int jl = 16 * ct + m16;
   // A transition column (SEG 1): column jl − V of the identity; the v it reads
   // weighs nothing.
@@ -309,12 +301,11 @@ __global__ __launch_bounds__(256 * C + 256) void team_scan_kernel(MfmaParams p) 
     const int cur = (n - n0) & 1, nn = min(n + 1, last);
     if constexpr (ST) {
       float* dst = p.states + chunk_of(n) * K * p.V + jl;
-      if (live)
 #pragma unroll
-        for (int i = 0; i < NR; ++i)
+      for (int i = 0; i < NR; ++i)
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            dst[size_t(16 * (tw + 4 * i) + 4 * g4 + r) * p.V] = S[i][r];
+        for (int r = 0; r < 4; ++r)
+          dst[size_t(16 * (tw + 4 * i) + 4 * g4 + r) * p.V] = S[i][r];
     }
     // Phase 1: X = w⊙v − (e⊙e^G)⊙(K·S) of this wave's tokens; yᵀ = Sᵀ·Qᵀ.
     f32x4 X = {0.f, 0.f, 0.f, 0.f}, X2 = X, yt = X;
@@ -433,7 +424,7 @@ __global__ __launch_bounds__(256 * C + 256) void team_scan_kernel(MfmaParams p) 
     if constexpr (kY) {
       TY* yb = static_cast<TY*>(p.y) + rows_of(n) * p.V;
       const int t = 16 * tb + m16;
-      if (live && t < p.S - n * kL) {
+      if (t < p.S - n * kL) {
         TY* dst = yb + uint32_t(t * HV + 16 * ct + 4 * g4);
         if constexpr (sizeof(TY) == 2)
           *reinterpret_cast<uint2*>(dst) = pack4(yt);
@@ -452,12 +443,11 @@ __global__ __launch_bounds__(256 * C + 256) void team_scan_kernel(MfmaParams p) 
     if (seg != P - 1) return;  // only the last segment's end state leaves the call
     out = p.seg_final + (size_t(b) * p.H + h) * K * p.V + jl;
   }
-  if (live)
 #pragma unroll
-    for (int i = 0; i < NR; ++i)
+  for (int i = 0; i < NR; ++i)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        out[size_t(16 * (tw + 4 * i) + 4 * g4 + r) * ld] = S[i][r];
+    for (int r = 0; r < 4; ++r)
+      out[size_t(16 * (tw + 4 * i) + 4 * g4 + r) * ld] = S[i][r];
 }
 
 // Reverse scan. ds_after in row-major [G][K][V]. Tiles as in the forward:
@@ -478,7 +468,7 @@ __global__ __launch_bounds__(256 * C + 256) void team_rev_kernel(RevParams p) {
   __shared__ uint4 Zx[C][128];         // −Z
   __shared__ __attribute__((aligned(16))) float ge[2][K];
 
-  const int ntile = (p.V / 16 + C - 1) / C, BH = p.B * p.H;
+  const int ntile = p.V / (16 * C), BH = p.B * p.H;
   const int group = blockIdx.x / (8 * ntile), within = blockIdx.x % (8 * ntile);
   const int tile = within / 8, bh = group * 8 + within % 8;
   if (bh >= BH) return;
@@ -583,8 +573,7 @@ __global__ __launch_bounds__(256 * C + 256) void team_rev_kernel(RevParams p) {
 
   const int team = wave >> 2, tw = wave & 3;
   const int tb = (team & 1) ? 3 - tw : tw;
-  const int ct = min(tile * C + team, p.V / 16 - 1);
-  const bool live = tile * C + team < p.V / 16;
+  const int ct = tile * C + team;
   const int jl = 16 * ct + m16;
   const int at4 = half_word(tb, lane), kmin = tb >> 1;
 
@@ -633,12 +622,11 @@ __global__ __launch_bounds__(256 * C + 256) void team_rev_kernel(RevParams p) {
   for (int it = 0; it < p.N; ++it) {
     const int n = p.N - 1 - it, cur = it & 1;
     float* dst = p.ds_after + chunk_of(n) * K * p.V + jl;
-    if (live)
 #pragma unroll
-      for (int i = 0; i < NR; ++i)
+    for (int i = 0; i < NR; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          dst[size_t(16 * (tw + 4 * i) + 4 * g4 + r) * p.V] = S[i][r];
+      for (int r = 0; r < 4; ++r)
+        dst[size_t(16 * (tw + 4 * i) + 4 * g4 + r) * p.V] = S[i][r];
     // Phase 1: dV' = attnᵀ·dY + Kc·dS of this wave's tokens.
     f32x4 a = {0.f, 0.f, 0.f, 0.f}, c = a, e = a;
     bf16x8 yf[2];
@@ -710,12 +698,11 @@ __global__ __launch_bounds__(256 * C + 256) void team_rev_kernel(RevParams p) {
     put_state();
     lds_barrier();
   }
-  if (live)
 #pragma unroll
-    for (int i = 0; i < NR; ++i)
+  for (int i = 0; i < NR; ++i)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        p.dstate[(size_t(bh) * K + 16 * (tw + 4 * i) + 4 * g4 + r) * p.V + jl] = S[i][r];
+    for (int r = 0; r < 4; ++r)
+      p.dstate[(size_t(bh) * K + 16 * (tw + 4 * i) + 4 * g4 + r) * p.V + jl] = S[i][r];
 }
 
 }  // namespace

@@ -64,6 +64,23 @@ __device__ inline int perm_pos(int k) {
   const int m = k & 31;
   return (k & ~31) + 8 * ((m & 15) >> 2) + 4 * (m >> 4) + (m & 3);
 }
+// v[0..15] summed over the 16 lanes that share lane/16; lane l receives the
+// total of index l%16 (a halving exchange: 15 shuffles instead of 64).
+__device__ inline float sum16(const float (&v)[16], int lane) {
+  float a[8], b[4], c[2];
+  const bool u8 = lane & 8, u4 = lane & 4, u2 = lane & 2, u1 = lane & 1;
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    a[j] = (u8 ? v[8 + j] : v[j]) + __shfl_xor(u8 ? v[j] : v[8 + j], 8);
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    b[j] = (u4 ? a[4 + j] : a[j]) + __shfl_xor(u4 ? a[j] : a[4 + j], 4);
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    c[j] = (u2 ? b[2 + j] : b[j]) + __shfl_xor(u2 ? b[j] : b[2 + j], 2);
+  return (u1 ? c[1] : c[0]) + __shfl_xor(u1 ? c[0] : c[1], 1);
+}
+
 // A workgroup barrier that orders LDS only: this wave's LDS accesses have
 // completed (lgkmcnt 0) when it arrives, and the compiler moves no memory
 // access across it. __syncthreads() also waits for every global load and
@@ -108,6 +125,11 @@ constexpr int kTriSteps = 6;
 __host__ __device__ constexpr int tril_tb(int s) { return s < 2 ? s : 2 + ((s - 2) >> 1); }
 __host__ __device__ constexpr int tril_kk(int s) { return s < 2 ? 0 : (s - 2) & 1; }
 __host__ __device__ constexpr int tril_step(int tb, int kk) { return tb < 2 ? tb : 2 * tb - 2 + kk; }
+
+// Upper triangular (Tᵀ, attnᵀ): row blocks 2 and 3 have no k-step 0.
+__host__ __device__ constexpr int triu_tb(int s) { return s < 4 ? s >> 1 : s - 2; }
+__host__ __device__ constexpr int triu_kk(int s) { return s < 4 ? s & 1 : 1; }
+__host__ __device__ constexpr int triu_step(int tb, int kk) { return tb < 2 ? 2 * tb + kk : tb + 2; }
 
 // The forward's T, T lo and attn of a chunk-head in HBM, packed: each
 // lower-triangular 64×64 tile as its six nonzero 16×32 blocks (in step order,
