@@ -2,15 +2,17 @@
 step of 32 columns more or less than two, ragged and single-token chunks, each
 gate width, fp32 and bf16 gradients, no forget gate, a write gate that is
 aligned to its elements only, and the shapes either side of the ones that
-chunk_bwd_mfma.hip keeps. Against the fp32 kernels, at the bf16 path's bar
-(attnᵀ and the decayed keys are single bf16 factors, 2^-9 of a term each)."""
+chunk_bwd_mfma.hip keeps. Against the fp32 kernels, which end in the same code
+(csrc/chunk_bwd_tail.hpp), and the float64 oracle, at the bf16 path's bar (attnᵀ
+and the decayed keys are single bf16 factors, 2^-9 of a term each)."""
 
 import numpy as np
 import pytest
 import torch
 
 from conftest import random_raw
-from gpu_util import announce, np_of, pkg, to_gpu
+from gpu_util import announce, as_oracle_inputs, np_of, pkg, to_gpu
+from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -43,10 +45,13 @@ def test_chunk_bwd_local(rng, S, K, V, widths, dtype):
     torch.cuda.synchronize()
     # d_g is a difference of q ⊙ d_q and k ⊙ d_k terms.
     least = max(float(np.abs(np_of(out[GENERIC][i]) * np_of(args[i])).max()) for i in (0, 1))
-    for i, (got, want) in enumerate(zip(out[MFMA], out[GENERIC])):
-        if want is not None:
-            scale = max(np.abs(np_of(want)).max(), least if i == 5 else 0.0)
-            assert np.abs(np_of(got) - np_of(want)).max() / scale < 2e-2, i
+    fp32 = [None if t is None else np_of(t) for t in out[GENERIC]]
+    exact = O.chunk_bwd(np_of(dy), np_of(ds), *as_oracle_inputs(args), chunk_len=64)
+    for i, got in enumerate(out[MFMA]):
+        for want in (fp32[i], exact[i]):
+            if want is not None:
+                scale = max(np.abs(want).max(), least if i == 5 else 0.0)
+                assert np.abs(np_of(got) - want).max() / scale < 2e-2, i
 
 
 @pytest.mark.parametrize("K,V,gates", [(128, 192, "head"), (64, 192, "none"), (64, 64, "channel"),

@@ -1,7 +1,8 @@
-"""The fp32 matrix-core chunk kernels (csrc/chunk_f32.hpp), which run what
-DN_ALGO_GENERIC names at head_k_dim up to 128, against the float64 oracle at
-the edges of their tiles: key blocks of 32, value columns of 16 in one- and
-two-team workgroups, a chunk's 64 tokens.
+"""What DN_ALGO_GENERIC names, against the float64 oracle: the fp32 matrix-core
+chunk kernels (csrc/chunk_f32.hpp; head_k_dim up to 128, chunks of 64) at the
+edges of their tiles (key blocks of 32, value columns of 16 in one- and two-team
+workgroups, a chunk's 64 tokens), and the kernels of any shape
+(csrc/chunk_generic.hip) in what is left to them.
 
 Bar: an output is a sum of products over at most K keys and two triangles of
 64 tokens, each rounded to 2^-24 of the running sum; twice that worst case,
@@ -45,6 +46,21 @@ CASES = [
     # 288 column tiles: more than the device's CUs, so two-team workgroups
     (9, 66, 16, 64, 24, 64, (1, 1, 1)),
     (9, 66, 16, 128, 24, 64, (128, 24, 128)),
+    # ... and chunks enough for every buffer to be filled a second and third time
+    (9, 330, 16, 64, 24, 64, (1, 1, 1)),
+    (9, 330, 16, 32, 40, 64, (32, 1, 32)),
+    (1, 330, 2, 128, 24, 64, (1, 24, 128)),
+]
+
+# The kernels of any shape, where the others do not go: head_k_dim above 128,
+# a per-channel forget gate in other chunks than 64, short chunks.
+ANY_SHAPE = [
+    (1, 70, 2, 129, 20, 64, (1, 1, 1)),
+    (1, 130, 1, 192, 40, 64, (192, 40, 192)),
+    (2, 65, 1, 256, 64, 64, (1, 64, None)),
+    (1, 33, 2, 300, 17, 100, (300, 1, 1)),
+    (1, 90, 2, 64, 24, 40, (1, 1, 64)),
+    (1, 200, 2, 66, 32, 32, (66, 1, None)),
 ]
 
 
@@ -61,20 +77,30 @@ def profiled(f, kernels="dn_f32"):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("case", CASES)
 def test_f32_forward_and_backward_match_oracle(rng, case, dtype):
+    match_oracle(rng, case, dtype, "dn_f32")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("case", ANY_SHAPE)
+def test_any_shape_forward_and_backward_match_oracle(rng, case, dtype):
+    match_oracle(rng, case, dtype, "dn_generic")
+
+
+def match_oracle(rng, case, dtype, kernels):
     B, S, H, K, V, L, (ew, ww, dw) = case
-    announce(f"f32 kernels {case} {dtype}")
+    announce(f"{kernels} kernels {case} {dtype}")
     args = inputs(rng, B, S, H, K, V, ew, ww, dw)
     g_args = to_gpu(args, dtype)
     ref = as_oracle_inputs(g_args)
     scale = 1.0 / np.sqrt(K)
     y, s = profiled(lambda: pkg.delta_chunk_recalculated(
-        *g_args, dw is not None, L, scale, algo=GENERIC, y_dtype=torch.float32))
+        *g_args, dw is not None, L, scale, algo=GENERIC, y_dtype=torch.float32), kernels)
     want_y, want_s = O.chunk_fwd(*ref, chunk_len=L)
     assert rel_err(np_of(y), want_y) < bar(K)
     assert rel_err(np_of(s), want_s) < bar(K)
     dy = torch.tensor(rng.standard_normal((B, S, H, V)), dtype=torch.float32, device=DEV)
     ds = torch.tensor(rng.standard_normal((B, H, K, V)), dtype=torch.float32, device=DEV)
-    got = profiled(lambda: pkg.combined_backward(dy, ds, *g_args, L, scale, algo=GENERIC))
+    got = profiled(lambda: pkg.combined_backward(dy, ds, *g_args, L, scale, algo=GENERIC), kernels)
     want = O.chunk_bwd(np_of(dy), np_of(ds), *ref, chunk_len=L)
     names = ("d_q_bshk", "d_k_bshk", "d_v_bshv", "d_erase_bshK", "d_write_bshV", "d_g_bshK",
              "d_state_bhkv")

@@ -18,11 +18,14 @@ MFMA, GENERIC = pkg.abi.DN_ALGO_MFMA, pkg.abi.DN_ALGO_GENERIC
 
 # On 256 CUs, H·V/16 teams: forward one team a workgroup to 256 of them, two to
 # 512, then 4 and 8 lone waves; the backward's pair of scans turns at half.
+# (tests/cpp/test_launches.cpp asserts which of them a call launches.) 330 tokens
+# are six chunks: every buffer of a scan is filled again.
 @pytest.mark.parametrize("H,K,V,gates", [
     (3, 128, 64, "none"), (7, 128, 256, "head"), (17, 128, 256, "head"), (32, 128, 256, "head"),
     (33, 128, 256, "head"), (65, 128, 256, "head"), (5, 64, 192, "none"), (65, 64, 64, "head"),
-    (9, 128, 128, "channel"), (33, 128, 256, "channel"), (66, 64, 128, "channel")])
-@pytest.mark.parametrize("S", [1, 70])
+    (9, 128, 128, "channel"), (33, 128, 256, "channel"), (66, 64, 128, "channel"),
+    (129, 64, 128, "head"), (128, 64, 192, "channel")])
+@pytest.mark.parametrize("S", [1, 70, 330])
 def test_scan_width(rng, H, K, V, gates, S):
     announce(f"scan width H {H} K {K} V {V} {gates} S {S}")
     raw = random_raw(rng, 1, S, H, K, V, gated=gates != "none", channel=gates == "channel")
