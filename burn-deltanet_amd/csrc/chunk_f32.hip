@@ -225,7 +225,7 @@ __global__ __launch_bounds__(256) void f32_intra_kernel(FParams p) {
 // and write each where the phase that reads it has just ended. With the
 // teams' waves loading and staging between two barriers of their own at each
 // chunk's end, B=4 T=1000 H=8 K=V=128 took 75 us forward and 124 in reverse,
-// B=1 T=512 H=4 K=V=64 28; so, 61, 99 and 23. What is left at K = 128 is half
+// B=1 T=512 H=4 K=V=64 28; so, 62, 97 and 20. What is left at K = 128 is half
 // matrix units (4100 cycles of a wave's fp32 MFMAs a chunk), the rest LDS
 // latency around the three exchanges.
 template <int KB, int C, bool FOLD, bool ST, class TV, class TY>

@@ -1,6 +1,7 @@
 // The chunkwise WY forward and its backward in fp32 on fp32 matrix cores
 // (v_mfma_f32_16x16x4_f32: fp32 products, fp32 sums), in chunks of 64 tokens:
-// fp32 q/k/v, and the bf16 head sizes that the bf16 MFMA kernels do not take.
+// fp32 q/k/v, and the bf16 head sizes that the bf16 MFMA kernels do not take,
+// at head_k_dim up to 128 (chunk_generic.hip chooses, and has the rest).
 //
 // Same mathematics as the bf16 kernels (X = w⊙V − kg·S, V' = T·X; neither U
 // nor W is formed):
@@ -15,10 +16,10 @@
 // do not. At B=4 S=1000 H=8 K=V=128 (23 GFLOP forward and backward, 165 us at
 // that rate; 256 teams of scan waves, one per CU), against the any-shape
 // kernels that ran these calls before, whose scores and inverse were scalar
-// loops over HBM: intra 769 -> 25 us, scan 605 -> 75, states scan 404 -> 63
-// beside the reverse scan 661 -> 124, chunk_bwd 1601 -> 90; forward and
-// backward through autograd 4812 -> 324 us. B=1 S=512 H=4 K=V=64: forward
-// 592 -> 31 us.
+// loops over HBM: intra 769 -> 23 us, scan 605 -> 62, states scan 404 -> 48
+// beside the reverse scan 661 -> 97, chunk_bwd 1601 -> 101; forward and
+// backward through autograd 4812 -> 316 us. B=1 S=512 H=4 K=V=64: forward
+// 592 -> 30 us.
 //
 // Tiles. Every operand is kept as 16×16 blocks of 256 floats. Element (i, j)
 // of a block sits at blk(i, j): float4s along j in the order of the MFMA

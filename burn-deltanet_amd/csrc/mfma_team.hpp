@@ -13,9 +13,16 @@
 //
 // Bound by the chain of a chunk: three exchanges through LDS, each a write, a
 // barrier and a read behind a dozen MFMAs, and LDS busy for 1350 of about 3300
-// cycles. us a chunk at head_k_dim 128, one round: lone waves, two to a
-// workgroup (32 columns) 3.2, per-channel gates 3.4; a team (16 columns) 1.7
-// and 1.85, two (32 columns) 2.05 and 2.25; the reverse scan 3.7 and 1.8, 2.2.
+// cycles. us a chunk at head_k_dim 128, one round of 16 chunks (a launch's
+// start and end in them): lone waves, two to a workgroup (32 columns) 3.2,
+// per-channel gates 3.4; a team (16 columns) 1.7 and 1.85, two (32 columns) 2.05
+// and 2.25; the reverse scan 3.7 and 1.8, 2.2. Over longer sequences 1.5 for a
+// team (24 chunks, 36 us) and 1.9 for two (256 chunks, 488).
+//
+// K·S_hi and K·S_lo are summed apart, as are T·X's three products, so that a
+// chunk's chain is half as long; with the lone kernels' order of sums the y of
+// B=4 S=16384 H=16 differs by 1.6e-4 (last bits that turn over the rounding of
+// V' to bf16), and either is 3.1e-3 from float64.
 // B=1 S=1531 H=16 dk 128 dv 256: forward 82 -> 44 us; B=4 S=16384 H=16
 // dk=dv=128: 910 -> 659.
 #pragma once

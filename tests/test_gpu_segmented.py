@@ -1,15 +1,15 @@
 """The segmented MFMA scan against the oracle.
 
-When batch × heads × head_v_dim/128 leaves most of the device's 256 CUs idle,
-the two-kernel forward cuts each sequence into P segments of whole chunks
-(P a power of two, at least 16 chunks per segment, head_k_dim 128): one scan
-forms every segment's transition M and offset H (the affine map the chunk
-updates compose to), a carry kernel walks the segments in order (start(s+1)
-= M_s·start(s) + H_s, as bf16 hi + lo MFMAs), and a second scan produces y
-and the final state from the carried starts. The shapes below give P = 2, 4
-and 8 on a 256-CU MI355X; the library's per-kernel profiler confirms the
-carry ran. Bar: the north_star's bf16 bar (normwise relative ≤ 2e-2, fp32
-state) against the oracle fed the bf16-rounded q/k/v the GPU reads."""
+Where a whole scan leaves most of the device's 256 CUs idle, the two-kernel
+forward cuts each sequence into P segments of whole chunks (a power of two, at
+head_k_dim 64 and 128): one scan forms every segment's transition M and offset
+H (the affine map the chunk updates compose to), a carry kernel walks the
+segments in order (start(s+1) = M_s·start(s) + H_s, as bf16 hi + lo MFMAs), and
+a second scan produces y and the final state from the carried starts, by teams
+of four waves or by 8-wave workgroups. The library's per-kernel profiler
+confirms that the carry ran (tests/cpp/test_launches.cpp, which kernels walked
+the segments). Bar: the bf16 path's, normwise relative ≤ 2e-2, fp32 state,
+against the oracle fed the bf16-rounded q/k/v the GPU reads."""
 
 import numpy as np
 import pytest
@@ -56,14 +56,14 @@ def run(g_args, y_dtype=torch.bfloat16, in_place=False):
 
 
 CASES = [
-    # B, S, H, K, V, gates, state_std: segments on a 256-CU device
-    (1, 4096, 2, 128, 128, "head", 0.02),      # P = 4
-    (1, 8192, 1, 128, 128, "channel", 0.02),   # P = 8, GDN-2 gate widths
-    (1, 2048, 1, 128, 256, "head", 0.0),       # P = 2, two 128-column tiles
-    (2, 4096, 1, 128, 128, None, 0.02),        # P = 4, ungated
-    (1, 4096, 1, 128, 128, "channel", 0.5),    # P = 4, a large initial state
-    (1, 8192, 12, 128, 128, "head", 0.02),     # P = 8, by eight-wave workgroups
-    (1, 8192, 16, 128, 128, "channel", 0.02),  # P = 8, by eight-wave workgroups
+    # B, S, H, K, V, gates, state_std
+    (1, 4096, 2, 128, 128, "head", 0.02),
+    (1, 8192, 1, 128, 128, "channel", 0.02),   # GDN-2 gate widths
+    (1, 2048, 1, 128, 256, "head", 0.0),
+    (2, 4096, 1, 128, 128, None, 0.02),        # ungated
+    (1, 4096, 1, 128, 128, "channel", 0.5),    # a large initial state
+    (1, 8192, 12, 128, 128, "head", 0.02),     # by 8-wave workgroups
+    (1, 8192, 16, 128, 128, "channel", 0.02),  # by 8-wave workgroups
 ]
 
 

@@ -96,7 +96,7 @@ def test_noalloc_keeps_to_its_scratch():
 
 def test_noalloc_refuses_arguments_above_its_scratch():
     announce("dn_chunk_fwd_noalloc: too large for the scratch array")
-    # BASELINE config 5 (GDN-2 per-channel gates): 737 MB of workspace.
+    # Per-channel gates at B=2 S=16384 H=16: 737 MB of workspace.
     B, S, H, K, V = 2, 16384, 16, 128, 128
     q = torch.empty((B, S, H, K), dtype=torch.bfloat16, device=DEV)
     v = torch.empty((B, S, H, V), dtype=torch.bfloat16, device=DEV)
