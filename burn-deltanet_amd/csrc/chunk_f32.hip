@@ -197,7 +197,7 @@ __global__ __launch_bounds__(256) void f32_intra_kernel(FParams p) {
     }
   }
   __syncthreads();
-  diag_inverse(A, Tm, wave, lane);
+  diag_inverse<true>(A, Tm, wave, lane);
   __syncthreads();
   merge_T(A, Tm, Xs, wave, lane, [] { __syncthreads(); });
 #pragma unroll
@@ -205,7 +205,7 @@ __global__ __launch_bounds__(256) void f32_intra_kernel(FParams p) {
     constexpr int ti_[10] = {0, 1, 1, 2, 2, 2, 3, 3, 3, 3}, tj_[10] = {0, 0, 1, 0, 1, 2, 0, 1, 2, 3};
     const int r = tid >> 4, c = tid & 15;
     const float x = Tm[16 * ti_[i] + r][16 * tj_[i] + c];
-    ws[o.t + i * kBlk + blk(r, c)] = ti_[i] > tj_[i] || c <= r ? x : 0.f;
+    ws[o.t + i * kBlk + blk(r, c)] = x;
   }
 }
 

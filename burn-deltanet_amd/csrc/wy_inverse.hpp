@@ -31,7 +31,10 @@ __device__ inline float quad_bcast(float v, int src) {
 // T's diagonal 16×16 block `wave` of T = (I + A)⁻¹ (A strict lower, fp32 in
 // LDS) by column elimination; one wave per block. Lane (c, g) holds rows g,
 // g+4, g+8, g+12 of column c; step k₂ broadcasts x[k₂] inside the lane quad
-// (DPP) and updates the rows below it.
+// (DPP) and updates the rows below it. Apart: what x holds on and above the
+// diagonal is known and not taken from the updates, in which a non-finite A[i]
+// meets x's zeros there, so that T's columns from i on keep their values.
+template <bool Apart = false>
 __device__ inline void diag_inverse(const float (*A)[kWyL + 1], float (*Tm)[kWyL + 1], int wave,
                                     int lane) {
   const int base = 16 * wave, c = lane >> 2, g = lane & 3;
@@ -57,14 +60,19 @@ __device__ inline void diag_inverse(const float (*A)[kWyL + 1], float (*Tm)[kWyL
 #pragma unroll
     for (int u = 0; u < 5; ++u) {
       const int k2 = 5 * batch + u;
-      const float xk = quad_bcast(x[k2 >> 2], k2 & 3);
+      float xk = quad_bcast(x[k2 >> 2], k2 & 3);
+      if constexpr (Apart) xk = c < k2 ? xk : c == k2 ? 1.f : 0.f;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         if (4 * j + 3 > k2) x[j] -= mul[batch & 1][u][j] * xk;
     }
   }
 #pragma unroll
-  for (int j = 0; j < 4; ++j) Tm[base + 4 * j + g][base + c] = x[j];
+  for (int j = 0; j < 4; ++j) {
+    const int i = 4 * j + g;
+    if constexpr (Apart) x[j] = c < i ? x[j] : c == i ? 1.f : 0.f;
+    Tm[base + i][base + c] = x[j];
+  }
 }
 
 // The two doubling merges that complete T from its diagonal blocks, in three

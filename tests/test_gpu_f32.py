@@ -150,6 +150,24 @@ def test_short_chunks_are_as_accurate_as_their_length(rng, L, K):
         assert rel_err(np_of(getattr(got, name)), want[i]) < bar(K), name
 
 
+@pytest.mark.parametrize("widths", [(1, 1, 1), (64, 24, 64)])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_erase_gate_that_is_not_finite(rng, value, widths):
+    """The gradients of v and the write gate from a token on do not meet its
+    erase gate, whatever that is: they are those of a finite one, to the bit."""
+    announce(f"f32 kernels: erase gate {value} {widths}")
+    S, K, V, t = 100, 64, 24, 20
+    args = to_gpu(inputs(rng, 1, S, 2, K, V, *widths))
+    dy = torch.tensor(rng.standard_normal((1, S, 2, V)), dtype=torch.float32, device=DEV)
+    out = []
+    for e in (0.5, value):
+        args[3][:, t, 0, 0] = e
+        g = profiled(lambda: pkg.combined_backward(dy, None, *args, 64, 0.5, algo=GENERIC))
+        out.append((g.d_v_bshv[:, t:], g.d_write_bshV[:, t:]))
+    for want, got in zip(*out):
+        assert bool(torch.isfinite(got).all()) and torch.equal(want, got)
+
+
 @pytest.mark.parametrize("V,widths", [(40, (1, 1, 1)), (24, (64, 24, 64))])
 def test_workspace_at_a_four_byte_boundary(rng, V, widths):
     """The generic path's workspace is owed the alignment of its floats: one
