@@ -1,4 +1,4 @@
-"""HIP-graph capture of the MFMA forward and backward.
+"""HIP-graph capture of the MFMA and the fp32 forward and backward.
 
 A captured dn_chunk_fwd + dn_chunk_bwd replays to the eager results. The
 backward forks its reverse scan onto the library's second stream and joins it
@@ -17,26 +17,28 @@ from test_gpu_mfma import gdn2_inputs, gdn_inputs
 
 pytestmark = pytest.mark.gpu
 
-MFMA = pkg.abi.DN_ALGO_MFMA
+MFMA, GENERIC = pkg.abi.DN_ALGO_MFMA, pkg.abi.DN_ALGO_GENERIC
 
 
 def _workspace(nbytes):
     return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=DEV)
 
 
-@pytest.mark.parametrize("gates", ["head", (128, 128)])
-def test_graph_replays_match_eager(rng, gates):
-    announce(f"graph capture fwd+bwd, gates {gates}")
+@pytest.mark.parametrize("gates,algo", [("head", MFMA), ((128, 128), MFMA), ("head", GENERIC),
+                                        ((128, 128), GENERIC)])
+def test_graph_replays_match_eager(rng, gates, algo):
+    announce(f"graph capture fwd+bwd, gates {gates}, algo {algo}")
     B, S, H, K, V = 1, 256, 2, 128, 128
     if gates == "head":
         args = gdn_inputs(rng, B, S, H, K, V, gated=True, state_std=0.05)
     else:
         args = gdn2_inputs(rng, B, S, H, K, V, gates[0], gates[1], state_std=0.05)
-    q, k, v, e, w, g, s = to_gpu(args, torch.bfloat16)
+    dtype = torch.bfloat16 if algo == MFMA else torch.float32
+    q, k, v, e, w, g, s = to_gpu(args, dtype)
     dy = torch.tensor(rng.standard_normal((B, S, H, V)), dtype=torch.float32,
-                      device=DEV).to(torch.bfloat16)
+                      device=DEV).to(dtype)
     abi = pkg.abi
-    y = torch.empty((B, S, H, V), dtype=torch.bfloat16, device=DEV)
+    y = torch.empty((B, S, H, V), dtype=dtype, device=DEV)
     s1 = torch.empty_like(s)
     fa = abi.chunk_fwd_args(q, k, v, e, w, g, s, y, s1, 64, None)
     wsf = _workspace(abi.lib().dn_chunk_fwd_workspace_bytes(fa))
@@ -46,8 +48,8 @@ def test_graph_replays_match_eager(rng, gates):
     ba = abi.chunk_bwd_args(dy, None, q, k, v, e, w, g, s, grads, 64, None)
     wsb = _workspace(abi.lib().dn_chunk_bwd_workspace_bytes(ba))
     ba.workspace, ba.workspace_bytes = wsb.data_ptr(), wsb.numel()
-    assert abi.lib().dn_chunk_fwd_algo(fa) == MFMA
-    assert abi.lib().dn_chunk_bwd_algo(ba) == MFMA
+    assert abi.lib().dn_chunk_fwd_algo(fa) == algo
+    assert abi.lib().dn_chunk_bwd_algo(ba) == algo
 
     def run():
         abi.run_chunk_fwd(fa)
